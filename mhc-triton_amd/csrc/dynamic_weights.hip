@@ -338,6 +338,7 @@ constexpr int kPoolUN = 4;  // rows in flight per lane in colsum_kernel
 // bits): at such lengths the pass is a few microseconds of latency, and the
 // second launch and the column-partial round trip are most of it.
 constexpr int64_t kPoolDirectRows = 8;
+constexpr int64_t kPoolPlainBytes = (int64_t)64 << 20;  // H up to here is read without the nt policy
 
 template <typename T, int W, bool PROJ>
 static int launch_meanpool(const T* H, float* x, const float* phi, float* projpart, float* colpart, int64_t B,
@@ -366,9 +367,11 @@ static int launch_meanpool(const T* H, float* x, const float* phi, float* projpa
     // The first half of each S chunk with nt loads, the second half plain: in
     // the layer, branch_input reads H next and finds the chunk tails in the
     // memory-side cache (colsum + branch_input: -4 us at config-3 size, -6 us
-    // at config 4, against all plain).
+    // at config 4, against all plain).  An H of up to 64 MB stays there whole, and all plain is
+    // 1-2 us faster at 33 MB (the two passes 28.4 -> 27.3 us) and equal at 67 MB.
+    const bool all_plain = B * S * K * (int64_t)sizeof(T) <= kPoolPlainBytes;
     colsum_kernel<T, W, kPoolUN><<<dim3((unsigned)p.ncc, (unsigned)p.nS, (unsigned)nb), kThreads, 0, st>>>(
-        H, colpart, S, K, p.SC, p.nS, p.SC / 2, b0);
+        H, colpart, S, K, p.SC, p.nS, all_plain ? 0 : p.SC / 2, b0);
     if (int rc = hip_status(hipGetLastError(), "mean_pool column-sum launch")) return rc;
     colsum_reduce_kernel<PROJ><<<dim3((unsigned)p.nrc, (unsigned)nb), kThreads, 0, st>>>(
         colpart, x, phi, projpart, K, p.nS, inv_S, b0, phi_vec);

@@ -90,13 +90,33 @@ static LayerWs layer_ws(int64_t B, int64_t S, int64_t D, int dtype) {
   return w;
 }
 
-template <typename T, int W>
+// H is read two or three times in a forward (mean-pool, branch_input, the closure's H_new), so an
+// H that fits the 256 MB memory-side cache several times over is better read with plain loads,
+// which leave it there, than with the streaming (nt) policy, and then 6 workgroups per CU beat 3:
+// these reads come back sooner than HBM's.  Measured (bf16, training steps as replayed graphs,
+// three sets of inputs in turn; nt at 3 per CU -> plain at 6, mean-pool included): H = 33 MB
+// 93.1 -> 86.3 us, 67 MB 147.3 -> 141.1; forward without the closure 30.9 -> 27.3 and 41.4 ->
+// 37.3.  The line lies where another 600 MB of traffic between branch_input and the closure (a
+// branch that streams its own data) makes the plain closure lose: at 67 MB it still ties (188.0
+// against 189.2 us), at 134 MB it loses 235 -> 239.
+constexpr int64_t kCachedHBytes = (int64_t)96 << 20;
+
+static bool h_cached(int64_t B, int64_t S, int64_t D, size_t esize) {
+  return B * S * 4 * D * (int64_t)esize <= kCachedHBytes;
+}
+
+// The NT policy and the occupancy cap of the two forward passes over H.
+constexpr int kNtCached = 2;  // plain loads, nt stores
+constexpr int fwd_wgs(bool cached) { return cached ? 6 : 3; }
+
+template <typename T, int W, int NT>
 static int launch_bi(const T* H, const float* w, T* bi, int64_t B, int64_t S, int64_t D, hipStream_t st) {
   return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
     const Geom g = make_geom<W, kLU>(S, D, b0);
     if (g.ntiles == 0) return (int)MHC_OK;
-    mix_fwd_kernel<T, T, W, kLU, true, false, false, kNt><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(3), st>>>(
-        H, (const T*)nullptr, WRow{w, kOut}, WRow{nullptr, 0}, WRow{nullptr, 0}, bi, nullptr, g);
+    mix_fwd_kernel<T, T, W, kLU, true, false, false, NT>
+        <<<dim3(g.ntiles, nb), kThreads, occupancy_lds(fwd_wgs(NT == kNtCached)), st>>>(
+            H, (const T*)nullptr, WRow{w, kOut}, WRow{nullptr, 0}, WRow{nullptr, 0}, bi, nullptr, g);
     return hip_status(hipGetLastError(), "layer branch_input launch");
   });
 }
@@ -106,8 +126,9 @@ static int branch_input_any(const void* H, int dtype, const float* w, void* bi, 
   if (S * D == 0) return MHC_OK;
   return MHC_DISPATCH_DTYPE(dtype, [&] {
     constexpr int WV = Vec<T>::N;
-    if (vec_ok(D, WV, {H, bi})) return launch_bi<T, WV>((const T*)H, w, (T*)bi, B, S, D, st);
-    return launch_bi<T, 1>((const T*)H, w, (T*)bi, B, S, D, st);
+    if (!vec_ok(D, WV, {H, bi})) return launch_bi<T, 1, kNt>((const T*)H, w, (T*)bi, B, S, D, st);
+    if (h_cached(B, S, D, sizeof(T))) return launch_bi<T, WV, kNtCached>((const T*)H, w, (T*)bi, B, S, D, st);
+    return launch_bi<T, WV, kNt>((const T*)H, w, (T*)bi, B, S, D, st);
   });
 }
 
@@ -473,22 +494,26 @@ extern "C" int mhc_layer_add_forward(const void* H, int dtype_h, const void* bra
   hipStream_t st = (hipStream_t)stream;
   return MHC_DISPATCH_DTYPE2(dtype_h, dtype_bo, [&] {
     constexpr int WV = Vec<TH>::N > Vec<TB>::N ? Vec<TH>::N : Vec<TB>::N;
-    auto go = [&](auto wtag) {
+    auto go = [&](auto wtag, auto nttag) {
       constexpr int W = decltype(wtag)::value;
+      constexpr int NT = decltype(nttag)::value;
       return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
         const Geom g = make_geom<W, kLU>(S, D, b0);
-        // 3 workgroups per CU: 188.5 us at config-3 size against 194.9 with 2 and 190.4 with 4
-        // when chosen; with the buffer-span loads and nt policy caps 2 and 3 time alike and 4
+        // With the nt policy 3 workgroups per CU: 188.5 us at config-3 size against 194.9 with 2
+        // and 190.4 with 4 when chosen; with the buffer-span loads caps 2 and 3 time alike and 4
         // is about 1 us slower (192.6-195.4 us event-timed in the bench).
-        mix_fwd_kernel<TH, TB, W, kLU, false, true, true, kNt>
-            <<<dim3(g.ntiles, nb), kThreads, occupancy_lds(3), st>>>(
+        mix_fwd_kernel<TH, TB, W, kLU, false, true, true, NT>
+            <<<dim3(g.ntiles, nb), kThreads, occupancy_lds(fwd_wgs(NT == kNtCached)), st>>>(
             (const TH*)H, (const TB*)branch_output, WRow{nullptr, 0}, WRow{w + 8, kOut}, WRow{w + 4, kOut},
             nullptr, (TH*)H_new, g);
         return hip_status(hipGetLastError(), "layer add forward launch");
       });
     };
-    if (vec_ok(D, WV, {H, branch_output, H_new})) return go(std::integral_constant<int, WV>{});
-    return go(std::integral_constant<int, 1>{});
+    using Stream = std::integral_constant<int, kNt>;
+    if (!vec_ok(D, WV, {H, branch_output, H_new})) return go(std::integral_constant<int, 1>{}, Stream{});
+    if (h_cached(B, S, D, sizeof(TH)))
+      return go(std::integral_constant<int, WV>{}, std::integral_constant<int, kNtCached>{});
+    return go(std::integral_constant<int, WV>{}, Stream{});
   });
 }
 
