@@ -41,6 +41,7 @@ constexpr int64_t kMfmaMinRows = 64;
 constexpr int64_t kMfmaTargetWg = 256;
 
 struct MfmaPlan {
+  int steps;            // 16-k steps per wave slice
   int64_t nsteps;       // K / 16
   int nK;               // chunks
   int64_t rows_per_wg;  // multiple of 32
@@ -54,11 +55,18 @@ static bool mfma_shape_ok(int64_t R, int64_t K, int esize) {
 
 static MfmaPlan mfma_plan(int64_t R, int64_t K, int esize) {
   MfmaPlan p;
-  const int64_t chunk_steps = (int64_t)kMfmaWaves * mfma_steps(esize);
   p.nsteps = K / 16;
-  p.nK = (int)((p.nsteps + chunk_steps - 1) / chunk_steps);
-  if (p.nK < 1) p.nK = 1;
   const int64_t tiles = (R + 31) / 32;
+  // A few row tiles with full slices leave most CUs idle (R = 64, K = 16384, bf16: 32 workgroups,
+  // 9.5 us); shorter slices split K further until every CU has a workgroup.
+  p.steps = mfma_steps(esize);
+  auto chunks = [&](int steps) {
+    const int64_t chunk_steps = (int64_t)kMfmaWaves * steps;
+    return (p.nsteps + chunk_steps - 1) / chunk_steps;
+  };
+  while (p.steps > kMfmaMinSteps && chunks(p.steps) * tiles < kMfmaTargetWg) p.steps /= 2;
+  p.nK = (int)chunks(p.steps);
+  if (p.nK < 1) p.nK = 1;
   int64_t ngr = (kMfmaTargetWg + p.nK - 1) / p.nK;
   if (ngr > tiles) ngr = tiles;
   if (ngr < 1) ngr = 1;
@@ -68,6 +76,21 @@ static MfmaPlan mfma_plan(int64_t R, int64_t K, int esize) {
   p.ngr = (int)((R + p.rows_per_wg - 1) / p.rows_per_wg);
   p.part_bytes = align256((size_t)R * p.nK * kPart * sizeof(float));
   return p;
+}
+
+// Runs the plan's projection: part[r][kc][0:25] for every row and K chunk.
+template <typename T>
+static hipError_t launch_mfma(const MfmaPlan& m, const T* x, const float* phi, float* part, int64_t R, int64_t K,
+                              hipStream_t st) {
+  const dim3 grid((unsigned)m.ngr, (unsigned)m.nK);
+  auto go = [&](auto steps) {
+    dynw_mfma_kernel<T, kMfmaWaves, decltype(steps)::value>
+        <<<grid, 64 * kMfmaWaves, 0, st>>>(x, phi, part, R, K, m.nK, m.rows_per_wg);
+  };
+  if (m.steps == 2) go(std::integral_constant<int, 2>{});
+  else if (m.steps == 4) go(std::integral_constant<int, 4>{});
+  else if constexpr (mfma_steps(sizeof(T)) == 8) go(std::integral_constant<int, 8>{});
+  return hipGetLastError();
 }
 
 }  // namespace mhc
@@ -112,10 +135,8 @@ extern "C" int mhc_dynamic_weights_forward(const void* x, int dtype_x, const flo
   if (mfma_shape_ok(R, K, esize) && aligned16(x)) {
     // rows in bulk: the projection on MFMA (HBM-bound instead of VALU-bound).
     const MfmaPlan m = mfma_plan(R, K, esize);
-    const dim3 grid((unsigned)m.ngr, (unsigned)m.nK);
     int rc = MHC_DISPATCH_DTYPE(dtype_x, [&] {
-      dynw_mfma_kernel<T><<<grid, 64 * kMfmaWaves, 0, st>>>((const T*)x, phi, part, R, K, m.nK, m.rows_per_wg);
-      return hip_status(hipGetLastError(), "dynamic_weights_forward mfma launch");
+      return hip_status(launch_mfma<T>(m, (const T*)x, phi, part, R, K, st), "dynamic_weights_forward mfma launch");
     });
     if (rc) return rc;
     nK = m.nK;
@@ -131,13 +152,9 @@ extern "C" int mhc_dynamic_weights_forward(const void* x, int dtype_x, const flo
     nK = p.nK;
   }
   DynParams P{bias, bias + 4, bias + 8, alpha_pre, alpha_post, alpha_res};
-  if (R >= kMfmaMinRows && nK <= 64)
-    dynw_finalize_rows_kernel<><<<dim3((unsigned)((R + kFinRowsWg - 1) / kFinRowsWg)), kThreads, 0, st>>>(
-        part, nK, R, K, P, OutRow{H_pre, 4}, OutRow{H_post, 4}, OutRow{H_res, 16}, aux, iters, eps);
-  else
-    dynw_finalize_kernel<><<<dim3((unsigned)((R + 3) / 4)), kThreads, 0, st>>>(
-        part, nK, R, K, P, OutRow{H_pre, 4}, OutRow{H_post, 4}, OutRow{H_res, 16}, aux, iters, eps);
-  return hip_status(hipGetLastError(), "dynamic_weights_forward finalize launch");
+  return hip_status(launch_finalize(part, nK, R, K, P, OutRow{H_pre, 4}, OutRow{H_post, 4}, OutRow{H_res, 16}, aux,
+                                    iters, eps, st),
+                    "dynamic_weights_forward finalize launch");
 }
 
 namespace mhc {
@@ -154,9 +171,7 @@ int dynw_project_rows(const void* x, int dtype, const float* phi, float* part, i
   const MfmaPlan m = mfma_plan(R, K, dtype == MHC_DTYPE_F32 ? 4 : 2);
   *nK = m.nK;
   return MHC_DISPATCH_DTYPE(dtype, [&] {
-    dynw_mfma_kernel<T><<<dim3((unsigned)m.ngr, (unsigned)m.nK), 64 * kMfmaWaves, 0, st>>>(
-        (const T*)x, phi, part, R, K, m.nK, m.rows_per_wg);
-    return hip_status(hipGetLastError(), "layer projection mfma launch");
+    return hip_status(launch_mfma<T>(m, (const T*)x, phi, part, R, K, st), "layer projection mfma launch");
   });
 }
 

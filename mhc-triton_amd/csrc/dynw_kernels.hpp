@@ -149,8 +149,9 @@ constexpr int kMfmaWaves = 8;                             // waves per workgroup
 constexpr int kMfmaSteps = 8;                             // 16-k steps per wave slice (16-bit x)
 constexpr int kMfmaChunkSteps = kMfmaWaves * kMfmaSteps;  // steps per K chunk (16-bit x)
 // fp32 x: half the steps per slice, so that a slice is still 256 bytes of a row
-// and the LDS tiles keep their size
+// and the LDS tiles keep their size.  A few rows take shorter slices (mfma_plan).
 __host__ __device__ constexpr int mfma_steps(int esize) { return esize == 4 ? kMfmaSteps / 2 : kMfmaSteps; }
+constexpr int kMfmaMinSteps = 2;  // K chunks of 256: as many records per row as the VALU plans hold
 constexpr int kMfmaRedCols = kPart;                       // 24 dot products and the sum of squares
 constexpr int kMfmaRedPitch = 36;                         // floats per (wave, column): 32 rows + pad
 
@@ -429,37 +430,71 @@ __device__ __forceinline__ void dyn_scaled(const DynParams& P, const float (&raw
 // Eq. 14-19 epilogue of one row in 16-lane form: lane e owns H_res element e;
 // lanes 0..3 also H_pre[e], lanes 4..7 H_post[e - 4].  raw_res = raw[8 + e],
 // raw_pp = raw[e & 7] and sumsq (the row's sum of x^2) are the row's totals.
-// All 16 lanes of the row must take part (DPP sums); lanes with !store
-// compute and write nothing.
-__device__ __forceinline__ void finalize_row16(int e, int64_t r, float raw_res, float raw_pp, float sumsq,
-                                               int64_t K, const DynParams& P, OutRow o_pre, OutRow o_post,
-                                               OutRow o_res, float* __restrict__ aux, int iters, float eps,
-                                               bool store) {
+// All 16 lanes of the row must take part (DPP sums).
+struct Row16 {
+  float res;      // H_res[e]
+  float pp;       // lanes 0..3 H_pre[e], lanes 4..7 H_post[e - 4]
+  float inv_rms;
+};
+
+__device__ __forceinline__ Row16 weights_row16(int e, float raw_res, float raw_pp, float sumsq, int64_t K,
+                                               const DynParams& P, int iters, float eps) {
   const int j = e & 3;
   const bool is_pre = e < 4;
-  const float inv_rms = 1.f / sqrtf(sumsq / (float)K + eps);
+  Row16 o;
+  o.inv_rms = 1.f / sqrtf(sumsq / (float)K + eps);
   // Eq. 19: H_res = Sinkhorn(|s_res| + eps)
-  const float m = sk16_forward(inv_rms * *P.alpha_res * raw_res + P.bias_res[e], iters, eps);
+  o.res = sk16_forward(o.inv_rms * *P.alpha_res * raw_res + P.bias_res[e], iters, eps);
   // Eq. 17: H_pre = sigmoid / (sum + eps); Eq. 18: H_post = 2 sigmoid
-  const float s_pp = inv_rms * (is_pre ? *P.alpha_pre : *P.alpha_post) * raw_pp +
+  const float s_pp = o.inv_rms * (is_pre ? *P.alpha_pre : *P.alpha_post) * raw_pp +
                      (is_pre ? P.bias_pre[j] : P.bias_post[j]);
   const float sg = sigmoidf(s_pp);
   const float den = sum_row16(sg) + eps;  // quad 0: the four H_pre sigmoids
-  if (!store) return;
-  o_res.p[r * o_res.stride + e] = m;
-  if (is_pre) o_pre.p[r * o_pre.stride + j] = sg / den;
-  else if (e < 8) o_post.p[r * o_post.stride + j] = 2.f * sg;
+  o.pp = is_pre ? sg / den : 2.f * sg;
+  return o;
+}
+
+// Writes a row's weights and, with aux, its record [raw (24), inv_rms] for the backward.
+__device__ __forceinline__ void store_row16(int e, int64_t r, const Row16& o, float raw_res, float raw_pp, OutRow o_pre,
+                                            OutRow o_post, OutRow o_res, float* __restrict__ aux) {
+  const int j = e & 3;
+  o_res.p[r * o_res.stride + e] = o.res;
+  if (e < 4) o_pre.p[r * o_pre.stride + j] = o.pp;
+  else if (e < 8) o_post.p[r * o_post.stride + j] = o.pp;
   if (aux) {
     aux[r * kPart + 8 + e] = raw_res;
     if (e < 8) aux[r * kPart + e] = raw_pp;
-    if (e == 0) aux[r * kPart + kOut] = inv_rms;
+    if (e == 0) aux[r * kPart + kOut] = o.inv_rms;
   }
 }
 
-// One wave per row.  Lane l sums the partial records l, l+64, l+128, ... (25
-// floats each) in chunk order; each 16-lane row of the wave then adds its lane
-// sums with DPP (sum_all16), and lanes 0..15 add the four row sums in order
-// and run the epilogue.  Keeping 64 independent load streams per row instead
+// The totals of one row's nK partial records, by one wave: lane l sums records l, l + 64, ...
+// (25 floats each) in chunk order and each 16-lane row adds its lane sums with DPP into
+// quarter[0..3]; the row's total j is then their sum in order (row_total).
+__device__ __forceinline__ void sum_records(const float* __restrict__ part, int nK, int lane,
+                                            float (*__restrict__ quarter)[kPart]) {
+  float acc[kPart];
+#pragma unroll
+  for (int j = 0; j < kPart; ++j) acc[j] = 0.f;
+  for (int k = lane; k < nK; k += 64) {
+    const float* p = part + (int64_t)k * kPart;
+#pragma unroll
+    for (int j = 0; j < kPart; ++j) acc[j] += p[j];
+  }
+#pragma unroll
+  for (int j = 0; j < kPart; ++j) acc[j] = sum_all16(acc[j]);
+  if ((lane & 15) == 0) {
+#pragma unroll
+    for (int j = 0; j < kPart; ++j) quarter[lane >> 4][j] = acc[j];
+  }
+}
+
+__device__ __forceinline__ float row_total(const float (*q)[kPart], int j) {
+  return ((q[0][j] + q[1][j]) + q[2][j]) + q[3][j];
+}
+
+// One wave per row: the row's totals (sum_records), then lanes 0..15 run the
+// epilogue.  Keeping 64 independent load streams per row instead
 // of one serial chain matters: R is the batch (4 at dim 4096) and this kernel
 // sits between two full passes over H.  (A __shfl_xor butterfly took 150
 // ds_bpermute per wave for the same sums.)
@@ -473,26 +508,13 @@ __global__ __launch_bounds__(kThreads) void dynw_finalize_kernel(const float* __
   const int lane = threadIdx.x & 63;
   const int64_t r = (int64_t)blockIdx.x * 4 + wave;
   const bool live = r < R;
-  float acc[kPart];
-#pragma unroll
-  for (int j = 0; j < kPart; ++j) acc[j] = 0.f;
-  for (int k = lane; live && k < nK; k += 64) {
-    const float* p = part + (r * nK + k) * kPart;
-#pragma unroll
-    for (int j = 0; j < kPart; ++j) acc[j] += p[j];
-  }
-#pragma unroll
-  for (int j = 0; j < kPart; ++j) acc[j] = sum_all16(acc[j]);
-  if ((lane & 15) == 0) {
-#pragma unroll
-    for (int j = 0; j < kPart; ++j) quarter[wave][lane >> 4][j] = acc[j];
-  }
+  if (live) sum_records(part + r * nK * kPart, nK, lane, quarter[wave]);
   __syncthreads();
   if (!live || lane >= 16) return;
   const float(*q)[kPart] = quarter[wave];
-  auto tot = [&](int j) { return ((q[0][j] + q[1][j]) + q[2][j]) + q[3][j]; };
-  finalize_row16(lane, r, tot(8 + lane), tot(lane & 7), tot(kOut), K, P, o_pre, o_post, o_res, aux, iters, eps,
-                 true);
+  const float raw_res = row_total(q, 8 + lane), raw_pp = row_total(q, lane & 7);
+  const Row16 o = weights_row16(lane, raw_res, raw_pp, row_total(q, kOut), K, P, iters, eps);
+  store_row16(lane, r, o, raw_res, raw_pp, o_pre, o_post, o_res, aux);
 }
 
 // The same for many rows with few chunks (the MFMA projection at R = tokens:
@@ -524,7 +546,23 @@ __global__ __launch_bounds__(kThreads) void dynw_finalize_rows_kernel(const floa
     raw_pp += p[e & 7];
     sumsq += p[kOut];
   }
-  finalize_row16(e, r, raw_res, raw_pp, sumsq, K, P, o_pre, o_post, o_res, aux, iters, eps, live);
+  const Row16 o = weights_row16(e, raw_res, raw_pp, sumsq, K, P, iters, eps);
+  if (live) store_row16(e, r, o, raw_res, raw_pp, o_pre, o_post, o_res, aux);
+}
+
+// The epilogue of R rows with nK partial records each: a 16-lane group per row adds the records
+// one after the other, so it pays for many rows with few records; else a wave per row.
+inline bool finalize_by_rows(int64_t R, int nK) { return nK <= 32 ? R >= 64 : (nK <= 64 && R >= 512); }
+
+inline hipError_t launch_finalize(const float* part, int nK, int64_t R, int64_t K, const DynParams& P, OutRow o_pre,
+                                  OutRow o_post, OutRow o_res, float* aux, int iters, float eps, hipStream_t st) {
+  if (finalize_by_rows(R, nK))
+    dynw_finalize_rows_kernel<><<<dim3((unsigned)((R + kFinRowsWg - 1) / kFinRowsWg)), kThreads, 0, st>>>(
+        part, nK, R, K, P, o_pre, o_post, o_res, aux, iters, eps);
+  else
+    dynw_finalize_kernel<><<<dim3((unsigned)((R + 3) / 4)), kThreads, 0, st>>>(part, nK, R, K, P, o_pre, o_post, o_res,
+                                                                                aux, iters, eps);
+  return hipGetLastError();
 }
 
 // Per-row backward record rowbuf[r][0:52]:

@@ -2,7 +2,8 @@
 // ops.py / _kernels.py / _backward.py).
 //
 // Forward, dynamic:   meanpool<PROJ> (reads H)  -> finalize (weights w[B,24])
-//                     -> branch_input pass (reads H, writes bi)
+//                     -> branch_input pass (reads H, writes bi; with few tiles it
+//                     runs the finalize itself)
 // Closure forward:    H_new = H_res @ H + H_post * bo (reads H, bo; writes H_new)
 // Closure backward:   d_bo, dH_post (reads dH_new, bo; writes d_bo)
 // Backward, dynamic:  pass B reductions dH_pre, dH_res (reads d_bi, dH_new, H)
@@ -51,6 +52,12 @@ int dynw_grad_pass(const void* x, int dtype_x, const float* phi, const float* ro
 constexpr int64_t kLayerBulkRows = 64;
 constexpr int64_t kLayerBulkProjRowsS1 = 64;
 constexpr int64_t kLayerBulkProjElems = (int64_t)1 << 19;  // B * D
+
+// Workgroups of branch_input up to which the epilogue runs in front of it (bi_finalize_kernel).
+// No-grad forwards as graphs, epilogue apart -> in front: B = 128, S = 1, D = 4096 (256 workgroups)
+// 21.5 -> 18.6 us, B = 256 24.5 -> 22.0, B = 512 29.3 -> 27.0, B = 1, S = 512 (1024) 29.1 -> 27.7;
+// at 2048 workgroups equal (38.5, 39.0), at 4096 equal or slower (69.9 -> 70.3).
+constexpr int64_t kFusedEpilogueTiles = 1024;
 
 constexpr int kLU = 1;   // items per lane per tile, streaming passes
 constexpr int kLRU = 2;  // items per lane per tile, the reduction-only pass B
@@ -130,6 +137,80 @@ static int branch_input_any(const void* H, int dtype, const float* w, void* bi, 
     if (h_cached(B, S, D, sizeof(T))) return launch_bi<T, WV, kNtCached>((const T*)H, w, (T*)bi, B, S, D, st);
     return launch_bi<T, WV, kNt>((const T*)H, w, (T*)bi, B, S, D, st);
   });
+}
+
+// branch_input with the Eq. 14-19 epilogue in front, for a call of few tiles (decode, short
+// prompts): the first wave of every workgroup forms its batch's weights from the projection
+// records, as dynw_finalize_kernel does (the same bits), while the tile's H loads are in flight;
+// the batch's first workgroup writes them (w, aux).  The launch that this saves costs as much as
+// the epilogue itself; with many tiles per batch the repeated epilogues would cost more.
+template <typename T, int W, int NT>
+__global__ __launch_bounds__(kThreads) void bi_finalize_kernel(const T* __restrict__ H, const float* __restrict__ part,
+                                                               int nK, int64_t K, DynParams P, float* __restrict__ w,
+                                                               float* __restrict__ aux, T* __restrict__ bi, Geom g,
+                                                               int iters, float eps) {
+  __shared__ float quarter[4][kPart];
+  __shared__ float pre[4];
+  const int64_t b = g.b0 + blockIdx.y;
+  const int64_t D = g.D;
+  const int64_t s_lo = (int64_t)(blockIdx.x * kThreads) / g.nch;
+  const int64_t t0 = b * g.S + s_lo;
+  const int64_t rest = g.S - s_lo;
+  const Span<T, true> hs(H + t0 * 4 * D, rest * 4 * D);
+  const Span<T, true> bis(bi + t0 * D, rest * D);
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  const bool ok = i < g.items;
+  const uint32_t s = ok ? i / g.nch : (uint32_t)s_lo;
+  const uint32_t c = ok ? i - s * g.nch : 0;
+  const uint32_t e1 = (s - (uint32_t)s_lo) * (uint32_t)D + c * W;
+  const uint32_t e4 = (s - (uint32_t)s_lo) * 4 * (uint32_t)D + c * W;
+  Frag<T, W> hf[4];
+  if (ok) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n) hf[n].template load<(NT & 1) != 0>(hs, e4 + n * (uint32_t)D);
+  }
+  loads_issued();
+  if (threadIdx.x < 64) sum_records(part + b * nK * kPart, nK, threadIdx.x, quarter);
+  __syncthreads();
+  if (threadIdx.x < 16) {
+    const int e = threadIdx.x;
+    const float raw_res = row_total(quarter, 8 + e), raw_pp = row_total(quarter, e & 7);
+    const Row16 o = weights_row16(e, raw_res, raw_pp, row_total(quarter, kOut), K, P, iters, eps);
+    if (e < 4) pre[e] = o.pp;
+    if (blockIdx.x == 0)
+      store_row16(e, b, o, raw_res, raw_pp, OutRow{w, kOut}, OutRow{w + 4, kOut}, OutRow{w + 8, kOut}, aux);
+  }
+  __syncthreads();
+  if (!ok) return;
+  float h[4][W], r[W];
+#pragma unroll
+  for (int n = 0; n < 4; ++n) hf[n].unpack(h[n]);
+#pragma unroll
+  for (int e = 0; e < W; ++e) r[e] = pre[0] * h[0][e] + pre[1] * h[1][e] + pre[2] * h[2][e] + pre[3] * h[3][e];
+  st<T, W, (NT & 2) != 0>(bis, e1, r);
+}
+
+// The dynamic forward's last step: the epilogue of the projection records part[b][nK][25] (the
+// weights w and their aux record) and branch_input.
+static int finalize_and_bi(const void* H, int dtype, const float* part, int nK, const DynParams& P, float* w,
+                           float* aux, void* bi, int64_t B, int64_t S, int64_t D, int iters, float eps,
+                           hipStream_t st) {
+  const int64_t K = 4 * D;
+  const int rc = MHC_DISPATCH_DTYPE(dtype, [&] {
+    constexpr int W = Vec<T>::N;
+    if (!vec_ok(D, W, {H, bi})) return -1;
+    const Geom g = make_geom<W, kLU>(S, D, 0);
+    if (g.ntiles == 0 || B * (int64_t)g.ntiles > kFusedEpilogueTiles) return -1;
+    bi_finalize_kernel<T, W, kNtCached><<<dim3(g.ntiles, (unsigned)B), kThreads, 0, st>>>(
+        (const T*)H, part, nK, K, P, w, aux, (T*)bi, g, iters, eps);
+    return hip_status(hipGetLastError(), "layer finalize and branch_input launch");
+  });
+  if (rc != -1) return rc;
+  if (int rc2 = hip_status(launch_finalize(part, nK, B, K, P, OutRow{w, kOut}, OutRow{w + 4, kOut}, OutRow{w + 8, kOut},
+                                           aux, iters, eps, st),
+                           "layer finalize launch"))
+    return rc2;
+  return branch_input_any(H, dtype, w, bi, B, S, D, st);
 }
 
 // Static weights (module.py:108-117), replicated for every batch row:
@@ -367,16 +448,10 @@ static int layer_dynamic_forward_run(const void* H, int dtype, const float* phi,
     if (int rc = s1 ? dynw_project_rows(H, dtype, phi, part, B, K, &nK, st)
                     : dynw_project_rows(xp, MHC_DTYPE_F32, phi, part, B, K, &nK, st))
       return rc;
-    dynw_finalize_rows_kernel<><<<dim3((unsigned)((B + kFinRowsWg - 1) / kFinRowsWg)), kThreads, 0, st>>>(
-        part, nK, B, K, P, OutRow{w, kOut}, OutRow{w + 4, kOut}, OutRow{w + 8, kOut}, aux, iters, eps);
-    if (int rc = hip_status(hipGetLastError(), "layer finalize launch")) return rc;
-    return branch_input_any(H, dtype, w, branch_input, B, S, D, st);
+    return finalize_and_bi(H, dtype, part, nK, P, w, aux, branch_input, B, S, D, iters, eps, st);
   }
   if (int rc = mean_pool_any(H, dtype, x, phi, part, (float*)(wsb + L.colpart), B, S, D, &nK, st)) return rc;
-  dynw_finalize_kernel<><<<dim3((unsigned)((B + 3) / 4)), kThreads, 0, st>>>(
-      part, nK, B, K, P, OutRow{w, kOut}, OutRow{w + 4, kOut}, OutRow{w + 8, kOut}, aux, iters, eps);
-  if (int rc = hip_status(hipGetLastError(), "layer finalize launch")) return rc;
-  return branch_input_any(H, dtype, w, branch_input, B, S, D, st);
+  return finalize_and_bi(H, dtype, part, nK, P, w, aux, branch_input, B, S, D, iters, eps, st);
 }
 
 extern "C" int mhc_layer_dynamic_forward(const void* H, int dtype, const float* phi, const float* H_pre_base,
