@@ -204,6 +204,43 @@ struct Span<T, false> {
   __device__ __forceinline__ Span(const T* base, int64_t) : p(const_cast<T*>(base)) {}
 };
 
+// A span of the ragged path (rows that are not whole 16-byte vectors, or tensors that do not
+// start on one): the same 16-byte accesses at whatever alignment the elements have, which global
+// memory takes on amdhsa (unaligned access mode); only buffer resources are left out.
+template <typename T>
+struct RagSpan {
+  T* p;
+  __device__ __forceinline__ RagSpan(const T* base, int64_t) : p(const_cast<T*>(base)) {}
+};
+typedef u32x4 __attribute__((aligned(2), may_alias)) u32x4_any;
+__device__ __forceinline__ u32x4 load16_any(const void* p, bool nt) {
+  const u32x4_any* q = reinterpret_cast<const u32x4_any*>(p);
+  return nt ? __builtin_nontemporal_load(q) : *q;
+}
+__device__ __forceinline__ void store16_any(void* p, u32x4 v, bool nt) {
+  u32x4_any* q = reinterpret_cast<u32x4_any*>(p);
+  if (nt) __builtin_nontemporal_store(v, q);
+  else *q = v;
+}
+
+// How a kernel addresses a tensor of T: buffer spans on the vector path, RagSpan on the ragged one,
+// a plain pointer for single elements (W = 1).
+template <typename T, int W, bool RAG> struct SpanOf { using type = Span<T, (W > 1)>; };
+template <typename T, int W> struct SpanOf<T, W, true> { using type = RagSpan<T>; };
+
+// The ragged path covers a row of n elements with ceil(n / W) lanes.  The last lane's vector is
+// moved back to end with the row, so its first `skip` elements are also its neighbour's: it computes
+// them too and leaves them out of what it stores and sums.
+template <int W, bool RAG>
+struct RowCol {
+  uint32_t col, skip;
+  __device__ __forceinline__ RowCol(uint32_t c, uint32_t n) {
+    const uint32_t at = c * W;
+    col = RAG ? (at + W > n ? n - W : at) : at;
+    skip = at - col;
+  }
+};
+
 // A workgroup's span of one tensor must stay under 2^31 bytes on the buffer
 // path; `span_elems` is the largest span (in elements) a launch can give it.
 inline bool span_ok(int64_t span_elems, int64_t elem_size) {
@@ -244,6 +281,13 @@ struct Frag {
     } else {
       load<NT>(sp.p + e);
     }
+  }
+
+  template <bool NT>
+  __device__ __forceinline__ void load(const RagSpan<T>& sp, uint32_t e) {
+    static_assert(kVec, "the ragged path moves 16-byte vectors");
+#pragma unroll
+    for (int q = 0; q < W / N; ++q) r[q] = __builtin_bit_cast(Raw, load16_any(sp.p + e + q * N, NT));
   }
 
   __device__ __forceinline__ void unpack(float* f) const {
@@ -293,6 +337,40 @@ __device__ __forceinline__ void st(const Span<T, BUF>& sp, uint32_t e, const flo
     for (int q = 0; q < W / N; ++q) sp.template store16<NT>(e + q * N, RawVec<T>::pack(f + q * N));
   } else {
     st<T, W, NT>(sp.p + e, f);
+  }
+}
+
+// The same, without the first `skip` elements (non-zero on the ragged path's last lane of a row).
+template <typename T, int W, bool NT, typename SP>
+__device__ __forceinline__ void st_from(const SP& sp, uint32_t e, const float* f, uint32_t skip) {
+  if constexpr (__is_same(SP, RagSpan<T>)) {
+    constexpr int N = Vec<T>::N;
+    if (skip == 0) {
+#pragma unroll
+      for (int q = 0; q < W / N; ++q) store16_any(sp.p + e + q * N, RawVec<T>::pack(f + q * N), NT);
+    } else {
+#pragma unroll
+      for (int i = 1; i < W; ++i)
+        if ((uint32_t)i >= skip) sp.p[e + i] = from_f32<T>(f[i]);
+    }
+  } else {
+    st<T, W, NT>(sp, e, f);
+  }
+}
+
+template <typename T, int W, bool NT>
+__device__ __forceinline__ void ld(const RagSpan<T>& sp, uint32_t e, float* f) {
+  Frag<T, W> fr;
+  fr.template load<NT>(sp, e);
+  fr.unpack(f);
+}
+
+// Zeroes the elements that a ragged row's last lane must not sum.
+template <int W, bool RAG>
+__device__ __forceinline__ void drop_skipped(float (&v)[W], uint32_t skip) {
+  if constexpr (RAG) {
+#pragma unroll
+    for (int e = 0; e < W; ++e) v[e] = (uint32_t)e < skip ? 0.f : v[e];
   }
 }
 

@@ -355,7 +355,7 @@ constexpr int kPoolUN = 4;  // rows in flight per lane in colsum_kernel
 constexpr int64_t kPoolDirectRows = 8;
 constexpr int64_t kPoolPlainBytes = (int64_t)64 << 20;  // H up to here is read without the nt policy
 
-template <typename T, int W, bool PROJ>
+template <typename T, int W, bool RAG, bool PROJ>
 static int launch_meanpool(const T* H, float* x, const float* phi, float* projpart, float* colpart, int64_t B,
                            int64_t S, int64_t K, hipStream_t st) {
   const PoolPlan p = pool_plan(B, S, K, W);
@@ -368,10 +368,10 @@ static int launch_meanpool(const T* H, float* x, const float* phi, float* projpa
     // itself (B = 4096, S = 16: 563 -> 419 us; B = 512, S = 64: 242 -> 232).  Longer ones keep
     // colsum_kernel, whose streaming loads read them faster (B = 48, S = 256: 69 against 71 us).
     const bool direct_vec =
-        !PROJ && W > 1 && aligned16(x) && (S <= kPoolDirectRows || (p.nS == 1 && S <= 64));
+        !PROJ && W > 1 && (RAG || aligned16(x)) && (S <= kPoolDirectRows || (p.nS == 1 && S <= 64));
     if (direct_vec || S <= kPoolDirectRows) {
       if (direct_vec)
-        colsum_direct_vec_kernel<T, W><<<dim3((unsigned)p.ncc, (unsigned)nb), kThreads, 0, st>>>(
+        colsum_direct_vec_kernel<T, W, RAG><<<dim3((unsigned)p.ncc, (unsigned)nb), kThreads, 0, st>>>(
             H, x, S, K, p.SC, inv_S, b0);
       else
         colsum_direct_kernel<T, PROJ><<<dim3((unsigned)p.nrc, (unsigned)nb), kThreads, 0, st>>>(
@@ -385,7 +385,7 @@ static int launch_meanpool(const T* H, float* x, const float* phi, float* projpa
     // at config 4, against all plain).  An H of up to 64 MB stays there whole, and all plain is
     // 1-2 us faster at 33 MB (the two passes 28.4 -> 27.3 us) and equal at 67 MB.
     const bool all_plain = B * S * K * (int64_t)sizeof(T) <= kPoolPlainBytes;
-    colsum_kernel<T, W, kPoolUN><<<dim3((unsigned)p.ncc, (unsigned)p.nS, (unsigned)nb), kThreads, 0, st>>>(
+    colsum_kernel<T, W, kPoolUN, RAG><<<dim3((unsigned)p.ncc, (unsigned)p.nS, (unsigned)nb), kThreads, 0, st>>>(
         H, colpart, S, K, p.SC, p.nS, all_plain ? 0 : p.SC / 2, b0);
     if (int rc = hip_status(hipGetLastError(), "mean_pool column-sum launch")) return rc;
     colsum_reduce_kernel<PROJ><<<dim3((unsigned)p.nrc, (unsigned)nb), kThreads, 0, st>>>(
@@ -398,12 +398,6 @@ static int launch_meanpool(const T* H, float* x, const float* phi, float* projpa
 static bool pool_vec(int dtype, int64_t K, const void* H) {
   const int W = dtype == MHC_DTYPE_F32 ? 4 : 8;
   return K % W == 0 && aligned16(H) && span_ok(kPoolUN * K, 4);
-}
-
-PoolPlan mean_pool_plan(int dtype, int64_t B, int64_t S, int64_t D, const void* H) {
-  const int64_t K = 4 * D;
-  const int W = (H == nullptr || pool_vec(dtype, K, H)) ? (dtype == MHC_DTYPE_F32 ? 4 : 8) : 1;
-  return pool_plan(B, S, K, W);
 }
 
 // Column-partial workspace of the mean-pool: the largest plan over the vector
@@ -429,12 +423,16 @@ int mean_pool_any(const void* H, int dtype, float* x, const float* phi, float* p
   if (nrc) *nrc = (int)pool_plan(B, S, K, 1).nrc;
   return MHC_DISPATCH_DTYPE(dtype, [&] {
     constexpr int WV = Vec<T>::N;
-    if (phi) {
-      if (vec) return launch_meanpool<T, WV, true>((const T*)H, x, phi, projpart, colpart, B, S, K, st);
-      return launch_meanpool<T, 1, true>((const T*)H, x, phi, projpart, colpart, B, S, K, st);
-    }
-    if (vec) return launch_meanpool<T, WV, false>((const T*)H, x, nullptr, nullptr, colpart, B, S, K, st);
-    return launch_meanpool<T, 1, false>((const T*)H, x, nullptr, nullptr, colpart, B, S, K, st);
+    auto go = [&](auto w_, auto rag_) {
+      constexpr int W = decltype(w_)::value;
+      constexpr bool RAG = decltype(rag_)::value;
+      if (phi) return launch_meanpool<T, W, RAG, true>((const T*)H, x, phi, projpart, colpart, B, S, K, st);
+      return launch_meanpool<T, W, RAG, false>((const T*)H, x, nullptr, nullptr, colpart, B, S, K, st);
+    };
+    if (vec) return go(std::integral_constant<int, WV>{}, std::false_type{});
+    // ragged: K = 4 D is not whole vectors (odd D in 16 bits), or H does not start on one
+    if (rag_ok(B * S * D, K, WV) && span_ok(kPoolUN * K, 4)) return go(std::integral_constant<int, WV>{}, std::true_type{});
+    return go(std::integral_constant<int, 1>{}, std::false_type{});
   });
 }
 

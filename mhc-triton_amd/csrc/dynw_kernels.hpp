@@ -1213,11 +1213,11 @@ __global__ __launch_bounds__(kThreads) void dynw_gphi_reduce_kernel(const float*
 // chunk are read with the streaming (nt) policy, the rest plain: what
 // branch_input reads next and can find in the 256 MB memory-side cache is the
 // tail of every chunk, and nt on the rest speeds this read up.
-template <bool NT, typename T, int W, int UN, bool BUF>
+template <bool NT, typename T, int W, int UN, bool RAG>
 __device__ __forceinline__ void colsum_rows(const T* base, int64_t K, uint32_t lane_e, int64_t& s, int64_t end,
                                             float* acc) {
   for (; s + (UN - 1) < end; s += UN) {
-    const Span<T, BUF> sp(base + s * K, (int64_t)UN * K);
+    const typename SpanOf<T, W, RAG>::type sp(base + s * K, (int64_t)UN * K);
     float v[UN][W];
 #pragma unroll
     for (int u = 0; u < UN; ++u) ld<T, W, NT>(sp, (uint32_t)(u * K) + lane_e, v[u]);
@@ -1227,7 +1227,7 @@ __device__ __forceinline__ void colsum_rows(const T* base, int64_t K, uint32_t l
       for (int e = 0; e < W; ++e) acc[e] += v[u][e];
   }
   for (; s < end; ++s) {
-    const Span<T, BUF> sp(base + s * K, K);
+    const typename SpanOf<T, W, RAG>::type sp(base + s * K, K);
     float v[W];
     ld<T, W, NT>(sp, lane_e, v);
 #pragma unroll
@@ -1235,15 +1235,16 @@ __device__ __forceinline__ void colsum_rows(const T* base, int64_t K, uint32_t l
   }
 }
 
-template <typename T, int W, int UN, bool BUF = (W > 1)>
+template <typename T, int W, int UN, bool RAG = false>
 __global__ __launch_bounds__(kThreads) void colsum_kernel(const T* __restrict__ H, float* __restrict__ colpart,
                                                           int64_t S, int64_t K, int64_t SC, int nS, int64_t nt_rows,
                                                           int64_t b0) {
   const int64_t b = b0 + blockIdx.z;
   const int sc = blockIdx.y;
   const int64_t cblk = (int64_t)blockIdx.x * (kThreads * W);
-  const int64_t col = cblk + (int64_t)threadIdx.x * W;
-  if (col >= K) return;
+  if (cblk + (int64_t)threadIdx.x * W >= K) return;
+  const RowCol<W, RAG> rc(threadIdx.x, (uint32_t)(K - cblk < kThreads * W ? K - cblk : kThreads * W));
+  const int64_t col = cblk + rc.col;
   const int64_t sbeg = (int64_t)sc * SC;
   const int64_t send = sbeg + SC < S ? sbeg + SC : S;
   const int64_t smid = sbeg + nt_rows < send ? sbeg + nt_rows : send;
@@ -1251,11 +1252,13 @@ __global__ __launch_bounds__(kThreads) void colsum_kernel(const T* __restrict__ 
 #pragma unroll
   for (int e = 0; e < W; ++e) acc[e] = 0.f;
   const T* base = H + b * S * K + cblk;
-  const uint32_t lane_e = (uint32_t)threadIdx.x * W;
+  const uint32_t lane_e = rc.col;
   int64_t s = sbeg;
-  colsum_rows<true, T, W, UN, BUF>(base, K, lane_e, s, smid, acc);
-  colsum_rows<false, T, W, UN, BUF>(base, K, lane_e, s, send, acc);
-  st<float, W>(colpart + ((b * nS + sc) * K + col), acc);
+  colsum_rows<true, T, W, UN, RAG>(base, K, lane_e, s, smid, acc);
+  colsum_rows<false, T, W, UN, RAG>(base, K, lane_e, s, send, acc);
+  float* out = colpart + ((b * nS + sc) * K + col);
+  if constexpr (RAG) st_from<float, W, false>(RagSpan<float>(out, W), 0u, acc, rc.skip);
+  else st<float, W>(out, acc);
 }
 
 template <bool PROJ>
@@ -1338,13 +1341,15 @@ __global__ __launch_bounds__(kThreads) void colsum_direct_kernel(const T* __rest
 // workgroup per 256 W columns of a batch instead of per 256: at B = 4096, S = 1,
 // D = 4096 the one-column form launched 262,144 workgroups); the per-column sums
 // are the same operations, so the bits are too.
-template <typename T, int W>
+template <typename T, int W, bool RAG>
 __global__ __launch_bounds__(kThreads) void colsum_direct_vec_kernel(const T* __restrict__ H, float* __restrict__ x,
                                                                      int64_t S, int64_t K, int64_t SC, float inv_S,
                                                                      int64_t b0) {
   const int64_t b = b0 + blockIdx.y;
-  const int64_t c = ((int64_t)blockIdx.x * kThreads + threadIdx.x) * W;
-  if (c >= K) return;
+  const int64_t cblk = (int64_t)blockIdx.x * (kThreads * W);
+  if (cblk + (int64_t)threadIdx.x * W >= K) return;
+  const RowCol<W, RAG> rc(threadIdx.x, (uint32_t)(K - cblk < kThreads * W ? K - cblk : kThreads * W));
+  const int64_t c = cblk + rc.col;
   const T* p = H + b * S * K + c;
   float v[W];
 #pragma unroll
@@ -1357,7 +1362,8 @@ __global__ __launch_bounds__(kThreads) void colsum_direct_vec_kernel(const T* __
 #pragma unroll 4
     for (int64_t s = s0; s < s1; ++s) {
       float f[W];
-      ld<T, W>(p + s * K, f);
+      if constexpr (RAG) ld<T, W, false>(RagSpan<T>(p + s * K, W), 0u, f);
+      else ld<T, W>(p + s * K, f);
 #pragma unroll
       for (int e = 0; e < W; ++e) a[e] += f[e];
     }
@@ -1366,7 +1372,8 @@ __global__ __launch_bounds__(kThreads) void colsum_direct_vec_kernel(const T* __
   }
 #pragma unroll
   for (int e = 0; e < W; ++e) v[e] *= inv_S;
-  st<float, W>(x + b * K + c, v);
+  if constexpr (RAG) st_from<float, W, false>(RagSpan<float>(x + b * K + c, W), 0u, v, rc.skip);
+  else st<float, W>(x + b * K + c, v);
 }
 
 // Launch plan of the two mean-pool kernels; depends only on the shape, so

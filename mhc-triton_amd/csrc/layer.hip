@@ -116,12 +116,12 @@ static bool h_cached(int64_t B, int64_t S, int64_t D, size_t esize) {
 constexpr int kNtCached = 2;  // plain loads, nt stores
 constexpr int fwd_wgs(bool cached) { return cached ? 6 : 3; }
 
-template <typename T, int W, int NT>
+template <typename T, int W, int NT, bool RAG>
 static int launch_bi(const T* H, const float* w, T* bi, int64_t B, int64_t S, int64_t D, hipStream_t st) {
   return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
     const Geom g = make_geom<W, kLU>(S, D, b0);
     if (g.ntiles == 0) return (int)MHC_OK;
-    mix_fwd_kernel<T, T, W, kLU, true, false, false, NT>
+    mix_fwd_kernel<T, T, W, kLU, true, false, false, NT, RAG>
         <<<dim3(g.ntiles, nb), kThreads, occupancy_lds(fwd_wgs(NT == kNtCached)), st>>>(
             H, (const T*)nullptr, WRow{w, kOut}, WRow{nullptr, 0}, WRow{nullptr, 0}, bi, nullptr, g);
     return hip_status(hipGetLastError(), "layer branch_input launch");
@@ -132,10 +132,13 @@ static int branch_input_any(const void* H, int dtype, const float* w, void* bi, 
                             hipStream_t st) {
   if (S * D == 0) return MHC_OK;
   return MHC_DISPATCH_DTYPE(dtype, [&] {
-    constexpr int WV = Vec<T>::N;
-    if (!vec_ok(D, WV, {H, bi})) return launch_bi<T, 1, kNt>((const T*)H, w, (T*)bi, B, S, D, st);
-    if (h_cached(B, S, D, sizeof(T))) return launch_bi<T, WV, kNtCached>((const T*)H, w, (T*)bi, B, S, D, st);
-    return launch_bi<T, WV, kNt>((const T*)H, w, (T*)bi, B, S, D, st);
+    return with_width<Vec<T>::N>(B, S, D, {H, bi}, [&](auto w_, auto rag_) {
+      constexpr int W = decltype(w_)::value;
+      constexpr bool RAG = decltype(rag_)::value;
+      if (W > 1 && h_cached(B, S, D, sizeof(T)))
+        return launch_bi<T, W, (W > 1 ? kNtCached : kNt), RAG>((const T*)H, w, (T*)bi, B, S, D, st);
+      return launch_bi<T, W, kNt, RAG>((const T*)H, w, (T*)bi, B, S, D, st);
+    });
   });
 }
 
@@ -144,7 +147,7 @@ static int branch_input_any(const void* H, int dtype, const float* w, void* bi, 
 // records, as dynw_finalize_kernel does (the same bits), while the tile's H loads are in flight;
 // the batch's first workgroup writes them (w, aux).  The launch that this saves costs as much as
 // the epilogue itself; with many tiles per batch the repeated epilogues would cost more.
-template <typename T, int W, int NT>
+template <typename T, int W, int NT, bool RAG>
 __global__ __launch_bounds__(kThreads) void bi_finalize_kernel(const T* __restrict__ H, const float* __restrict__ part,
                                                                int nK, int64_t K, DynParams P, float* __restrict__ w,
                                                                float* __restrict__ aux, T* __restrict__ bi, Geom g,
@@ -156,14 +159,14 @@ __global__ __launch_bounds__(kThreads) void bi_finalize_kernel(const T* __restri
   const int64_t s_lo = (int64_t)(blockIdx.x * kThreads) / g.nch;
   const int64_t t0 = b * g.S + s_lo;
   const int64_t rest = g.S - s_lo;
-  const Span<T, true> hs(H + t0 * 4 * D, rest * 4 * D);
-  const Span<T, true> bis(bi + t0 * D, rest * D);
+  const typename SpanOf<T, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
+  const typename SpanOf<T, W, RAG>::type bis(bi + t0 * D, rest * D);
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   const bool ok = i < g.items;
   const uint32_t s = ok ? i / g.nch : (uint32_t)s_lo;
-  const uint32_t c = ok ? i - s * g.nch : 0;
-  const uint32_t e1 = (s - (uint32_t)s_lo) * (uint32_t)D + c * W;
-  const uint32_t e4 = (s - (uint32_t)s_lo) * 4 * (uint32_t)D + c * W;
+  const RowCol<W, RAG> rc(ok ? i - s * g.nch : 0, (uint32_t)D);
+  const uint32_t e1 = (s - (uint32_t)s_lo) * (uint32_t)D + rc.col;
+  const uint32_t e4 = (s - (uint32_t)s_lo) * 4 * (uint32_t)D + rc.col;
   Frag<T, W> hf[4];
   if (ok) {
 #pragma unroll
@@ -187,7 +190,7 @@ __global__ __launch_bounds__(kThreads) void bi_finalize_kernel(const T* __restri
   for (int n = 0; n < 4; ++n) hf[n].unpack(h[n]);
 #pragma unroll
   for (int e = 0; e < W; ++e) r[e] = pre[0] * h[0][e] + pre[1] * h[1][e] + pre[2] * h[2][e] + pre[3] * h[3][e];
-  st<T, W, (NT & 2) != 0>(bis, e1, r);
+  st_from<T, W, (NT & 2) != 0>(bis, e1, r, rc.skip);
 }
 
 // The dynamic forward's last step: the epilogue of the projection records part[b][nK][25] (the
@@ -197,13 +200,14 @@ static int finalize_and_bi(const void* H, int dtype, const float* part, int nK, 
                            hipStream_t st) {
   const int64_t K = 4 * D;
   const int rc = MHC_DISPATCH_DTYPE(dtype, [&] {
-    constexpr int W = Vec<T>::N;
-    if (!vec_ok(D, W, {H, bi})) return -1;
-    const Geom g = make_geom<W, kLU>(S, D, 0);
-    if (g.ntiles == 0 || B * (int64_t)g.ntiles > kFusedEpilogueTiles) return -1;
-    bi_finalize_kernel<T, W, kNtCached><<<dim3(g.ntiles, (unsigned)B), kThreads, 0, st>>>(
-        (const T*)H, part, nK, K, P, w, aux, (T*)bi, g, iters, eps);
-    return hip_status(hipGetLastError(), "layer finalize and branch_input launch");
+    return with_width<Vec<T>::N>(B, S, D, {H, bi}, [&](auto w_, auto rag_) {
+      constexpr int W = decltype(w_)::value;
+      const Geom g = make_geom<W, kLU>(S, D, 0);
+      if (g.ntiles == 0 || B * (int64_t)g.ntiles > kFusedEpilogueTiles) return -1;
+      bi_finalize_kernel<T, W, kNtCached, decltype(rag_)::value><<<dim3(g.ntiles, (unsigned)B), kThreads, 0, st>>>(
+          (const T*)H, part, nK, K, P, w, aux, (T*)bi, g, iters, eps);
+      return hip_status(hipGetLastError(), "layer finalize and branch_input launch");
+    });
   });
   if (rc != -1) return rc;
   if (int rc2 = hip_status(launch_finalize(part, nK, B, K, P, OutRow{w, kOut}, OutRow{w + 4, kOut}, OutRow{w + 8, kOut},
@@ -286,7 +290,7 @@ __global__ __launch_bounds__(kThreads) void static_weights_bwd_kernel(
 
 // Pass B (REDUCE only), the static pass BC (REDUCE + WRITE_DH) and the
 // generic mix backward share mix_bwd_kernel.
-template <typename T, int W, bool HAS_DHN, bool REDUCE, bool WRITE_DH>
+template <typename T, int W, bool RAG, bool HAS_DHN, bool REDUCE, bool WRITE_DH>
 static int launch_mix_bwd(const T* dbi, const T* dhn, const T* H, const float* w, T* dH, float* part, int64_t B,
                           int64_t S, int64_t D, uint32_t* nblk_out, hipStream_t st) {
   // Pass B writes nothing bulk: two items per lane, full occupancy, workgroups
@@ -305,7 +309,7 @@ static int launch_mix_bwd(const T* dbi, const T* dhn, const T* H, const float* w
     const Geom g = make_geom<W, U>(S, D, b0);
     // Pass B (REDUCE only): nt on the H loads alone; d_bi and dH_new are read again by pass C.
     constexpr int NT = WRITE_DH ? kNt : 4;
-    mix_bwd_kernel<T, W, U, HAS_DHN, REDUCE, WRITE_DH, NT, (W > 1), ONE><<<dim3(nblk, nb), kThreads, lds, st>>>(
+    mix_bwd_kernel<T, W, U, HAS_DHN, REDUCE, WRITE_DH, NT, RAG, ONE><<<dim3(nblk, nb), kThreads, lds, st>>>(
         dbi, dhn, H, WRow{w, kOut}, WRow{w + 8, kOut}, dH, part, g);
     return hip_status(hipGetLastError(), "layer mix backward launch");
   });
@@ -314,20 +318,15 @@ static int launch_mix_bwd(const T* dbi, const T* dhn, const T* H, const float* w
 template <typename T, bool REDUCE, bool WRITE_DH>
 static int mix_bwd_dispatch(const void* dbi, const void* dhn, const void* H, const float* w, void* dH, float* part,
                             int64_t B, int64_t S, int64_t D, uint32_t* nblk, hipStream_t st) {
-  constexpr int WV = Vec<T>::N;
-  const bool vec = vec_ok(D, WV, {dbi, dhn, H, dH});
-  if (dhn) {
-    if (vec)
-      return launch_mix_bwd<T, WV, true, REDUCE, WRITE_DH>((const T*)dbi, (const T*)dhn, (const T*)H, w, (T*)dH,
-                                                           part, B, S, D, nblk, st);
-    return launch_mix_bwd<T, 1, true, REDUCE, WRITE_DH>((const T*)dbi, (const T*)dhn, (const T*)H, w, (T*)dH, part,
-                                                        B, S, D, nblk, st);
-  }
-  if (vec)
-    return launch_mix_bwd<T, WV, false, REDUCE, WRITE_DH>((const T*)dbi, nullptr, (const T*)H, w, (T*)dH, part, B,
-                                                          S, D, nblk, st);
-  return launch_mix_bwd<T, 1, false, REDUCE, WRITE_DH>((const T*)dbi, nullptr, (const T*)H, w, (T*)dH, part, B, S,
-                                                       D, nblk, st);
+  return with_width<Vec<T>::N>(B, S, D, {dbi, dhn, H, dH}, [&](auto w_, auto rag_) {
+    constexpr int W = decltype(w_)::value;
+    constexpr bool RAG = decltype(rag_)::value;
+    if (dhn)
+      return launch_mix_bwd<T, W, RAG, true, REDUCE, WRITE_DH>((const T*)dbi, (const T*)dhn, (const T*)H, w, (T*)dH,
+                                                               part, B, S, D, nblk, st);
+    return launch_mix_bwd<T, W, RAG, false, REDUCE, WRITE_DH>((const T*)dbi, nullptr, (const T*)H, w, (T*)dH, part, B,
+                                                              S, D, nblk, st);
+  });
 }
 
 // Pass C of the dynamic backward: TT tokens per lane, grad_x loaded once for all of them, 2
@@ -342,47 +341,45 @@ static int mix_bwd_dispatch(const void* dbi, const void* dhn, const void* H, con
 // S = 16: 1.7 us more).
 static int dh_tokens(int64_t B, int64_t S, int64_t D, int W) {
   for (int tt = S <= 2 ? 2 : (S <= 4 ? 4 : (S <= 16 ? 8 : 2)); tt > 2; tt /= 2)
-    if (B * ((S + tt - 1) / tt) * (D / W) >= 1024 * (int64_t)kThreads) return tt;
+    if (B * ((S + tt - 1) / tt) * ((D + W - 1) / W) >= 1024 * (int64_t)kThreads) return tt;
   return 2;
 }
 
-template <typename T, int W, bool HAS_DHN, int TT>
+template <typename T, int W, bool RAG, bool HAS_DHN, int TT>
 static int launch_dh(const T* dbi, const T* dhn, const float* gx, const float* w, T* dH, int64_t B, int64_t S,
                      int64_t D, hipStream_t st) {
   const int64_t groups = (S + TT - 1) / TT;
-  const int64_t items = groups * (D / W);  // (token group, column vector) pairs, < 2^32 by check_bsd
+  const int64_t items = groups * ((D + W - 1) / W);  // (token group, column vector) pairs, < 2^32 by check_bsd
   if (items == 0) return MHC_OK;
   const unsigned nwg = (unsigned)((items + kThreads - 1) / kThreads);
   const float inv_S = 1.f / (float)S;
   return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
-    dh_kernel<T, W, TT, HAS_DHN, kNt><<<dim3(nwg, (unsigned)nb), kThreads, occupancy_lds(2), st>>>(
+    dh_kernel<T, W, TT, HAS_DHN, kNt, RAG><<<dim3(nwg, (unsigned)nb), kThreads, occupancy_lds(2), st>>>(
         dbi, dhn, gx, inv_S, WRow{w, kOut}, WRow{w + 8, kOut}, dH, S, D, (uint32_t)groups, b0);
     return hip_status(hipGetLastError(), "layer dH launch");
   });
 }
 
-template <typename T, int W, bool HAS_DHN>
+template <typename T, int W, bool RAG, bool HAS_DHN>
 static int launch_dh_tt(int tt, const T* dbi, const T* dhn, const float* gx, const float* w, T* dH, int64_t B,
                         int64_t S, int64_t D, hipStream_t st) {
-  if (tt == 8) return launch_dh<T, W, HAS_DHN, 8>(dbi, dhn, gx, w, dH, B, S, D, st);
-  if (tt == 4) return launch_dh<T, W, HAS_DHN, 4>(dbi, dhn, gx, w, dH, B, S, D, st);
-  return launch_dh<T, W, HAS_DHN, 2>(dbi, dhn, gx, w, dH, B, S, D, st);
+  if (tt == 8) return launch_dh<T, W, RAG, HAS_DHN, 8>(dbi, dhn, gx, w, dH, B, S, D, st);
+  if (tt == 4) return launch_dh<T, W, RAG, HAS_DHN, 4>(dbi, dhn, gx, w, dH, B, S, D, st);
+  return launch_dh<T, W, RAG, HAS_DHN, 2>(dbi, dhn, gx, w, dH, B, S, D, st);
 }
 
 template <typename T>
 static int dh_dispatch(const void* dbi, const void* dhn, const float* gx, const float* w, void* dH, int64_t B,
                        int64_t S, int64_t D, hipStream_t st) {
-  constexpr int WV = Vec<T>::N;
-  const bool vec = vec_ok(D, WV, {dbi, dhn, dH}) && aligned16(gx);
-  int tt = dh_tokens(B, S, D, vec ? WV : 1);
-  // a tile's buffer spans grow with the tokens per lane (vec_ok bounds them for two)
-  if (vec && !span_ok(tt / 2 * (16384 + 8 * D), 4)) tt = 2;
-  if (dhn) {
-    if (vec) return launch_dh_tt<T, WV, true>(tt, (const T*)dbi, (const T*)dhn, gx, w, (T*)dH, B, S, D, st);
-    return launch_dh_tt<T, 1, true>(tt, (const T*)dbi, (const T*)dhn, gx, w, (T*)dH, B, S, D, st);
-  }
-  if (vec) return launch_dh_tt<T, WV, false>(tt, (const T*)dbi, nullptr, gx, w, (T*)dH, B, S, D, st);
-  return launch_dh_tt<T, 1, false>(tt, (const T*)dbi, nullptr, gx, w, (T*)dH, B, S, D, st);
+  return with_width<Vec<T>::N>(B, S, D, {dbi, dhn, dH, gx}, [&](auto w_, auto rag_) {
+    constexpr int W = decltype(w_)::value;
+    constexpr bool RAG = decltype(rag_)::value;
+    int tt = dh_tokens(B, S, D, W);
+    // a tile's spans grow with the tokens per lane (vec_ok bounds them for two)
+    if (W > 1 && !span_ok(tt / 2 * (16384 + 8 * D), 4)) tt = 2;
+    if (dhn) return launch_dh_tt<T, W, RAG, true>(tt, (const T*)dbi, (const T*)dhn, gx, w, (T*)dH, B, S, D, st);
+    return launch_dh_tt<T, W, RAG, false>(tt, (const T*)dbi, nullptr, gx, w, (T*)dH, B, S, D, st);
+  });
 }
 
 }  // namespace mhc
@@ -569,26 +566,26 @@ extern "C" int mhc_layer_add_forward(const void* H, int dtype_h, const void* bra
   hipStream_t st = (hipStream_t)stream;
   return MHC_DISPATCH_DTYPE2(dtype_h, dtype_bo, [&] {
     constexpr int WV = Vec<TH>::N > Vec<TB>::N ? Vec<TH>::N : Vec<TB>::N;
-    auto go = [&](auto wtag, auto nttag) {
-      constexpr int W = decltype(wtag)::value;
-      constexpr int NT = decltype(nttag)::value;
-      return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
-        const Geom g = make_geom<W, kLU>(S, D, b0);
-        // With the nt policy 3 workgroups per CU: 188.5 us at config-3 size against 194.9 with 2
-        // and 190.4 with 4 when chosen; with the buffer-span loads caps 2 and 3 time alike and 4
-        // is about 1 us slower (192.6-195.4 us event-timed in the bench).
-        mix_fwd_kernel<TH, TB, W, kLU, false, true, true, NT>
-            <<<dim3(g.ntiles, nb), kThreads, occupancy_lds(fwd_wgs(NT == kNtCached)), st>>>(
-            (const TH*)H, (const TB*)branch_output, WRow{nullptr, 0}, WRow{w + 8, kOut}, WRow{w + 4, kOut},
-            nullptr, (TH*)H_new, g);
-        return hip_status(hipGetLastError(), "layer add forward launch");
-      });
-    };
-    using Stream = std::integral_constant<int, kNt>;
-    if (!vec_ok(D, WV, {H, branch_output, H_new})) return go(std::integral_constant<int, 1>{}, Stream{});
-    if (h_cached(B, S, D, sizeof(TH)))
-      return go(std::integral_constant<int, WV>{}, std::integral_constant<int, kNtCached>{});
-    return go(std::integral_constant<int, WV>{}, Stream{});
+    return with_width<WV>(B, S, D, {H, branch_output, H_new}, [&](auto w_, auto rag_) {
+      constexpr int W = decltype(w_)::value;
+      constexpr bool RAG = decltype(rag_)::value;
+      auto go = [&](auto nt_) {
+        constexpr int NT = decltype(nt_)::value;
+        return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
+          const Geom g = make_geom<W, kLU>(S, D, b0);
+          // With the nt policy 3 workgroups per CU: 188.5 us at config-3 size against 194.9 with 2
+          // and 190.4 with 4 when chosen; with the buffer-span loads caps 2 and 3 time alike and 4
+          // is about 1 us slower (192.6-195.4 us event-timed in the bench).
+          mix_fwd_kernel<TH, TB, W, kLU, false, true, true, NT, RAG>
+              <<<dim3(g.ntiles, nb), kThreads, occupancy_lds(fwd_wgs(NT == kNtCached)), st>>>(
+                  (const TH*)H, (const TB*)branch_output, WRow{nullptr, 0}, WRow{w + 8, kOut}, WRow{w + 4, kOut},
+                  nullptr, (TH*)H_new, g);
+          return hip_status(hipGetLastError(), "layer add forward launch");
+        });
+      };
+      if (W > 1 && h_cached(B, S, D, sizeof(TH))) return go(std::integral_constant<int, (W > 1 ? kNtCached : kNt)>{});
+      return go(std::integral_constant<int, kNt>{});
+    });
   });
 }
 

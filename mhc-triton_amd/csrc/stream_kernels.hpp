@@ -53,7 +53,7 @@ struct WRow {
 
 struct Geom {
   int64_t S, D;   // sequence, per-stream dim
-  uint32_t nch;   // D / W
+  uint32_t nch;   // ceil(D / W)
   uint32_t items; // S * nch
   uint32_t ntiles;
   int64_t b0;     // first batch of this launch
@@ -64,8 +64,8 @@ __host__ inline Geom make_geom(int64_t S, int64_t D, int64_t b0) {
   Geom g;
   g.S = S;
   g.D = D;
-  g.nch = (uint32_t)(D / W);
-  g.items = (uint32_t)(S * (D / W));
+  g.nch = (uint32_t)((D + W - 1) / W);
+  g.items = (uint32_t)(S * ((D + W - 1) / W));
   g.ntiles = (g.items + kThreads * U - 1) / (kThreads * U);
   g.b0 = b0;
   return g;
@@ -89,7 +89,7 @@ __device__ __forceinline__ void load_w16(WRow w, int64_t b, float (&v)[16]) {
 // Used for fused_stream_mix (BI + RES), the layer's branch_input pass (BI)
 // and the layer closure (RES + ADD_BO, H_residual never stored).
 // ---------------------------------------------------------------------------
-template <typename T, typename TB, int W, int U, bool BI, bool RES, bool ADD_BO, int NT = 0, bool BUF = (W > 1)>
+template <typename T, typename TB, int W, int U, bool BI, bool RES, bool ADD_BO, int NT = 0, bool RAG = false>
 __global__ __launch_bounds__(kThreads) void mix_fwd_kernel(const T* __restrict__ H, const TB* __restrict__ bo,
                                                            WRow pre, WRow res, WRow post, T* __restrict__ bi,
                                                            T* __restrict__ out, Geom g) {
@@ -101,25 +101,26 @@ __global__ __launch_bounds__(kThreads) void mix_fwd_kernel(const T* __restrict__
   const int64_t s_lo = (int64_t)(tile * (kThreads * U)) / g.nch;
   const int64_t t0 = b * g.S + s_lo;
   const int64_t rest = g.S - s_lo;
-  const Span<T, BUF> hs(H + t0 * 4 * D, rest * 4 * D);
+  const typename SpanOf<T, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
   Frag<T, W> hf[U][4];
   Frag<TB, W> bf[U];
-  uint32_t e4[U], e1[U];  // element offsets in the [.,4,D] and [.,D] spans
+  uint32_t e4[U], e1[U], skip[U];  // element offsets in the [.,4,D] and [.,D] spans
   bool ok[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t i = tile * (kThreads * U) + u * kThreads + threadIdx.x;
     ok[u] = i < g.items;
     const uint32_t s = ok[u] ? i / g.nch : (uint32_t)s_lo;
-    const uint32_t c = ok[u] ? i - s * g.nch : 0;
+    const RowCol<W, RAG> rc(ok[u] ? i - s * g.nch : 0, (uint32_t)D);
     const uint32_t ds = s - (uint32_t)s_lo;
-    e4[u] = ds * 4 * (uint32_t)D + c * W;
-    e1[u] = ds * (uint32_t)D + c * W;
+    e4[u] = ds * 4 * (uint32_t)D + rc.col;
+    e1[u] = ds * (uint32_t)D + rc.col;
+    skip[u] = rc.skip;
     if (ok[u]) {
 #pragma unroll
       for (int n = 0; n < 4; ++n) hf[u][n].template load<(NT & 1) != 0>(hs, e4[u] + n * (uint32_t)D);
       if constexpr (ADD_BO) {
-        const Span<TB, BUF> bs(bo + t0 * D, rest * D);
+        const typename SpanOf<TB, W, RAG>::type bs(bo + t0 * D, rest * D);
         bf[u].template load<(NT & 1) != 0>(bs, e1[u]);
       }
     }
@@ -143,11 +144,11 @@ __global__ __launch_bounds__(kThreads) void mix_fwd_kernel(const T* __restrict__
 #pragma unroll
       for (int e = 0; e < W; ++e)
         r[e] = wp[0] * h[0][e] + wp[1] * h[1][e] + wp[2] * h[2][e] + wp[3] * h[3][e];
-      const Span<T, BUF> bis(bi + t0 * D, rest * D);
-      st<T, W, (NT & 2) != 0>(bis, e1[u], r);
+      const typename SpanOf<T, W, RAG>::type bis(bi + t0 * D, rest * D);
+      st_from<T, W, (NT & 2) != 0>(bis, e1[u], r, skip[u]);
     }
     if constexpr (RES) {
-      const Span<T, BUF> os(out + t0 * 4 * D, rest * 4 * D);
+      const typename SpanOf<T, W, RAG>::type os(out + t0 * 4 * D, rest * 4 * D);
 #pragma unroll
       for (int n = 0; n < 4; ++n) {
         float r[W];
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(kThreads) void mix_fwd_kernel(const T* __restrict__
           if constexpr (ADD_BO) v += wq[n] * bv[e];
           r[e] = v;
         }
-        st<T, W, (NT & 2) != 0>(os, e4[u] + n * (uint32_t)D, r);
+        st_from<T, W, (NT & 2) != 0>(os, e4[u] + n * (uint32_t)D, r, skip[u]);
       }
     }
   }
@@ -168,7 +169,7 @@ __global__ __launch_bounds__(kThreads) void mix_fwd_kernel(const T* __restrict__
 // Add residual forward from a materialised H_residual (fused_add_residual):
 //   out[s,n,:] = hr[s,n,:] + post[n] bo[s,:]
 // ---------------------------------------------------------------------------
-template <typename T, typename TB, int W, int U, int NT = 0, bool BUF = (W > 1)>
+template <typename T, typename TB, int W, int U, int NT = 0, bool RAG = false>
 __global__ __launch_bounds__(kThreads) void add_residual_fwd_kernel(const T* __restrict__ hr,
                                                                     const TB* __restrict__ bo, WRow post,
                                                                     T* __restrict__ out, Geom g) {
@@ -179,30 +180,31 @@ __global__ __launch_bounds__(kThreads) void add_residual_fwd_kernel(const T* __r
   const int64_t s_lo = (int64_t)(tile * (kThreads * U)) / g.nch;
   const int64_t t0 = b * g.S + s_lo;
   const int64_t rest = g.S - s_lo;
-  const Span<T, BUF> hs(hr + t0 * 4 * D, rest * 4 * D);
-  const Span<TB, BUF> bs(bo + t0 * D, rest * D);
+  const typename SpanOf<T, W, RAG>::type hs(hr + t0 * 4 * D, rest * 4 * D);
+  const typename SpanOf<TB, W, RAG>::type bs(bo + t0 * D, rest * D);
   Frag<T, W> hf[U][4];
   Frag<TB, W> bf[U];
-  uint32_t e4[U];
+  uint32_t e4[U], skip[U];
   bool ok[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const uint32_t i = tile * (kThreads * U) + u * kThreads + threadIdx.x;
     ok[u] = i < g.items;
     const uint32_t s = ok[u] ? i / g.nch : (uint32_t)s_lo;
-    const uint32_t c = ok[u] ? i - s * g.nch : 0;
+    const RowCol<W, RAG> rc(ok[u] ? i - s * g.nch : 0, (uint32_t)D);
     const uint32_t ds = s - (uint32_t)s_lo;
-    e4[u] = ds * 4 * (uint32_t)D + c * W;
+    e4[u] = ds * 4 * (uint32_t)D + rc.col;
+    skip[u] = rc.skip;
     if (ok[u]) {
 #pragma unroll
       for (int n = 0; n < 4; ++n) hf[u][n].template load<(NT & 1) != 0>(hs, e4[u] + n * (uint32_t)D);
-      bf[u].template load<(NT & 1) != 0>(bs, ds * (uint32_t)D + c * W);
+      bf[u].template load<(NT & 1) != 0>(bs, ds * (uint32_t)D + rc.col);
     }
   }
   loads_issued();
   float wq[4];
   load_w4(post, b, wq);
-  const Span<T, BUF> os(out + t0 * 4 * D, rest * 4 * D);
+  const typename SpanOf<T, W, RAG>::type os(out + t0 * 4 * D, rest * 4 * D);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (!ok[u]) continue;
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(kThreads) void add_residual_fwd_kernel(const T* __r
       float r[W];
 #pragma unroll
       for (int e = 0; e < W; ++e) r[e] = h[n][e] + wq[n] * bv[e];
-      st<T, W, (NT & 2) != 0>(os, e4[u] + n * (uint32_t)D, r);
+      st_from<T, W, (NT & 2) != 0>(os, e4[u] + n * (uint32_t)D, r, skip[u]);
     }
   }
 }
@@ -225,7 +227,7 @@ __global__ __launch_bounds__(kThreads) void add_residual_fwd_kernel(const T* __r
 //   d_bo[s,:] = sum_n post[n] dHn[s,n,:]              (written, dtype TB)
 //   part[k]   = sum dHn[s,k,:] * bo[s,:]   k < 4      (reduced -> dH_post)
 // ---------------------------------------------------------------------------
-template <typename T, typename TB, int W, int U, int NT = 0, bool BUF = (W > 1), bool ONE = false>
+template <typename T, typename TB, int W, int U, int NT = 0, bool RAG = false, bool ONE = false>
 __global__ __launch_bounds__(kThreads) void add_residual_bwd_kernel(const T* __restrict__ dhn,
                                                                     const TB* __restrict__ bo, WRow post,
                                                                     TB* __restrict__ dbo, float* __restrict__ part,
@@ -242,23 +244,24 @@ __global__ __launch_bounds__(kThreads) void add_residual_bwd_kernel(const T* __r
     const int64_t s_lo = (int64_t)(tile * (kThreads * U)) / g.nch;
     const int64_t t0 = b * g.S + s_lo;
     const int64_t rest = g.S - s_lo;
-    const Span<T, BUF> hs(dhn + t0 * 4 * D, rest * 4 * D);
-    const Span<TB, BUF> bs(bo + t0 * D, rest * D);
-    const Span<TB, BUF> ds_(dbo + t0 * D, rest * D);
+    const typename SpanOf<T, W, RAG>::type hs(dhn + t0 * 4 * D, rest * 4 * D);
+    const typename SpanOf<TB, W, RAG>::type bs(bo + t0 * D, rest * D);
+    const typename SpanOf<TB, W, RAG>::type ds_(dbo + t0 * D, rest * D);
     float h[U][4][W];
     float bv[U][W];
-    uint32_t e1[U];
+    uint32_t e1[U], skip[U];
     bool ok[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t i = tile * (kThreads * U) + u * kThreads + threadIdx.x;
       ok[u] = i < g.items;
       const uint32_t s = ok[u] ? i / g.nch : (uint32_t)s_lo;
-      const uint32_t c = ok[u] ? i - s * g.nch : 0;
+      const RowCol<W, RAG> rc(ok[u] ? i - s * g.nch : 0, (uint32_t)D);
       const uint32_t dt = s - (uint32_t)s_lo;
-      e1[u] = dt * (uint32_t)D + c * W;
+      e1[u] = dt * (uint32_t)D + rc.col;
+      skip[u] = rc.skip;
       if (ok[u]) {
-        const uint32_t e4 = dt * 4 * (uint32_t)D + c * W;
+        const uint32_t e4 = dt * 4 * (uint32_t)D + rc.col;
 #pragma unroll
         for (int n = 0; n < 4; ++n) ld<T, W, (NT & 1) != 0>(hs, e4 + n * (uint32_t)D, h[u][n]);
         ld<TB, W, (NT & 1) != 0>(bs, e1[u], bv[u]);
@@ -268,6 +271,7 @@ __global__ __launch_bounds__(kThreads) void add_residual_bwd_kernel(const T* __r
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (!ok[u]) continue;
+      drop_skipped<W, RAG>(bv[u], skip[u]);
       float r[W];
 #pragma unroll
       for (int e = 0; e < W; ++e) {
@@ -275,7 +279,7 @@ __global__ __launch_bounds__(kThreads) void add_residual_bwd_kernel(const T* __r
 #pragma unroll
         for (int n = 0; n < 4; ++n) acc[n] += h[u][n][e] * bv[u][e];
       }
-      st<TB, W, (NT & 2) != 0>(ds_, e1[u], r);
+      st_from<TB, W, (NT & 2) != 0>(ds_, e1[u], r, skip[u]);
     }
     if constexpr (ONE) break;
   }
@@ -295,7 +299,7 @@ __global__ __launch_bounds__(kThreads) void add_residual_bwd_kernel(const T* __r
 // reads H for the last time but d_bi and dH_new again in pass C, which then
 // finds part of them in the 256 MB memory-side cache.
 // ---------------------------------------------------------------------------
-template <typename T, int W, int U, bool HAS_DHN, bool REDUCE, bool WRITE_DH, int NT = 0, bool BUF = (W > 1),
+template <typename T, int W, int U, bool HAS_DHN, bool REDUCE, bool WRITE_DH, int NT = 0, bool RAG = false,
           bool ONE = false>
 __global__ __launch_bounds__(kThreads) void mix_bwd_kernel(const T* __restrict__ dbi, const T* __restrict__ dhn,
                                                            const T* __restrict__ H, WRow pre, WRow res,
@@ -317,24 +321,25 @@ __global__ __launch_bounds__(kThreads) void mix_bwd_kernel(const T* __restrict__
     const int64_t s_lo = (int64_t)(tile * (kThreads * U)) / g.nch;
     const int64_t t0 = b * g.S + s_lo;
     const int64_t rest = g.S - s_lo;
-    const Span<T, BUF> dbs(dbi + t0 * D, rest * D);
-    const Span<T, BUF> dns(dhn + t0 * 4 * D, rest * 4 * D);
-    const Span<T, BUF> hs(H + t0 * 4 * D, rest * 4 * D);
+    const typename SpanOf<T, W, RAG>::type dbs(dbi + t0 * D, rest * D);
+    const typename SpanOf<T, W, RAG>::type dns(dhn + t0 * 4 * D, rest * 4 * D);
+    const typename SpanOf<T, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
     float db[U][W];
     float dn[U][4][W];
     float h[U][4][W];
-    uint32_t e4[U];  // element offset of (s, n=0, c*W) in the [.,4,D] spans
+    uint32_t e4[U], skip[U];  // element offset of (s, n=0, column) in the [.,4,D] spans
     bool ok[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t i = tile * (kThreads * U) + u * kThreads + threadIdx.x;
       ok[u] = i < g.items;
       const uint32_t s = ok[u] ? i / g.nch : (uint32_t)s_lo;
-      const uint32_t c = ok[u] ? i - s * g.nch : 0;
+      const RowCol<W, RAG> rc(ok[u] ? i - s * g.nch : 0, (uint32_t)D);
       const uint32_t dt = s - (uint32_t)s_lo;
-      e4[u] = dt * 4 * (uint32_t)D + c * W;
+      e4[u] = dt * 4 * (uint32_t)D + rc.col;
+      skip[u] = rc.skip;
       if (ok[u]) {
-        ld<T, W, (NT & 1) != 0>(dbs, dt * (uint32_t)D + c * W, db[u]);
+        ld<T, W, (NT & 1) != 0>(dbs, dt * (uint32_t)D + rc.col, db[u]);
         if constexpr (HAS_DHN) {
 #pragma unroll
           for (int n = 0; n < 4; ++n) ld<T, W, (NT & 1) != 0>(dns, e4[u] + n * (uint32_t)D, dn[u][n]);
@@ -350,11 +355,13 @@ __global__ __launch_bounds__(kThreads) void mix_bwd_kernel(const T* __restrict__
       load_w4(pre, b, wp);
       if constexpr (HAS_DHN) load_w16(res, b, wr);
     }
-    const Span<T, BUF> dHs(dH + t0 * 4 * D, rest * 4 * D);
+    const typename SpanOf<T, W, RAG>::type dHs(dH + t0 * 4 * D, rest * 4 * D);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (!ok[u]) continue;
       if constexpr (REDUCE) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) drop_skipped<W, RAG>(h[u][n], skip[u]);
 #pragma unroll
         for (int e = 0; e < W; ++e) {
 #pragma unroll
@@ -382,7 +389,7 @@ __global__ __launch_bounds__(kThreads) void mix_bwd_kernel(const T* __restrict__
             }
             r[e] = v;
           }
-          st<T, W, (NT & 2) != 0>(dHs, e4[u] + m * (uint32_t)D, r);
+          st_from<T, W, (NT & 2) != 0>(dHs, e4[u] + m * (uint32_t)D, r, skip[u]);
         }
       }
     }
@@ -408,32 +415,36 @@ __global__ __launch_bounds__(kThreads) void mix_bwd_kernel(const T* __restrict__
 // left one block in four half idle: pass C at config 4 ran at 76% of 8 TB/s).
 // Grid: x = ceil(groups * nch / 256), y = batch within the launch.
 // ---------------------------------------------------------------------------
-template <typename T, int W, int TT, bool HAS_DHN, int NT = 0, bool BUF = (W > 1)>
+template <typename T, int W, int TT, bool HAS_DHN, int NT = 0, bool RAG = false>
 __global__ __launch_bounds__(kThreads) void dh_kernel(const T* __restrict__ dbi, const T* __restrict__ dhn,
                                                       const float* __restrict__ gx, float inv_S, WRow pre,
                                                       WRow res, T* __restrict__ dH, int64_t S, int64_t D,
                                                       uint32_t groups, int64_t b0) {
   const int64_t b = b0 + blockIdx.y;
-  const uint32_t nch = (uint32_t)(D / W);
+  const uint32_t nch = (uint32_t)((D + W - 1) / W);
   const uint32_t i = blockIdx.x * (uint32_t)kThreads + threadIdx.x;
   const uint32_t grp = i / nch;
   if (grp >= groups) return;
-  const int64_t cw = (int64_t)(i - grp * nch) * W;
+  const RowCol<W, RAG> rc(i - grp * nch, (uint32_t)D);
+  const uint32_t cw = rc.col;
   // Spans start at the workgroup's first token; dt0 is this lane's token offset in them.
   const int64_t s_lo = (int64_t)((blockIdx.x * (uint32_t)kThreads) / nch) * TT;
   const int64_t s0 = (int64_t)grp * TT;
   const uint32_t dt0 = (uint32_t)(s0 - s_lo);
   const int64_t t0 = b * S + s_lo;
   const int64_t rest = S - s_lo;
-  const Span<T, BUF> dbs(dbi + t0 * D, rest * D);
-  const Span<T, BUF> dns(dhn + t0 * 4 * D, rest * 4 * D);
-  const Span<T, BUF> dHs(dH + t0 * 4 * D, rest * 4 * D);
+  const typename SpanOf<T, W, RAG>::type dbs(dbi + t0 * D, rest * D);
+  const typename SpanOf<T, W, RAG>::type dns(dhn + t0 * 4 * D, rest * 4 * D);
+  const typename SpanOf<T, W, RAG>::type dHs(dH + t0 * 4 * D, rest * 4 * D);
   float wp[4], wr[16];
   load_w4(pre, b, wp);
   if constexpr (HAS_DHN) load_w16(res, b, wr);
   float gv[4][W];
 #pragma unroll
-  for (int m = 0; m < 4; ++m) ld<float, W>(gx + b * 4 * D + m * D + cw, gv[m]);
+  for (int m = 0; m < 4; ++m) {
+    if constexpr (RAG) ld<float, W, false>(RagSpan<float>(gx + b * 4 * D, 0), (uint32_t)(m * D) + cw, gv[m]);
+    else ld<float, W>(gx + b * 4 * D + m * D + cw, gv[m]);
+  }
 #pragma unroll
   for (int t = 0; t < TT; ++t) {
     const int64_t s = s0 + t;
@@ -466,7 +477,7 @@ __global__ __launch_bounds__(kThreads) void dh_kernel(const T* __restrict__ dbi,
         }
         r[e] = __builtin_fmaf(gv[m][e], inv_S, v);
       }
-      st<T, W, (NT & 2) != 0>(dHs, e4 + m * (uint32_t)D, r);
+      st_from<T, W, (NT & 2) != 0>(dHs, e4 + m * (uint32_t)D, r, rc.skip);
     }
   }
 }
@@ -480,7 +491,7 @@ __global__ __launch_bounds__(kThreads) void dh_kernel(const T* __restrict__ dbi,
 // each other's backward.  An item is W consecutive elements of one token row;
 // W is the wider 16-byte vector of the two dtypes (or 1 on the ragged path).
 // ---------------------------------------------------------------------------
-template <typename TX, typename TH, int W, int NT = 0, bool BUF = (W > 1)>
+template <typename TX, typename TH, int W, int NT = 0, bool RAG = false>
 __global__ __launch_bounds__(kThreads) void expand_kernel(const TX* __restrict__ x, TH* __restrict__ H,
                                                           float scale, Geom g) {
   const int64_t b = g.b0 + blockIdx.y;
@@ -492,20 +503,22 @@ __global__ __launch_bounds__(kThreads) void expand_kernel(const TX* __restrict__
     const uint32_t i = tile * kThreads + threadIdx.x;
     if (i >= g.items) continue;
     const uint32_t s = i / g.nch;
-    const uint32_t cw = (i - s * g.nch) * W;
+    const RowCol<W, RAG> rc(i - s * g.nch, (uint32_t)D);
+    const uint32_t cw = rc.col;
     const uint32_t dt = s - (uint32_t)s_lo;
-    const Span<TX, BUF> xs(x + t0 * D, rest * D);
-    const Span<TH, BUF> hs(H + t0 * 4 * D, rest * 4 * D);
+    const typename SpanOf<TX, W, RAG>::type xs(x + t0 * D, rest * D);
+    const typename SpanOf<TH, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
     float v[W];
     ld<TX, W, (NT & 1) != 0>(xs, dt * (uint32_t)D + cw, v);
 #pragma unroll
     for (int e = 0; e < W; ++e) v[e] *= scale;
 #pragma unroll
-    for (int n = 0; n < 4; ++n) st<TH, W, (NT & 2) != 0>(hs, dt * 4 * (uint32_t)D + cw + n * (uint32_t)D, v);
+    for (int n = 0; n < 4; ++n)
+      st_from<TH, W, (NT & 2) != 0>(hs, dt * 4 * (uint32_t)D + cw + n * (uint32_t)D, v, rc.skip);
   }
 }
 
-template <typename TH, typename TY, int W, int NT = 0, bool BUF = (W > 1)>
+template <typename TH, typename TY, int W, int NT = 0, bool RAG = false>
 __global__ __launch_bounds__(kThreads) void collapse_kernel(const TH* __restrict__ H, TY* __restrict__ y,
                                                             float scale, Geom g) {
   const int64_t b = g.b0 + blockIdx.y;
@@ -517,9 +530,10 @@ __global__ __launch_bounds__(kThreads) void collapse_kernel(const TH* __restrict
     const uint32_t i = tile * kThreads + threadIdx.x;
     const bool ok = i < g.items;
     const uint32_t s = ok ? i / g.nch : (uint32_t)s_lo;
-    const uint32_t cw = ok ? (i - s * g.nch) * W : 0;
+    const RowCol<W, RAG> rc(ok ? i - s * g.nch : 0, (uint32_t)D);
+    const uint32_t cw = rc.col;
     const uint32_t dt = s - (uint32_t)s_lo;
-    const Span<TH, BUF> hs(H + t0 * 4 * D, rest * 4 * D);
+    const typename SpanOf<TH, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
     Frag<TH, W> hf[4];
     if (ok) {
 #pragma unroll
@@ -532,8 +546,8 @@ __global__ __launch_bounds__(kThreads) void collapse_kernel(const TH* __restrict
     for (int n = 0; n < 4; ++n) hf[n].unpack(h[n]);
 #pragma unroll
     for (int e = 0; e < W; ++e) r[e] = (((h[0][e] + h[1][e]) + h[2][e]) + h[3][e]) * scale;
-    const Span<TY, BUF> ys(y + t0 * D, rest * D);
-    st<TY, W, (NT & 2) != 0>(ys, dt * (uint32_t)D + cw, r);
+    const typename SpanOf<TY, W, RAG>::type ys(y + t0 * D, rest * D);
+    st_from<TY, W, (NT & 2) != 0>(ys, dt * (uint32_t)D + cw, r, rc.skip);
   }
 }
 
@@ -637,6 +651,29 @@ inline bool vec_ok(int64_t D, int W, std::initializer_list<const void*> ptrs) {
   return true;
 }
 
+// Otherwise the ragged path (RagSpan, RowCol) still moves 16-byte vectors, at the elements' own
+// alignment; it needs rows of at least one vector, and offsets within a tile that fit 32 bits.
+// Training steps as graphs, single elements -> ragged vectors: B=3, S=1023, D=1500 bf16 185.0 ->
+// 111.4 us, D=1501 197.6 -> 112.5, B=4, S=4096, D=2050 1145.7 -> 528.7 (D = 2048: 460.6), B=4,
+// S=2048, D=1001 fp16 313.8 -> 159.1, fp32 366.8 -> 261.3.  Of little work single elements make
+// more workgroups, without the last lane's element stores: at 160 k elements (B S D) they win by
+// 3-10 us of 40-60 at any D, at 320 k it goes either way (D = 1001 51.3 -> 49.4, D = 37 54.4 ->
+// 56.2), at 640 k ragged vectors win (59.8 -> 51.4, 64.2 -> 62.9).
+constexpr int64_t kRagMinElems = (int64_t)3 << 17;
+
+inline bool rag_ok(int64_t elems, int64_t row, int W) {
+  return elems >= kRagMinElems && row >= W && span_ok(16384 + 8 * row, 4);
+}
+
+// How a streaming kernel walks B * S rows of D, and the launch of fn(std::integral_constant<int, W>,
+// std::bool_constant<RAG>) for it: whole vectors, ragged vectors, or single elements.
+template <int WV, class F>
+inline int with_width(int64_t B, int64_t S, int64_t D, std::initializer_list<const void*> ptrs, F&& fn) {
+  if (vec_ok(D, WV, ptrs)) return fn(std::integral_constant<int, WV>{}, std::false_type{});
+  if (rag_ok(B * S * D, D, WV)) return fn(std::integral_constant<int, WV>{}, std::true_type{});
+  return fn(std::integral_constant<int, 1>{}, std::false_type{});
+}
+
 // Workgroups per batch for a reduction kernel: about kRedBlocks in total
 // (8 per CU on a 256-CU MI355X), never more than there are tiles.  The cap is
 // a constant so workspace sizes do not depend on the device.
@@ -661,7 +698,7 @@ inline size_t partial_bytes(int64_t B, int nv) {
 // lane, one item per lane), because the path is chosen per call from the
 // pointers' alignment.
 inline size_t tile_partial_bytes(int64_t B, int64_t S, int64_t D, int nv) {
-  const int64_t tiles = (S * D / 4 + kThreads - 1) / kThreads;
+  const int64_t tiles = (S * ((D + 3) / 4) + kThreads - 1) / kThreads;
   const size_t vec = (size_t)(B > 0 ? B : 1) * (size_t)(tiles > 0 ? tiles : 1) * nv * sizeof(float);
   const size_t rag = partial_bytes(B, nv);
   return vec > rag ? vec : rag;

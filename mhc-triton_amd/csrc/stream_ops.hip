@@ -7,24 +7,24 @@ namespace mhc {
 
 constexpr int kU = 1;  // items per lane per tile
 
-template <typename T, int W>
+template <typename T, int W, bool RAG>
 static int stream_mix_fwd(const T* H, const float* pre, const float* res, T* bi, T* out, int64_t B, int64_t S,
                           int64_t D, hipStream_t st) {
   return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
     const Geom g = make_geom<W, kU>(S, D, b0);
     if (g.ntiles == 0) return (int)MHC_OK;
-    mix_fwd_kernel<T, T, W, kU, true, true, false, kNt><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(2), st>>>(
+    mix_fwd_kernel<T, T, W, kU, true, true, false, kNt, RAG><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(2), st>>>(
         H, (const T*)nullptr, WRow{pre, 4}, WRow{res, 16}, WRow{nullptr, 0}, bi, out, g);
     return hip_status(hipGetLastError(), "stream_mix_forward launch");
   });
 }
 
-template <typename T, int W>
+template <typename T, int W, bool RAG>
 static int stream_mix_bwd(const T* dbi, const T* dhr, const T* H, const float* pre, const float* res, T* dH,
                           float* dpre, float* dres, int64_t B, int64_t S, int64_t D, float* part,
                           hipStream_t st) {
-  // Vector path: one workgroup per tile, weights fetched behind its loads, up
-  // to 6 per CU, a partial per tile.  Ragged path: workgroups stride over the
+  // Vectors: one workgroup per tile, weights fetched behind its loads, up to 6
+  // per CU, a partial per tile.  Single elements: workgroups stride over the
   // tiles at 3 per CU.
   const Geom g0 = make_geom<W, kU>(S, D, 0);
   const uint32_t nblk = W > 1 ? g0.ntiles : reduce_blocks(g0.ntiles, B);
@@ -32,7 +32,7 @@ static int stream_mix_bwd(const T* dbi, const T* dhr, const T* H, const float* p
   int rc = nblk == 0 ? (int)MHC_OK : for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
     const Geom g = make_geom<W, kU>(S, D, b0);
     if constexpr (W > 1)
-      mix_bwd_kernel<T, W, kU, true, true, true, kNt, true, true><<<dim3(nblk, nb), kThreads, occupancy_lds(6), st>>>(
+      mix_bwd_kernel<T, W, kU, true, true, true, kNt, RAG, true><<<dim3(nblk, nb), kThreads, occupancy_lds(6), st>>>(
           dbi, dhr, H, WRow{pre, 4}, WRow{res, 16}, dH, part, g);
     else
       mix_bwd_kernel<T, W, kU, true, true, true, kNt><<<dim3(nblk, nb), kThreads, occupancy_lds(3), st>>>(
@@ -44,24 +44,24 @@ static int stream_mix_bwd(const T* dbi, const T* dhr, const T* H, const float* p
                     "stream_mix_backward reduce launch");
 }
 
-template <typename TH, typename TB, int W>
+template <typename TH, typename TB, int W, bool RAG>
 static int add_res_fwd(const TH* hr, const TB* bo, const float* post, TH* out, int64_t B, int64_t S, int64_t D,
                        hipStream_t st) {
   return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
     const Geom g = make_geom<W, kU>(S, D, b0);
     if (g.ntiles == 0) return (int)MHC_OK;
-    add_residual_fwd_kernel<TH, TB, W, kU, kNt><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(4), st>>>(
+    add_residual_fwd_kernel<TH, TB, W, kU, kNt, RAG><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(4), st>>>(
         hr, bo, WRow{post, 4}, out, g);
     return hip_status(hipGetLastError(), "add_residual_forward launch");
   });
 }
 
-template <typename TH, typename TB, int W>
+template <typename TH, typename TB, int W, bool RAG>
 static int add_res_bwd(const TH* dhn, const TB* bo, WRow post, TB* dbo, float* dpost, int64_t B, int64_t S,
                        int64_t D, float* part, hipStream_t st) {
-  // Vector path: one workgroup per tile at 4 per CU (the closure backward at
+  // Vectors: one workgroup per tile at 4 per CU (the closure backward at
   // config-3 size: 134 -> 128 us against 512 looping workgroups per batch at
-  // 2 per CU).  Ragged path: a capped count of looping workgroups.
+  // 2 per CU).  Single elements: a capped count of looping workgroups.
   const Geom g0 = make_geom<W, kU>(S, D, 0);
   // At least one workgroup: with no tiles it writes zero partials, so dH_post comes out zero.
   uint32_t nblk = W > 1 ? g0.ntiles : reduce_blocks(g0.ntiles, B);
@@ -69,7 +69,7 @@ static int add_res_bwd(const TH* dhn, const TB* bo, WRow post, TB* dbo, float* d
   int rc = for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
     const Geom g = make_geom<W, kU>(S, D, b0);
     if constexpr (W > 1)
-      add_residual_bwd_kernel<TH, TB, W, kU, kNt, true, true><<<dim3(nblk, nb), kThreads, occupancy_lds(4), st>>>(
+      add_residual_bwd_kernel<TH, TB, W, kU, kNt, RAG, true><<<dim3(nblk, nb), kThreads, occupancy_lds(4), st>>>(
           dhn, bo, post, dbo, part, g);
     else
       add_residual_bwd_kernel<TH, TB, W, kU, kNt><<<dim3(nblk, nb), kThreads, occupancy_lds(2), st>>>(
@@ -103,10 +103,10 @@ int check_workspace(const char* who, const void* ws, size_t have, size_t need) {
 template <typename TH, typename TB>
 int add_residual_backward_t(const void* dhn, const void* bo, WRow post, void* dbo, float* dpost, int64_t B,
                             int64_t S, int64_t D, float* part, hipStream_t st) {
-  constexpr int WV = wide_w<TH, TB>();
-  if (vec_ok(D, WV, {dhn, bo, dbo}))
-    return add_res_bwd<TH, TB, WV>((const TH*)dhn, (const TB*)bo, post, (TB*)dbo, dpost, B, S, D, part, st);
-  return add_res_bwd<TH, TB, 1>((const TH*)dhn, (const TB*)bo, post, (TB*)dbo, dpost, B, S, D, part, st);
+  return with_width<wide_w<TH, TB>()>(B, S, D, {dhn, bo, dbo}, [&](auto w, auto rag) {
+    return add_res_bwd<TH, TB, decltype(w)::value, decltype(rag)::value>((const TH*)dhn, (const TB*)bo, post, (TB*)dbo,
+                                                                         dpost, B, S, D, part, st);
+  });
 }
 
 int add_residual_backward_any(const void* dhn, int dtype_h, const void* bo, int dtype_bo, WRow post, void* dbo,
@@ -131,10 +131,10 @@ extern "C" int mhc_stream_mix_forward(const void* H, const float* H_pre, const f
   }
   hipStream_t st = (hipStream_t)stream;
   return MHC_DISPATCH_DTYPE(dtype, [&] {
-    constexpr int WV = Vec<T>::N;
-    if (vec_ok(D, WV, {H, branch_input, H_residual}))
-      return stream_mix_fwd<T, WV>((const T*)H, H_pre, H_res, (T*)branch_input, (T*)H_residual, B, S, D, st);
-    return stream_mix_fwd<T, 1>((const T*)H, H_pre, H_res, (T*)branch_input, (T*)H_residual, B, S, D, st);
+    return with_width<Vec<T>::N>(B, S, D, {H, branch_input, H_residual}, [&](auto w, auto rag) {
+      return stream_mix_fwd<T, decltype(w)::value, decltype(rag)::value>((const T*)H, H_pre, H_res, (T*)branch_input,
+                                                                         (T*)H_residual, B, S, D, st);
+    });
   });
 }
 
@@ -167,12 +167,11 @@ extern "C" int mhc_stream_mix_backward(const void* d_branch_input, const void* d
   hipStream_t st = (hipStream_t)stream;
   float* part = (float*)workspace;
   return MHC_DISPATCH_DTYPE(dtype, [&] {
-    constexpr int WV = Vec<T>::N;
-    if (vec_ok(D, WV, {d_branch_input, dH_residual, H, dH}))
-      return stream_mix_bwd<T, WV>((const T*)d_branch_input, (const T*)dH_residual, (const T*)H, H_pre, H_res,
-                                   (T*)dH, dH_pre, dH_res, B, S, D, part, st);
-    return stream_mix_bwd<T, 1>((const T*)d_branch_input, (const T*)dH_residual, (const T*)H, H_pre, H_res,
-                                (T*)dH, dH_pre, dH_res, B, S, D, part, st);
+    return with_width<Vec<T>::N>(B, S, D, {d_branch_input, dH_residual, H, dH}, [&](auto w, auto rag) {
+      return stream_mix_bwd<T, decltype(w)::value, decltype(rag)::value>(
+          (const T*)d_branch_input, (const T*)dH_residual, (const T*)H, H_pre, H_res, (T*)dH, dH_pre, dH_res, B, S, D,
+          part, st);
+    });
   });
 }
 
@@ -187,12 +186,10 @@ extern "C" int mhc_add_residual_forward(const void* H_residual, int dtype_h, con
   }
   hipStream_t st = (hipStream_t)stream;
   return MHC_DISPATCH_DTYPE2(dtype_h, dtype_bo, [&] {
-    constexpr int WV = wide_w<TH, TB>();
-    if (vec_ok(D, WV, {H_residual, branch_output, H_new}))
-      return add_res_fwd<TH, TB, WV>((const TH*)H_residual, (const TB*)branch_output, H_post, (TH*)H_new, B, S, D,
-                                     st);
-    return add_res_fwd<TH, TB, 1>((const TH*)H_residual, (const TB*)branch_output, H_post, (TH*)H_new, B, S, D,
-                                  st);
+    return with_width<wide_w<TH, TB>()>(B, S, D, {H_residual, branch_output, H_new}, [&](auto w, auto rag) {
+      return add_res_fwd<TH, TB, decltype(w)::value, decltype(rag)::value>(
+          (const TH*)H_residual, (const TB*)branch_output, H_post, (TH*)H_new, B, S, D, st);
+    });
   });
 }
 
@@ -227,21 +224,21 @@ extern "C" int mhc_add_residual_backward(const void* dH_new, int dtype_h, const 
 
 namespace mhc {
 
-template <typename TX, typename TH, int W>
+template <typename TX, typename TH, int W, bool RAG>
 static int expand_launch(const TX* x, TH* H, float scale, int64_t B, int64_t S, int64_t D, hipStream_t st) {
   return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
     const Geom g = make_geom<W, 1>(S, D, b0);
     // nt stores only: with nt on its one load this write-dominated kernel runs 10% slower.
-    expand_kernel<TX, TH, W, 2><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(2), st>>>(x, H, scale, g);
+    expand_kernel<TX, TH, W, 2, RAG><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(2), st>>>(x, H, scale, g);
     return hip_status(hipGetLastError(), "stream_expand launch");
   });
 }
 
-template <typename TH, typename TY, int W>
+template <typename TH, typename TY, int W, bool RAG>
 static int collapse_launch(const TH* H, TY* y, float scale, int64_t B, int64_t S, int64_t D, hipStream_t st) {
   return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
     const Geom g = make_geom<W, 1>(S, D, b0);
-    collapse_kernel<TH, TY, W, kNt><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(4), st>>>(H, y, scale, g);
+    collapse_kernel<TH, TY, W, kNt, RAG><<<dim3(g.ntiles, nb), kThreads, occupancy_lds(4), st>>>(H, y, scale, g);
     return hip_status(hipGetLastError(), "stream_collapse launch");
   });
 }
@@ -259,9 +256,9 @@ extern "C" int mhc_stream_expand(const void* x, int dtype_x, void* H, int dtype_
   hipStream_t st = (hipStream_t)stream;
   // TH: the stream tensor's dtype, TB: x's dtype.
   return MHC_DISPATCH_DTYPE2(dtype_h, dtype_x, [&] {
-    constexpr int WV = wide_w<TH, TB>();
-    if (vec_ok(D, WV, {x, H})) return expand_launch<TB, TH, WV>((const TB*)x, (TH*)H, scale, B, S, D, st);
-    return expand_launch<TB, TH, 1>((const TB*)x, (TH*)H, scale, B, S, D, st);
+    return with_width<wide_w<TH, TB>()>(B, S, D, {x, H}, [&](auto w, auto rag) {
+      return expand_launch<TB, TH, decltype(w)::value, decltype(rag)::value>((const TB*)x, (TH*)H, scale, B, S, D, st);
+    });
   });
 }
 
@@ -276,8 +273,9 @@ extern "C" int mhc_stream_collapse(const void* H, int dtype_h, void* y, int dtyp
   hipStream_t st = (hipStream_t)stream;
   // TH: the stream tensor's dtype, TB: y's dtype.
   return MHC_DISPATCH_DTYPE2(dtype_h, dtype_y, [&] {
-    constexpr int WV = wide_w<TH, TB>();
-    if (vec_ok(D, WV, {H, y})) return collapse_launch<TH, TB, WV>((const TH*)H, (TB*)y, scale, B, S, D, st);
-    return collapse_launch<TH, TB, 1>((const TH*)H, (TB*)y, scale, B, S, D, st);
+    return with_width<wide_w<TH, TB>()>(B, S, D, {H, y}, [&](auto w, auto rag) {
+      return collapse_launch<TH, TB, decltype(w)::value, decltype(rag)::value>((const TH*)H, (TB*)y, scale, B, S, D,
+                                                                               st);
+    });
   });
 }

@@ -43,3 +43,94 @@ def test_forward_reads_of_a_small_and_a_large_H_agree():
         bi3, add3 = hc(H[:3])
         assert torch.equal(bi3, bi4[:3])
         assert torch.equal(add3(bo[:3]), add4(bo)[:3])
+
+
+def off_by_one(t):
+    """A contiguous copy of t that starts one element past a 16-byte boundary."""
+    flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    out = flat[1:].view(t.shape)
+    out.copy_(t)
+    return out
+
+
+# Rows that are not whole 16-byte vectors, with enough elements (B S D >= 3 * 2^17) for the ragged
+# vectors: one vector and one element, a vector less one past it, an even and an odd long row, rows
+# one vector long; the last three start off a 16-byte boundary (whole vectors otherwise).
+RAGGED = [(2, 21850, 9, torch.bfloat16, False), (3, 8750, 15, torch.float16, False),
+          (2, 197, 1001, torch.bfloat16, False), (1, 265, 1500, torch.float16, False),
+          (1, 78700, 5, torch.float32, False), (3, 131, 1003, torch.float32, False),
+          (400, 1, 1001, torch.bfloat16, False), (70, 6, 1001, torch.float16, False),
+          (1, 49200, 8, torch.bfloat16, True), (2, 200, 1024, torch.bfloat16, True),
+          (1, 400, 1000, torch.float32, True)]
+
+
+@pytest.mark.parametrize("B,S,D,dtype,shifted", RAGGED)
+@pytest.mark.parametrize("dynamic", [True, False])
+def test_layer_on_ragged_rows(B, S, D, dtype, shifted, dynamic):
+    assert B * S * D >= 3 << 17
+    hc, H, bo, dHn, dbi = make_case(B, S, D, dtype, dynamic=dynamic, phi_std=0.02, res_std=1.0)
+    copy = off_by_one if shifted else torch.clone
+    check_layer(hc, H, bo, copy(dHn), copy(dbi), *FWD[dtype], 1e-4, copy=copy)
+
+
+@pytest.mark.parametrize("B,S,D,dtype,shifted", RAGGED)
+def test_ops_on_ragged_rows_match_whole_vectors(B, S, D, dtype, shifted):
+    """The four stream ops and their backwards give the same bits on ragged rows as on the same rows
+    padded with zeros to whole vectors, and the weight gradients the same sums to fp32 rounding
+    (both add at most B S D products in fp32 over fixed trees: a few 2^-24 of their largest
+    partial sums; 1e-4 of the largest gradient leaves room for the trees' different shapes)."""
+    import mhc
+    from mhc import streams
+
+    g = torch.Generator(device=DEV).manual_seed(11)
+    P = (D + 7) // 8 * 8 + (8 if shifted else 0)
+
+    def rows(*shape):
+        return torch.randn(shape, generator=g, device=DEV).to(dtype)
+
+    x, bo, d_bi, d_y = (rows(B, S, D) for _ in range(4))
+    pre, post = torch.rand((B, 4), generator=g, device=DEV), torch.rand((B, 4), generator=g, device=DEV)
+    res = torch.rand((B, 4, 4), generator=g, device=DEV)
+
+    def run(make):
+        a, b = (make(t).requires_grad_(True) for t in (x, bo))
+        w = [t.clone().requires_grad_(True) for t in (pre, post, res)]
+        H = streams.expand_streams(a)
+        bi, hr = mhc.fused_stream_mix(make(H[..., :D]) if shifted and make is off_by_one else H, w[0], w[2])
+        Hn = mhc.fused_add_residual(hr, b, w[1])
+        y = streams.collapse_streams(Hn)
+        torch.autograd.backward([bi, y], [make(d_bi), make(d_y)])
+        return [t[..., :D] for t in (bi, Hn, y, a.grad, b.grad)], [t.grad for t in w]
+
+    pad = lambda t: torch.nn.functional.pad(t, (0, P - D)).contiguous()  # noqa: E731
+    got, got_w = run(off_by_one if shifted else torch.clone)
+    want, want_w = run(pad)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert torch.equal(a, b), i
+    for i, (a, b) in enumerate(zip(got_w, want_w)):
+        assert float((a - b).abs().max()) <= 1e-4 * float(b.abs().max()), i
+
+
+@pytest.mark.parametrize("B,S,D,dtype", [(5, 7, 11235, torch.bfloat16), (3, 130, 1009, torch.float16),
+                                         (2, 9, 21846, torch.float32)])
+@pytest.mark.parametrize("shifted", [False, True])
+def test_mean_pool_on_ragged_rows(B, S, D, dtype, shifted):
+    """fp32 sums of S values each: 2 S 2^-24 of the mean of |H|, at most 2^-14 here."""
+    from mhc._kernels import mean_pool
+
+    g = torch.Generator(device=DEV).manual_seed(2)
+    H = torch.randn((B, S, 4, D), generator=g, device=DEV).to(dtype)
+    x = mean_pool(off_by_one(H) if shifted else H)
+    want = H.double().mean(dim=1).reshape(B, 4 * D)
+    assert float((x.double() - want).abs().max()) <= 2.0 ** -14
+
+
+def test_mixed_types_on_ragged_rows():
+    """H in fp32 with a bf16 branch output (8 elements a lane): the bits of the single-element path,
+    which the same rows take in pieces too small for the ragged one."""
+    hc, H, bo, _, _ = make_case(2, 200, 1001, torch.float32, dynamic=False, res_std=1.0)
+    bo = bo.to(torch.bfloat16)
+    with torch.no_grad():
+        whole = hc(H)[1](bo)
+        for s in range(0, 200, 50):
+            assert torch.equal(hc(H[:, s:s + 50].contiguous())[1](bo[:, s:s + 50].contiguous()), whole[:, s:s + 50])
