@@ -629,12 +629,12 @@ __global__ __launch_bounds__(kThreads) void dynw_bwd_rows_kernel(const float* __
     if (RPW == 1) {
       if (threadIdx.x < 20) {
         const int v = threadIdx.x;
-        float t = 0.f;
+        double t = 0.0;  // the largest sums of the reduction, without rounding of their own
 #pragma unroll
         for (int w = 0; w < 4; ++w)
 #pragma unroll
           for (int h = 0; h < 4; ++h) t += quarter[w][h][v];
-        red[0][v] = t;
+        red[0][v] = (float)t;
       }
     } else if (lane < 20) {
       red[wave][lane] = ((quarter[wave][0][lane] + quarter[wave][1][lane]) + quarter[wave][2][lane]) +

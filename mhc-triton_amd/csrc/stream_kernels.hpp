@@ -582,13 +582,15 @@ __global__ __launch_bounds__(kRedThreads) void reduce_split_kernel(const float* 
   }
   __syncthreads();
   if (threadIdx.x < 4) {
+    // 64 sums in a row, the largest values of the whole reduction: in fp64, so that they add no
+    // rounding of their own (in fp32 they were most of the error of dH_post, dH_pre and dH_res)
     const int c = threadIdx.x;
-    float t = 0.f;
+    double t = 0.0;
 #pragma unroll 8
     for (int r = 0; r < kRows; ++r) t += lds[r * 4 + c];
     const int i = 4 * q + c;
-    if (i < SPLIT) out0[b * SPLIT + i] = t;
-    else out1[b * (NV - SPLIT) + (i - SPLIT)] = t;
+    if (i < SPLIT) out0[b * SPLIT + i] = (float)t;
+    else out1[b * (NV - SPLIT) + (i - SPLIT)] = (float)t;
   }
 }
 
