@@ -349,8 +349,7 @@ extern "C" int mhc_dynamic_weights_backward(const void* x, int dtype_x, const fl
 namespace mhc {
 
 constexpr int kPoolUN = 4;  // rows in flight per lane in colsum_kernel
-// Sequences up to this length take colsum_direct_kernel (one launch, the same
-// bits): at such lengths the pass is a few microseconds of latency, and the
+// Sequences up to this length take colsum_direct_kernel (one launch): at such lengths the pass is a few microseconds of latency, and the
 // second launch and the column-partial round trip are most of it.
 constexpr int64_t kPoolDirectRows = 8;
 constexpr int64_t kPoolPlainBytes = (int64_t)64 << 20;  // H up to here is read without the nt policy
@@ -371,7 +370,8 @@ static int launch_meanpool(const T* H, float* x, const float* phi, float* projpa
         !PROJ && W > 1 && (RAG || aligned16(x)) && (S <= kPoolDirectRows || (p.nS == 1 && S <= 64));
     if (direct_vec || S <= kPoolDirectRows) {
       if (direct_vec)
-        colsum_direct_vec_kernel<T, W, RAG><<<dim3((unsigned)p.ncc, (unsigned)nb), kThreads, 0, st>>>(
+        colsum_direct_vec_kernel<T, W, RAG><<<dim3((unsigned)((K + kThreads * W - 1) / (kThreads * W)), (unsigned)nb),
+                                              kThreads, 0, st>>>(
             H, x, S, K, p.SC, inv_S, b0);
       else
         colsum_direct_kernel<T, PROJ><<<dim3((unsigned)p.nrc, (unsigned)nb), kThreads, 0, st>>>(
@@ -379,17 +379,17 @@ static int launch_meanpool(const T* H, float* x, const float* phi, float* projpa
       if (int rc = hip_status(hipGetLastError(), "mean_pool direct launch")) return rc;
       continue;
     }
-    // The first half of each S chunk with nt loads, the second half plain: in
+    // The first half of each wave's rows with nt loads, the second half plain: in
     // the layer, branch_input reads H next and finds the chunk tails in the
     // memory-side cache (colsum + branch_input: -4 us at config-3 size, -6 us
     // at config 4, against all plain).  An H of up to 64 MB stays there whole, and all plain is
     // 1-2 us faster at 33 MB (the two passes 28.4 -> 27.3 us) and equal at 67 MB.
     const bool all_plain = B * S * K * (int64_t)sizeof(T) <= kPoolPlainBytes;
     colsum_kernel<T, W, kPoolUN, RAG><<<dim3((unsigned)p.ncc, (unsigned)p.nS, (unsigned)nb), kThreads, 0, st>>>(
-        H, colpart, S, K, p.SC, p.nS, all_plain ? 0 : p.SC / 2, b0);
+        H, colpart, S, K, p.SC, p.nS, all_plain ? 0 : p.SC / kPoolRG / 2, b0);
     if (int rc = hip_status(hipGetLastError(), "mean_pool column-sum launch")) return rc;
-    colsum_reduce_kernel<PROJ><<<dim3((unsigned)p.nrc, (unsigned)nb), kThreads, 0, st>>>(
-        colpart, x, phi, projpart, K, p.nS, inv_S, b0, phi_vec);
+    colsum_reduce_kernel<PROJ><<<dim3((unsigned)p.nrc, (unsigned)nb), kThreads * kRedGroups, 0, st>>>(
+        colpart, x, phi, projpart, K, p.nS, inv_S, b0);
     if (int rc = hip_status(hipGetLastError(), "mean_pool reduce launch")) return rc;
   }
   return MHC_OK;

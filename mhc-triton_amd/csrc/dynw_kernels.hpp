@@ -1196,18 +1196,26 @@ __global__ __launch_bounds__(kThreads) void dynw_gphi_reduce_kernel(const float*
 // flattened [S, K = 4D] view (c = n*D + d), in two launches.
 //
 // colsum_kernel: grid (column chunks, S chunks, batch).  A workgroup owns
-//   256*W columns (one 16-byte vector per lane: the workgroup reads 4 KiB of a
-//   row contiguously) and SC consecutive rows, which it walks with UN rows in
-//   flight per lane; each lane sums its own W columns, so no cross-lane step
-//   is needed, and the fp32 sums of the chunk go to colpart[b][sc][c].
+//   64*W columns (one 16-byte vector per lane: a wave reads 1 KiB of a row
+//   contiguously) and SC consecutive rows, a quarter of them per wave, which
+//   walks its quarter with UN rows in flight per lane; the four waves' sums
+//   meet in LDS and the fp32 sums of the chunk go to colpart[b][sc][c].
 //   Splitting S gives enough workgroups at B = 1, but not too many: on MI355X
 //   this read peaks (80% of 8 TB/s) with about 1.5 workgroups x 4 rows in
-//   flight per CU; twice that loses 10%.
-// colsum_reduce_kernel: one thread per column sums the S-chunk partials in
-//   chunk order, scales by 1/S and writes x; with PROJ it also forms the 25
-//   projection partials of its 256 columns (x . phi[c,:] and x^2), so the
+//   flight per CU; twice that loses 10%.  With 256*W columns and every row per
+//   workgroup instead, the same number of workgroups meant four times the S
+//   chunks, and narrow layers had the reduce walk up to 384 of them (no-grad
+//   forward at B=1, S=4096, D=512: 30.4 -> 25.6 us; B=4, S=512, D=2048 39.8 ->
+//   38.2; B=4, S=4096, D=4096 392.7 -> 389.1).
+// colsum_reduce_kernel: four groups of 256 threads, each summing a quarter of
+//   the S-chunk partials of 256 columns (one walk over all of them left its
+//   load latency exposed: the forward at D=512 above 48.2 -> 30.4 us), then
+//   scaled by 1/S into x; with PROJ it also forms the 25 projection partials of
+//   its columns (x . phi[c,:] and x^2, six columns of phi per group), so the
 //   dynamic-weight projection needs no extra pass over x.
 // ---------------------------------------------------------------------------
+constexpr int kPoolRG = 4;  // row groups (waves) of a colsum workgroup
+
 // Loads go through a buffer span rebased at each group of UN rows (the host
 // keeps UN rows of K under 2^31 bytes).  The first nt_rows rows of each S
 // chunk are read with the streaming (nt) policy, the rest plain: what
@@ -1239,67 +1247,105 @@ template <typename T, int W, int UN, bool RAG = false>
 __global__ __launch_bounds__(kThreads) void colsum_kernel(const T* __restrict__ H, float* __restrict__ colpart,
                                                           int64_t S, int64_t K, int64_t SC, int nS, int64_t nt_rows,
                                                           int64_t b0) {
+  constexpr int RG = kPoolRG;
+  constexpr int LW = kThreads / RG;  // lanes per row group: LW * W columns
+  __shared__ float sums[kThreads * W];
   const int64_t b = b0 + blockIdx.z;
   const int sc = blockIdx.y;
-  const int64_t cblk = (int64_t)blockIdx.x * (kThreads * W);
-  if (cblk + (int64_t)threadIdx.x * W >= K) return;
-  const RowCol<W, RAG> rc(threadIdx.x, (uint32_t)(K - cblk < kThreads * W ? K - cblk : kThreads * W));
+  static_assert(LW % 64 == 0, "a wave lies in one row group: its buffer spans stay in SGPRs");
+  const int lane = threadIdx.x % LW;
+  const int rg = __builtin_amdgcn_readfirstlane(threadIdx.x / LW);
+  const int64_t cblk = (int64_t)blockIdx.x * (LW * W);
+  const bool live = cblk + (int64_t)lane * W < K;
+  const RowCol<W, RAG> rc(live ? lane : 0, (uint32_t)(K - cblk < LW * W ? K - cblk : LW * W));
   const int64_t col = cblk + rc.col;
-  const int64_t sbeg = (int64_t)sc * SC;
-  const int64_t send = sbeg + SC < S ? sbeg + SC : S;
+  // the chunk's rows in RG consecutive runs, one per row group
+  const int64_t sbeg0 = (int64_t)sc * SC;
+  const int64_t send0 = sbeg0 + SC < S ? sbeg0 + SC : S;
+  const int64_t run = (send0 - sbeg0 + RG - 1) / RG;
+  const int64_t sbeg = sbeg0 + rg * run < send0 ? sbeg0 + rg * run : send0;
+  const int64_t send = sbeg + run < send0 ? sbeg + run : send0;
   const int64_t smid = sbeg + nt_rows < send ? sbeg + nt_rows : send;
   float acc[W];
 #pragma unroll
   for (int e = 0; e < W; ++e) acc[e] = 0.f;
-  const T* base = H + b * S * K + cblk;
-  const uint32_t lane_e = rc.col;
-  int64_t s = sbeg;
-  colsum_rows<true, T, W, UN, RAG>(base, K, lane_e, s, smid, acc);
-  colsum_rows<false, T, W, UN, RAG>(base, K, lane_e, s, send, acc);
+  if (live) {
+    const T* base = H + b * S * K + cblk;
+    const uint32_t lane_e = rc.col;
+    int64_t s = sbeg;
+    colsum_rows<true, T, W, UN, RAG>(base, K, lane_e, s, smid, acc);
+    colsum_rows<false, T, W, UN, RAG>(base, K, lane_e, s, send, acc);
+  }
+#pragma unroll
+  for (int e = 0; e < W; ++e) sums[(rg * W + e) * LW + lane] = acc[e];
+  __syncthreads();
+  if (rg != 0 || !live) return;
+#pragma unroll
+  for (int g = 1; g < RG; ++g)
+#pragma unroll
+    for (int e = 0; e < W; ++e) acc[e] += sums[(g * W + e) * LW + lane];
   float* out = colpart + ((b * nS + sc) * K + col);
   if constexpr (RAG) st_from<float, W, false>(RagSpan<float>(out, W), 0u, acc, rc.skip);
   else st<float, W>(out, acc);
 }
 
+constexpr int kRedGroups = 4;
+constexpr int kRedCols = kOut / kRedGroups;
+
 template <bool PROJ>
-__global__ __launch_bounds__(kThreads) void colsum_reduce_kernel(const float* __restrict__ colpart,
-                                                                 float* __restrict__ x,
-                                                                 const float* __restrict__ phi,
-                                                                 float* __restrict__ projpart, int64_t K, int nS,
-                                                                 float inv_S, int64_t b0, bool phi_vec) {
-  __shared__ float red[(kThreads / 16) * kPart];
+__global__ __launch_bounds__(kThreads * kRedGroups) void colsum_reduce_kernel(
+    const float* __restrict__ colpart, float* __restrict__ x, const float* __restrict__ phi,
+    float* __restrict__ projpart, int64_t K, int nS, float inv_S, int64_t b0) {
+  __shared__ float part[kRedGroups][kThreads];
+  __shared__ float red[kThreads / 16][kPart];
   const int64_t b = b0 + blockIdx.y;
-  const int64_t c = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-  float pv[kPart];
+  const int lc = threadIdx.x & (kThreads - 1), grp = threadIdx.x >> 8;
+  const int64_t c = (int64_t)blockIdx.x * kThreads + lc;
+  float ph[kRedCols];
 #pragma unroll
-  for (int j = 0; j < kPart; ++j) pv[j] = 0.f;
+  for (int j = 0; j < kRedCols; ++j) ph[j] = 0.f;
+  float v = 0.f;
   if (c < K) {
-    const float* p = colpart + b * nS * K + c;
-    float v = 0.f;
-#pragma unroll 8
-    for (int k = 0; k < nS; ++k) v += p[(int64_t)k * K];
-    v *= inv_S;
-    if (x) x[b * K + c] = v;  // with the projection x is optional (nothing reads it after a no-grad forward)
     if constexpr (PROJ) {
-      float ph[kOut];
-      load_phi_row(phi, c, phi_vec, ph);
 #pragma unroll
-      for (int j = 0; j < kOut; ++j) pv[j] = v * ph[j];
-      pv[kOut] = v * v;
+      for (int j = 0; j < kRedCols; ++j) ph[j] = phi[c * kOut + grp * kRedCols + j];
     }
+    const int per = (nS + kRedGroups - 1) / kRedGroups;
+    const int k1 = (grp + 1) * per < nS ? (grp + 1) * per : nS;
+    const float* p = colpart + b * nS * K + c;
+#pragma unroll 8
+    for (int k = grp * per; k < k1; ++k) v += p[(int64_t)k * K];
   }
+  part[grp][lc] = v;
+  __syncthreads();
+  v = (((part[0][lc] + part[1][lc]) + part[2][lc]) + part[3][lc]) * inv_S;
+  if (grp == 0 && c < K && x) x[b * K + c] = v;  // optional: nothing reads x after a no-grad forward
   if constexpr (PROJ) {
-    const float tot = block_sum_rows<kPart>(pv, red);
-    if (threadIdx.x < kPart) projpart[(b * gridDim.x + blockIdx.x) * kPart + threadIdx.x] = tot;
+    if (c >= K) v = 0.f;
+    const int row = lc >> 4;
+#pragma unroll
+    for (int j = 0; j < kRedCols; ++j) {
+      const float t = sum_all16(v * ph[j]);
+      if ((lc & 15) == 0) red[row][grp * kRedCols + j] = t;
+    }
+    if (grp == 0) {
+      const float t = sum_all16(v * v);
+      if ((lc & 15) == 0) red[row][kOut] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < kPart) {
+      float t = 0.f;
+#pragma unroll
+      for (int q = 0; q < kThreads / 16; ++q) t += red[q][threadIdx.x];
+      projpart[(b * gridDim.x + blockIdx.x) * kPart + threadIdx.x] = t;
+    }
   }
 }
 
-// Short sequences (the decode regime): the two kernels above in one launch.
-// One thread per column sums H[b, s, c] over the same S chunks of SC rows, in
-// the same order, as colsum_kernel and colsum_reduce_kernel do (each chunk from
-// zero, then the chunk sums in chunk order, then the 1/S scale), so x and the
-// projection partials come out bit for bit as on the two-kernel path; what
-// goes is the column-partial round trip and one dependent launch.
+// Short sequences (the decode regime): the two kernels above in one launch, one
+// thread per column (S chunks of SC rows, each from zero, then the chunk sums in
+// order and the 1/S scale); what goes is the column-partial round trip and one
+// dependent launch.
 template <typename T, bool PROJ>
 __global__ __launch_bounds__(kThreads) void colsum_direct_kernel(const T* __restrict__ H, float* __restrict__ x,
                                                                  const float* __restrict__ phi,
@@ -1380,7 +1426,7 @@ __global__ __launch_bounds__(kThreads) void colsum_direct_vec_kernel(const T* __
 // workspace sizes can be queried without a device.
 struct PoolPlan {
   int W;         // elements per lane (16 bytes, or 1 on the unaligned path)
-  int64_t ncc;   // column chunks of 256*W
+  int64_t ncc;   // column chunks of 64 * W
   int64_t SC;    // rows per S chunk
   int nS;        // S chunks
   int64_t nrc;   // column chunks of the reduce kernel (256 columns)
@@ -1391,7 +1437,8 @@ constexpr int kPoolWG = 384;  // target colsum workgroups: 1.5 per CU on MI355X
 __host__ inline PoolPlan pool_plan(int64_t B, int64_t S, int64_t K, int W) {
   PoolPlan p;
   p.W = W;
-  p.ncc = (K + kThreads * W - 1) / (kThreads * W);
+  const int64_t cols = kThreads / kPoolRG * W;
+  p.ncc = (K + cols - 1) / cols;
   if (p.ncc < 1) p.ncc = 1;
   const int64_t per = p.ncc * (B > 0 ? B : 1);
   int64_t ns = (kPoolWG + per - 1) / per;

@@ -134,3 +134,21 @@ def test_mixed_types_on_ragged_rows():
         whole = hc(H)[1](bo)
         for s in range(0, 200, 50):
             assert torch.equal(hc(H[:, s:s + 50].contiguous())[1](bo[:, s:s + 50].contiguous()), whole[:, s:s + 50])
+
+
+@pytest.mark.parametrize("B,S,D,dtype", [
+    # one column chunk in 384 S chunks of a few rows, rows that leave whole waves without any (S = 9:
+    # one chunk of a row per wave), a partial last chunk, a column chunk of one vector
+    (1, 4096, 128, torch.bfloat16), (1, 9, 64, torch.float32), (130, 9, 512, torch.bfloat16),
+    (3, 1027, 130, torch.float16), (2, 517, 1032, torch.bfloat16)])
+def test_mean_pool_chunks(B, S, D, dtype):
+    """fp32 sums of S unit normals, each within 2^-24 of its partial sum (a few sqrt(S)): the mean is
+    off by at most a few 2^-24, far inside 2^-16."""
+    from mhc._kernels import mean_pool
+
+    g = torch.Generator(device=DEV).manual_seed(4)
+    H = torch.randn((B, S, 4, D), generator=g, device=DEV).to(dtype)
+    want = H.double().mean(dim=1).reshape(B, 4 * D)
+    assert float((mean_pool(H).double() - want).abs().max()) <= 2.0 ** -16
+    hc, H, bo, dHn, dbi = make_case(min(B, 3), S, D, dtype, phi_std=0.02)
+    check_layer(hc, H, bo, dHn, dbi, *FWD[dtype], 1e-4)
