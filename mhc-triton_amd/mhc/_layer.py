@@ -21,6 +21,10 @@ writes the complete ``dH`` once.  The engine sums the closure's
 gradients when it is called more than once, and a backward call that reaches
 node B but not node A leaves no state behind.  The traced path (``_library.py``)
 uses the same wiring on the ``torch.ops.mhc`` ops.
+
+Plain eager calls on the GPU take the dynamic, static and closure nodes in C++
+(csrc/native/native.cpp: the same inputs, outputs and saved tensors); the Python
+ones here serve the calls that those leave alone.
 """
 
 from __future__ import annotations

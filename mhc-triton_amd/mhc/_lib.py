@@ -98,6 +98,27 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The binding of the eager entry points (csrc/native/native.cpp, built next to the library).  Its
+    functions return None for calls they leave to the Python nodes."""
+    global _native
+    if _native is None:
+        load()
+        with _lock:
+            if _native is None:
+                try:
+                    from . import _native as mod
+                except ImportError as e:
+                    raise MHCError(f"mhc: binding not built or not loadable ({e}); run `make -C mhc-triton_amd` or "
+                                   "`python -c 'import __graft_entry__ as g; g.build()'`") from e
+                mod.set_error(MHCError)
+                _native = mod
+    return _native
+
+
 def check(rc: int, name: str) -> None:
     if rc != 0:
         msg = load().mhc_last_error().decode(errors="replace")

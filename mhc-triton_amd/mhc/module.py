@@ -13,7 +13,7 @@ from typing import Callable, Tuple
 import torch
 import torch.nn as nn
 
-from . import _layer, _library
+from . import _layer, _lib, _library
 from ._kernels import mean_pool
 from .ops import fused_add_residual, fused_dynamic_weights, fused_stream_mix, sinkhorn_knopp
 
@@ -180,7 +180,17 @@ class HyperConnection(nn.Module):
             return self._forward_traced(H)
         # inference tensors (made under torch.inference_mode) keep no version counter
         version = None if H.is_inference() else H._version
-        if not self.dynamic:
+        # plain eager calls take node A and the closure in C++, the rest the Python nodes
+        native = _lib.native() if H.is_cuda else None
+        out = None
+        if native is not None and not self.dynamic:
+            out = native.static_layer(H, self.H_pre_base, self.H_post_base, self.H_res_base, self.sinkhorn_iters)
+        elif native is not None and self.use_fused_weights:
+            out = native.dynamic_layer(H, self.phi, self.H_pre_base, self.H_post_base, self.H_res_base,
+                                       self.alpha_pre, self.alpha_post, self.alpha_res, self.sinkhorn_iters, self.eps)
+        if out is not None:
+            bi, w, link, post_link = out
+        elif not self.dynamic:
             bi, w, link, post_link = _layer._StaticLayer.apply(H, self.H_pre_base, self.H_post_base,
                                                                self.H_res_base, self.sinkhorn_iters)
         elif self.use_fused_weights:
@@ -203,7 +213,8 @@ class HyperConnection(nn.Module):
                     "HyperConnection: H was modified in place after forward(H); add_residual recomputes "
                     "H_res @ H from H and would mix the modified values. Clone H before modifying it "
                     "(the version counter is shared by every view of H's storage).")
-            return _layer._LayerAdd.apply(link, branch_output, w, post_link)
+            H_new = native.layer_add(link, branch_output, w, post_link) if native is not None else None
+            return _layer._LayerAdd.apply(link, branch_output, w, post_link) if H_new is None else H_new
 
         return bi, add_residual
 

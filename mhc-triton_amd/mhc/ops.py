@@ -1,7 +1,9 @@
 """High-level ops with autograd support (reference src/mhc/ops.py).
 
 Same Function names, forward signatures, outputs and gradient signatures as the
-reference; every forward and backward runs on the gfx950 HIP kernels.
+reference; every forward and backward runs on the gfx950 HIP kernels.  Plain eager
+calls take the same nodes in C++ (``_lib.native()``); the Functions here serve the
+calls that the C++ nodes leave alone.
 """
 
 from __future__ import annotations
@@ -12,6 +14,7 @@ import torch
 
 from . import _backward as _bwd
 from . import _kernels as _k
+from . import _lib
 from . import _library  # noqa: F401  (registers torch.ops.mhc.*)
 
 
@@ -102,6 +105,10 @@ def sinkhorn_knopp(M: torch.Tensor, num_iters: int = 20, eps: float = 1e-8) -> t
     """Project (batch, 4, 4) matrices to doubly stochastic via Sinkhorn-Knopp."""
     if torch.compiler.is_compiling():
         return torch.ops.mhc.sinkhorn_forward(M, num_iters, eps)
+    if M.is_cuda:
+        P = _lib.native().sinkhorn(M, num_iters, eps)
+        if P is not None:
+            return P
     return _SinkhornKnopp.apply(M, num_iters, eps)
 
 
@@ -109,6 +116,10 @@ def fused_stream_mix(H: torch.Tensor, H_pre: torch.Tensor, H_res: torch.Tensor) 
     """branch_input (batch, seq, dim) and H_residual (batch, seq, 4, dim) of H (batch, seq, 4, dim)."""
     if torch.compiler.is_compiling():
         return torch.ops.mhc.stream_mix_forward(H, H_pre, H_res)
+    if H.is_cuda:
+        out = _lib.native().stream_mix(H, H_pre, H_res)
+        if out is not None:
+            return out
     return _FusedStreamMix.apply(H, H_pre, H_res)
 
 
@@ -116,6 +127,10 @@ def fused_add_residual(H_residual: torch.Tensor, branch_output: torch.Tensor, H_
     """H_new[n] = H_residual[n] + H_post[n] * branch_output."""
     if torch.compiler.is_compiling():
         return torch.ops.mhc.add_residual_forward(H_residual, branch_output, H_post)
+    if H_residual.is_cuda:
+        H_new = _lib.native().add_residual(H_residual, branch_output, H_post)
+        if H_new is not None:
+            return H_new
     return _FusedAddResidual.apply(H_residual, branch_output, H_post)
 
 
@@ -134,4 +149,8 @@ def fused_dynamic_weights(
         alphas = [a if isinstance(a, torch.Tensor) else torch.tensor([float(a)], device=x.device)
                   for a in (alpha_pre, alpha_post, alpha_res)]
         return torch.ops.mhc.dynamic_weights_forward(x, phi, bias, *alphas, sinkhorn_iters, eps)[:3]
+    if x.is_cuda:
+        out = _lib.native().dynamic_weights(x, phi, bias, alpha_pre, alpha_post, alpha_res, sinkhorn_iters, eps)
+        if out is not None:
+            return out
     return _FusedDynamicWeights.apply(x, phi, bias, alpha_pre, alpha_post, alpha_res, sinkhorn_iters, eps)

@@ -21,6 +21,7 @@ from typing import Optional
 import torch
 
 from . import _kernels as _k
+from . import _lib
 from . import _library  # noqa: F401  (registers torch.ops.mhc.*)
 
 __all__ = ["expand_streams", "collapse_streams"]
@@ -59,6 +60,10 @@ def expand_streams(x: torch.Tensor, num_streams: int = 4, scale: float = 1.0,
         raise ValueError("HIP kernels require num_streams=4")
     if torch.compiler.is_compiling():
         return torch.ops.mhc.stream_expand(x, float(scale), dtype)
+    if dtype is None and x.is_cuda:
+        H = _lib.native().expand(x, float(scale))
+        if H is not None:
+            return H
     return _StreamExpand.apply(x, float(scale), dtype)
 
 
@@ -70,4 +75,8 @@ def collapse_streams(H: torch.Tensor, reduction: str = "mean",
     scale = _REDUCTIONS[reduction]
     if torch.compiler.is_compiling():
         return torch.ops.mhc.stream_collapse(H, scale, dtype)
+    if dtype is None and H.is_cuda:
+        y = _lib.native().collapse(H, scale)
+        if y is not None:
+            return y
     return _StreamCollapse.apply(H, scale, dtype)
