@@ -330,6 +330,18 @@ int mhc_stream_expand(const void* x, int dtype_x, void* H, int dtype_h, int64_t 
 int mhc_stream_collapse(const void* H, int dtype_h, void* y, int dtype_y, int64_t B, int64_t S,
                         int64_t D, float scale, mhc_stream_t stream);
 
+/* ------------------------------------------------------------------------
+ * Small tensors between dtypes, in one launch: dst[i][0:count[i]] =
+ * src[i][0:count[i]] for i < n <= MHC_CONVERT_MAX, each in its own dtype
+ * (round to nearest even).  A module cast to 16 bits has seven parameters to
+ * convert before its kernels and seven gradients after them.  The four arrays
+ * are host memory, read before the call returns; src and dst may not overlap.
+ * ------------------------------------------------------------------------ */
+#define MHC_CONVERT_MAX 8
+
+int mhc_convert(int n, const void* const* src, const int* src_dtype, void* const* dst, const int* dst_dtype,
+                const int64_t* count, mhc_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

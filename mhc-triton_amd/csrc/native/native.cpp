@@ -84,6 +84,73 @@ Tensor empty_f32(at::IntArrayRef sizes, const Tensor& like) {
   return at::empty(sizes, like.options().dtype(at::kFloat).requires_grad(false));
 }
 
+// The f32 values of N <= 8 parameters: the parameters' own memory, or, where any is stored in another
+// dtype, one buffer of them all, converted in one launch.  The forward keeps the buffer for the
+// backward (which then reads nothing from the parameters, so what a saved-tensor hook does to their
+// layout does not matter).
+template <int N>
+struct Params {
+  const float* p[N];
+  Tensor buf;
+
+  Params(const Tensor* t, const Tensor& have) : buf(have) {
+    int64_t at[N], total = 0;
+    bool own = !buf.defined();
+    for (int i = 0; i < N; ++i) {
+      at[i] = total;
+      total += (t[i].numel() + 3) / 4 * 4;  // 16-byte aligned parts
+      own = own && t[i].scalar_type() == at::kFloat && t[i].is_contiguous();
+    }
+    if (own) {
+      for (int i = 0; i < N; ++i) p[i] = fptr(t[i]);
+      return;
+    }
+    if (!buf.defined()) {
+      buf = empty_f32({total}, t[0]);
+      const void* src[N];
+      void* dst[N];
+      int sd[N], dd[N];
+      int64_t count[N];
+      Tensor hold[N];
+      for (int i = 0; i < N; ++i) {
+        hold[i] = (code(t[i]) < 0 ? t[i].to(at::kFloat) : t[i]).contiguous();
+        src[i] = ptr(hold[i]);
+        sd[i] = code(hold[i]);
+        dst[i] = wptr(buf) + at[i];
+        dd[i] = MHC_DTYPE_F32;
+        count[i] = hold[i].numel();
+      }
+      check(mhc_convert(N, src, sd, dst, dd, count, stream(buf)), "convert");
+    }
+    for (int i = 0; i < N; ++i) p[i] = fptr(buf) + at[i];
+  }
+};
+
+// The gradients of N parameters from f32 parts, each in its parameter's shape and dtype; those that
+// are not f32 are converted in one launch.
+template <int N>
+void param_grads(const Tensor* prm, const Tensor* part, variable_list& out) {
+  const void* src[N];
+  void* dst[N];
+  int sd[N], dd[N], n = 0;
+  int64_t count[N];
+  for (int i = 0; i < N; ++i) {
+    const Tensor& p = prm[i];
+    if (p.scalar_type() == at::kFloat || code(p) < 0) {
+      out.push_back(grad_like(part[i], p));
+      continue;
+    }
+    Tensor g = at::empty(p.sizes(), p.options().requires_grad(false));
+    src[n] = ptr(part[i]);
+    sd[n] = MHC_DTYPE_F32;
+    dst[n] = ptr(g);
+    dd[n] = code(p);
+    count[n++] = p.numel();
+    out.push_back(std::move(g));
+  }
+  if (n) check(mhc_convert(n, src, sd, dst, dd, count, stream(part[0])), "convert");
+}
+
 struct Workspace {
   Tensor t;
   size_t bytes;
@@ -166,22 +233,23 @@ struct Dims {
 // phi, H_pre_base, H_post_base, H_res_base, alpha_pre, alpha_post, alpha_res
 constexpr int kDyn = 7;
 
-struct DynOut { Tensor bi, x, w, aux; };
+struct DynOut { Tensor bi, x, w, aux, params; };
 
 DynOut dynamic_forward(const Tensor& H, const Tensor* prm, int64_t iters, double eps, bool keep_x) {
   const c10::DeviceGuard guard(H.device());
   const Dims d(H);
-  Tensor p[kDyn];
-  for (int i = 0; i < kDyn; ++i) p[i] = f32(prm[i]);
+  const Params<kDyn> q(prm, Tensor());
+  const float* const* p = q.p;
   DynOut o;
+  o.params = q.buf;
   o.bi = at::empty({d.B, d.S, d.D}, H.options().requires_grad(false));
   if (keep_x) o.x = empty_f32({d.B, 4 * d.D}, H);
   o.w = empty_f32({d.B, 24}, H);
   o.aux = empty_f32({d.B, 25}, H);
   const Workspace ws(mhc_layer_workspace_bytes(d.B, d.S, d.D, code(H)), H);
-  check(mhc_layer_dynamic_forward(ptr(H), code(H), fptr(p[0]), fptr(p[1]), fptr(p[2]), fptr(p[3]), fptr(p[4]),
-                                  fptr(p[5]), fptr(p[6]), ptr(o.bi), wptr(o.x), wptr(o.w), wptr(o.aux), d.B, d.S, d.D,
-                                  (int)iters, (float)eps, ws.p(), ws.bytes, stream(H)),
+  check(mhc_layer_dynamic_forward(ptr(H), code(H), p[0], p[1], p[2], p[3], p[4], p[5], p[6], ptr(o.bi), wptr(o.x),
+                                  wptr(o.w), wptr(o.aux), d.B, d.S, d.D, (int)iters, (float)eps, ws.p(), ws.bytes,
+                                  stream(H)),
         "layer_dynamic_forward");
   return o;
 }
@@ -200,7 +268,7 @@ struct DynamicLayer : Function<DynamicLayer> {
     const Tensor prm[kDyn] = {phi, pre, post, res, a_pre, a_post, a_res};
     // at S = 1 the pooled rows are H's rows, which the backward reads from H
     DynOut o = dynamic_forward(H, prm, iters, eps, H.size(1) != 1);
-    ctx->save_for_backward({H, o.x, o.w, o.aux, phi, pre, post, res, a_pre, a_post, a_res});
+    ctx->save_for_backward({H, o.x, o.w, o.aux, phi, pre, post, res, a_pre, a_post, a_res, o.params});
     ctx->saved_data["iters"] = iters;
     ctx->saved_data["eps"] = eps;
     ctx->set_materialize_grads(false);
@@ -216,23 +284,30 @@ struct DynamicLayer : Function<DynamicLayer> {
     const Tensor d_bi = d_bi_or_zeros(g[0], H, d);
     const Tensor dHn = in_dtype(g[2], H.scalar_type());
     const Tensor dpost = f32(g[3]);
-    Tensor p[kDyn];
-    for (int i = 0; i < kDyn; ++i) p[i] = f32(prm[i]);
+    const Params<kDyn> q(prm, s[4 + kDyn]);
+    const float* const* p = q.p;
     const Tensor x = f32(s[1]), w = f32(s[2]), aux = f32(s[3]);
     Tensor dH;
     if (ctx->needs_input_grad(0)) dH = at::empty_like(H);
     const Tensor gphi = empty_f32({4 * d.D, 24}, H);
     const Tensor small = empty_f32({27}, H);  // grad_bias [24], grad_alpha [3]
     const Workspace ws(mhc_layer_workspace_bytes(d.B, d.S, d.D, code(H)), H);
-    check(mhc_layer_dynamic_backward(ptr(H), code(H), ptr(d_bi), ptr(dHn), fptr(dpost), fptr(p[0]), fptr(p[1]),
-                                     fptr(p[2]), fptr(p[3]), fptr(p[4]), fptr(p[5]), fptr(p[6]), fptr(x), fptr(w),
-                                     fptr(aux), ptr(dH), wptr(gphi), wptr(small), wptr(small) + 24, d.B, d.S, d.D,
-                                     (int)ctx->saved_data["iters"].toInt(), (float)ctx->saved_data["eps"].toDouble(),
-                                     ws.p(), ws.bytes, stream(H)),
+    check(mhc_layer_dynamic_backward(ptr(H), code(H), ptr(d_bi), ptr(dHn), fptr(dpost), p[0], p[1], p[2], p[3], p[4],
+                                     p[5], p[6], fptr(x), fptr(w), fptr(aux), ptr(dH), wptr(gphi), wptr(small),
+                                     wptr(small) + 24, d.B, d.S, d.D, (int)ctx->saved_data["iters"].toInt(),
+                                     (float)ctx->saved_data["eps"].toDouble(), ws.p(), ws.bytes, stream(H)),
           "layer_dynamic_backward");
-    auto part = [&](int i, int64_t at, int64_t n) { return grad_like(small.narrow(0, at, n), prm[i]); };
-    return {dH,           grad_like(gphi, prm[0]), part(1, 0, 4),  part(2, 4, 4), part(3, 8, 16),
-            part(4, 24, 1), part(5, 25, 1),          part(6, 26, 1), Tensor(),      Tensor()};
+    const Tensor part[kDyn] = {gphi,
+                               small.narrow(0, 0, 4),
+                               small.narrow(0, 4, 4),
+                               small.narrow(0, 8, 16),
+                               small.narrow(0, 24, 1),
+                               small.narrow(0, 25, 1),
+                               small.narrow(0, 26, 1)};
+    variable_list out{dH};
+    param_grads<kDyn>(prm, part, out);
+    out.resize(kDyn + 3);  // iters, eps
+    return out;
   }
 };
 
@@ -261,16 +336,17 @@ PyObject* py_dynamic_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-struct StaticOut { Tensor bi, w; };
+struct StaticOut { Tensor bi, w, params; };
 
 StaticOut static_forward(const Tensor& H, const Tensor* prm, int64_t iters) {
   const c10::DeviceGuard guard(H.device());
   const Dims d(H);
-  const Tensor p[3] = {f32(prm[0]), f32(prm[1]), f32(prm[2])};
+  const Params<3> q(prm, Tensor());
   StaticOut o;
+  o.params = q.buf;
   o.bi = at::empty({d.B, d.S, d.D}, H.options().requires_grad(false));
   o.w = empty_f32({d.B, 24}, H);
-  check(mhc_layer_static_forward(ptr(H), code(H), fptr(p[0]), fptr(p[1]), fptr(p[2]), ptr(o.bi), wptr(o.w), d.B, d.S,
+  check(mhc_layer_static_forward(ptr(H), code(H), q.p[0], q.p[1], q.p[2], ptr(o.bi), wptr(o.w), d.B, d.S,
                                  d.D, (int)iters, stream(H)),
         "layer_static_forward");
   return o;
@@ -281,7 +357,7 @@ struct StaticLayer : Function<StaticLayer> {
                                const Tensor& res, int64_t iters) {
     const Tensor prm[3] = {pre, post, res};
     StaticOut o = static_forward(H, prm, iters);
-    ctx->save_for_backward({H, o.w, pre, post, res});
+    ctx->save_for_backward({H, o.w, pre, post, res, o.params});
     ctx->saved_data["iters"] = iters;
     ctx->set_materialize_grads(false);
     return {o.bi, o.w, H.view_as(H), post_link(o.w)};
@@ -296,17 +372,19 @@ struct StaticLayer : Function<StaticLayer> {
     const Tensor d_bi = d_bi_or_zeros(g[0], H, d);
     const Tensor dHn = in_dtype(g[2], H.scalar_type());
     const Tensor dpost = f32(g[3]), w = f32(s[1]);
-    const Tensor p[3] = {f32(prm[0]), f32(prm[1]), f32(prm[2])};
+    const Params<3> q(prm, s[5]);
     Tensor dH;
     if (ctx->needs_input_grad(0)) dH = at::empty_like(H);
     const Tensor gb = empty_f32({24}, H);
     const Workspace ws(mhc_layer_workspace_bytes(d.B, d.S, d.D, code(H)), H);
-    check(mhc_layer_static_backward(ptr(H), code(H), ptr(d_bi), ptr(dHn), fptr(dpost), fptr(p[0]), fptr(p[1]),
-                                    fptr(p[2]), fptr(w), ptr(dH), wptr(gb), d.B, d.S, d.D,
+    check(mhc_layer_static_backward(ptr(H), code(H), ptr(d_bi), ptr(dHn), fptr(dpost), q.p[0], q.p[1], q.p[2], fptr(w), ptr(dH), wptr(gb), d.B, d.S, d.D,
                                     (int)ctx->saved_data["iters"].toInt(), ws.p(), ws.bytes, stream(H)),
           "layer_static_backward");
-    return {dH, grad_like(gb.narrow(0, 0, 4), prm[0]), grad_like(gb.narrow(0, 4, 4), prm[1]),
-            grad_like(gb.narrow(0, 8, 16), prm[2]), Tensor()};
+    const Tensor part[3] = {gb.narrow(0, 0, 4), gb.narrow(0, 4, 4), gb.narrow(0, 8, 16)};
+    variable_list out{dH};
+    param_grads<3>(prm, part, out);
+    out.resize(5);  // iters
+    return out;
   }
 };
 
@@ -541,18 +619,17 @@ PyObject* py_add_residual(PyObject*, PyObject* const* a, Py_ssize_t n) {
 // x, phi, bias, alpha_pre, alpha_post, alpha_res
 constexpr int kDw = 6;
 
-struct DwOut { Tensor pre, post, res, aux; };
+struct DwOut { Tensor pre, post, res, aux, params; };
 
 DwOut dynamic_weights_forward(const Tensor* t, int64_t iters, double eps) {
   const c10::DeviceGuard guard(t[0].device());
   const Tensor x = t[0].contiguous();
   const int64_t R = x.size(0), K = x.size(1);
-  Tensor p[kDw];
-  for (int i = 1; i < kDw; ++i) p[i] = f32(t[i]);
-  DwOut o{empty_f32({R, 4}, x), empty_f32({R, 4}, x), empty_f32({R, 4, 4}, x), empty_f32({R, 25}, x)};
+  const Params<kDw - 1> q(t + 1, Tensor());
+  const float* const* p = q.p;
+  DwOut o{empty_f32({R, 4}, x), empty_f32({R, 4}, x), empty_f32({R, 4, 4}, x), empty_f32({R, 25}, x), q.buf};
   const Workspace ws(mhc_dynamic_weights_workspace_bytes(R, K), x);
-  check(mhc_dynamic_weights_forward(ptr(x), code(x), fptr(p[1]), fptr(p[2]), fptr(p[3]), fptr(p[4]), fptr(p[5]),
-                                    wptr(o.pre), wptr(o.post), wptr(o.res), wptr(o.aux), R, K, (int)iters, (float)eps,
+  check(mhc_dynamic_weights_forward(ptr(x), code(x), p[0], p[1], p[2], p[3], p[4], wptr(o.pre), wptr(o.post), wptr(o.res), wptr(o.aux), R, K, (int)iters, (float)eps,
                                     ws.p(), ws.bytes, stream(x)),
         "dynamic_weights_forward");
   return o;
@@ -564,7 +641,7 @@ struct DynamicWeights : Function<DynamicWeights> {
                                double eps) {
     const Tensor t[kDw] = {x, phi, bias, a_pre, a_post, a_res};
     DwOut o = dynamic_weights_forward(t, iters, eps);
-    ctx->save_for_backward({x, phi, bias, a_pre, a_post, a_res, o.pre, o.aux});
+    ctx->save_for_backward({x, phi, bias, a_pre, a_post, a_res, o.pre, o.aux, o.params});
     ctx->saved_data["iters"] = iters;
     ctx->saved_data["eps"] = eps;
     ctx->set_materialize_grads(false);
@@ -576,20 +653,23 @@ struct DynamicWeights : Function<DynamicWeights> {
     const c10::DeviceGuard guard(s[0].device());
     const Tensor x = s[0].contiguous();
     const int64_t R = x.size(0), K = x.size(1);
-    Tensor p[kDw];
-    for (int i = 1; i < kDw; ++i) p[i] = f32(s[i]);
+    const Params<kDw - 1> q(&s[1], s[8]);
+    const float* const* p = q.p;
     const Tensor g0 = f32(g[0]), g1 = f32(g[1]), g2 = f32(g[2]);
     const Tensor gx = at::empty(x.sizes(), x.options().requires_grad(false));
     const Tensor gphi = empty_f32({K, 24}, x), small = empty_f32({27}, x);
     const Workspace ws(mhc_dynamic_weights_backward_workspace_bytes(R, K), x);
-    check(mhc_dynamic_weights_backward(ptr(x), code(x), fptr(p[1]), fptr(p[2]), fptr(p[3]), fptr(p[4]), fptr(p[5]),
-                                       fptr(s[7]), fptr(s[6]), fptr(g0), fptr(g1), fptr(g2), ptr(gx), wptr(gphi),
-                                       wptr(small), wptr(small) + 24, R, K, (int)ctx->saved_data["iters"].toInt(),
+    check(mhc_dynamic_weights_backward(ptr(x), code(x), p[0], p[1], p[2], p[3], p[4], fptr(s[7]), fptr(s[6]), fptr(g0),
+                                       fptr(g1), fptr(g2), ptr(gx), wptr(gphi), wptr(small), wptr(small) + 24, R, K,
+                                       (int)ctx->saved_data["iters"].toInt(),
                                        (float)ctx->saved_data["eps"].toDouble(), ws.p(), ws.bytes, stream(x)),
           "dynamic_weights_backward");
-    auto part = [&](int i, int64_t at, int64_t n) { return grad_like(small.narrow(0, at, n), s[i]); };
-    return {gx,          grad_like(gphi, s[1]), part(2, 0, 24), part(3, 24, 1),
-            part(4, 25, 1), part(5, 26, 1),        Tensor(),       Tensor()};
+    const Tensor part[kDw - 1] = {gphi, small.narrow(0, 0, 24), small.narrow(0, 24, 1), small.narrow(0, 25, 1),
+                                  small.narrow(0, 26, 1)};
+    variable_list out{gx};
+    param_grads<kDw - 1>(&s[1], part, out);
+    out.resize(kDw + 2);  // iters, eps
+    return out;
   }
 };
 

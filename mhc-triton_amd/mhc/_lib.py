@@ -30,6 +30,7 @@ _SZ = ctypes.c_size_t
 _SIGNATURES = {
     "mhc_abi_version": (_I, []),
     "mhc_last_error": (ctypes.c_char_p, []),
+    "mhc_convert": (_I, [_I, _P, _P, _P, _P, _P, _P]),
     "mhc_sinkhorn_forward": (_I, [_P, _P, _I64, _I, _I, _F, _P]),
     "mhc_sinkhorn_backward": (_I, [_P, _I, _P, _I, _P, _I64, _I, _F, _P]),
     "mhc_stream_mix_forward": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _P]),

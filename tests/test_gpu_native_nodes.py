@@ -174,3 +174,24 @@ def test_in_place_change_of_a_saved_parameter_is_refused():
         hc.phi.mul_(2)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         torch.autograd.backward([add(bo), bi], [dHn, dbi])
+
+
+@pytest.mark.parametrize("dtypes", [(torch.bfloat16,) * 7, (torch.float16, torch.float32, torch.bfloat16, torch.float64,
+                                                            torch.float32, torch.float16, torch.float32)])
+@pytest.mark.parametrize("offload", [False, True])
+def test_converted_parameters(monkeypatch, dtypes, offload):
+    """Parameters in 16 bits, and each in its own dtype (phi strided besides): converted in one launch
+    into a buffer that the backward reads, also through hooks that change the saved layout."""
+    hc, H, bo, dHn, dbi = make_case(3, 7, 20, torch.float32, phi_std=0.02, res_std=1.0)
+    for p, dt in zip((hc.phi, hc.H_pre_base, hc.H_post_base, hc.H_res_base, hc.alpha_pre, hc.alpha_post, hc.alpha_res),
+                     dtypes):
+        p.data = p.data.to(dt)
+    hc.phi.data = hc.phi.data.T.contiguous().T
+
+    def step():
+        hooks = (lambda t: t.cpu(), lambda t: t.to(DEV).contiguous()) if offload else (lambda t: t, lambda t: t)
+        with torch.autograd.graph.saved_tensors_hooks(*hooks):
+            bi, Hn, grads = run_gpu(hc, H, bo, dHn, dbi)
+        return [bi, Hn] + [grads[k] for k in sorted(grads)]
+
+    same(*both(monkeypatch, step))
