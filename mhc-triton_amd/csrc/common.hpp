@@ -447,16 +447,17 @@ __device__ __forceinline__ float sum_col16(float v) {
 
 __device__ __forceinline__ float sum_all16(float v) { return sum_col16(sum_row16(v)); }
 
-// Sum of NV (<= 256) per-thread values over a 256-thread workgroup, for many
+// Sum of NV (<= NTH) per-thread values over a workgroup of NTH threads, for many
 // values at once: each 16-lane row adds with DPP (sum_all16, full-rate VALU
-// with no LDS crossbar traffic), the 16 row sums of each value go through LDS,
+// with no LDS crossbar traffic), the row sums of each value go through LDS,
 // and thread i < NV adds value i's row sums in row order.  Returns the total
 // of value threadIdx.x in threads < NV.  A wave butterfly over __shfl_xor costs
 // 6 ds_bpermute per value instead (600 for the weights projection's 100
 // partials).
-template <int NV>
+// `lds` must hold NTH / 16 * NV floats.
+template <int NV, int NTH = kThreads>
 __device__ __forceinline__ float block_sum_rows(float (&v)[NV], float* lds) {
-  static_assert(NV <= kThreads, "one output per thread");
+  static_assert(NV <= NTH, "one output per thread");
   const int row = threadIdx.x >> 4;
 #pragma unroll
   for (int i = 0; i < NV; ++i) v[i] = sum_all16(v[i]);
@@ -468,7 +469,7 @@ __device__ __forceinline__ float block_sum_rows(float (&v)[NV], float* lds) {
   float t = 0.f;
   if (threadIdx.x < NV) {
 #pragma unroll
-    for (int q = 0; q < kThreads / 16; ++q) t += lds[q * NV + threadIdx.x];
+    for (int q = 0; q < NTH / 16; ++q) t += lds[q * NV + threadIdx.x];
   }
   return t;
 }

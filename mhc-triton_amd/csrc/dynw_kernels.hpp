@@ -565,6 +565,52 @@ inline hipError_t launch_finalize(const float* part, int nK, int64_t R, int64_t 
   return hipGetLastError();
 }
 
+// The backward of weights_row16 for one row, in 16-lane form: lane e owns H_res element e, lanes
+// 0..3 also H_pre[e], lanes 4..7 H_post[e - 4]; gpre, gpost and hp are those of column e & 3.
+// slot: this lane's LDS slots of the Sinkhorn states, 64 apart.  All 16 lanes take part; with
+// store they write the row's record rb.
+constexpr int kSkSlots = 32;  // Sinkhorn states kept in LDS per lane
+
+__device__ __forceinline__ void weights_row16_bwd(int e, const float* __restrict__ a, const DynParams& P, float hp,
+                                                  float gpre, float gpost, float gres, float* __restrict__ rb,
+                                                  int64_t K, int iters, float eps, float* slot, bool store) {
+  const int j = e & 3;
+  const float inv_rms = a[kOut];
+  const float ar = *P.alpha_res;
+  const float raw_res = a[8 + e];
+  const float raw_pp = a[e & 7];
+  // H_res = Sinkhorn(|s_res| + eps): gradient w.r.t. s_res.
+  const float s_res = inv_rms * ar * raw_res + P.bias_res[e];
+  const float gs_res = iters == 20 ? sk16_backward_fixed<20>(s_res, gres, eps)
+                                   : sk16_backward<kSkSlots>(s_res, gres, iters, eps, slot, 64);
+  // H_pre = sigmoid / (sum + eps) on lanes 0..3, H_post = 2 sigmoid on lanes 4..7.
+  const bool is_pre = (e & 4) == 0;
+  const float al_pp = is_pre ? *P.alpha_pre : *P.alpha_post;
+  const float sg = sigmoidf(inv_rms * al_pp * raw_pp + (is_pre ? P.bias_pre[j] : P.bias_post[j]));
+  const float den = sum_row16(sg) + eps;   // quad 0: sum of the H_pre sigmoids
+  const float dot = sum_row16(gpre * hp);  // quad 0: <g_pre, H_pre>
+  const float gs_pp = is_pre ? (gpre - dot) / den * sg * (1.f - sg) : gpost * 2.f * sg * (1.f - sg);
+  const bool has_pp = e < 8;
+  // Group sums for grad_alpha and the rms path.
+  const float ga_res = sum_all16(gs_res * inv_rms * raw_res);
+  const float ga_pp = sum_row16(has_pp ? gs_pp * inv_rms * raw_pp : 0.f);  // lane 0: pre, lane 4: post
+  const float g_inv = sum_all16(gs_res * ar * raw_res + (has_pp ? gs_pp * al_pp * raw_pp : 0.f));
+  if (!store) return;
+  rb[8 + e] = gs_res * inv_rms * ar;
+  rb[33 + e] = gs_res;
+  if (has_pp) {
+    rb[e] = gs_pp * inv_rms * al_pp;
+    rb[25 + e] = gs_pp;
+  }
+  // inv_rms = 1/rms, rms = sqrt(sum x^2 / K + eps): d rms / d x = x / (K rms)
+  if (e == 0) {
+    rb[24] = g_inv * (-inv_rms * inv_rms) * inv_rms / (float)K;
+    rb[49] = ga_pp;
+    rb[51] = ga_res;
+  }
+  if (e == 4) rb[50] = ga_pp;
+}
+
 // Per-row backward record rowbuf[r][0:52]:
 //   [0:24]  grad_raw  = g_scaled * inv_rms * alpha_g
 //   [24]    coef      : grad_x += coef * x  (rms path)
@@ -584,8 +630,6 @@ inline hipError_t launch_finalize(const float* part, int nK, int64_t R, int64_t 
 // passes the gradients as rows (g_pre [R,4], g_res [R,16]).  Wave 0 then runs
 // the rows in 16-lane form: lane e of a group owns H_res element e, lanes 0..3
 // also H_pre[e], lanes 4..7 H_post[e - 4].
-constexpr int kSkSlots = 32;  // Sinkhorn states kept in LDS per lane
-
 template <int RPW>
 __global__ __launch_bounds__(kThreads) void dynw_bwd_rows_kernel(const float* __restrict__ aux, DynParams P,
                                                                  InRow h_pre, InRow g_pre, InRow g_post,
@@ -655,44 +699,8 @@ __global__ __launch_bounds__(kThreads) void dynw_bwd_rows_kernel(const float* __
   const float gpre = from_part ? red[rr][j] : (g_pre.p ? g_pre.p[r * g_pre.stride + j] : 0.f);
   const float gres = from_part ? red[rr][4 + e] : (g_res.p ? g_res.p[r * g_res.stride + e] : 0.f);
   const float gpost = g_post.p ? g_post.p[r * g_post.stride + j] : 0.f;
-  const float* a = aux + r * kPart;
-  const float inv_rms = a[kOut];
-  const float ar = *P.alpha_res;
-  const float raw_res = a[8 + e];
-  const float raw_pp = a[e & 7];
-  // H_res = Sinkhorn(|s_res| + eps): gradient w.r.t. s_res.
-  const float s_res = inv_rms * ar * raw_res + P.bias_res[e];
-  const float gs_res = iters == 20 ? sk16_backward_fixed<20>(s_res, gres, eps)
-                                   : sk16_backward<kSkSlots>(s_res, gres, iters, eps,
-                                                             slots + (RPW == 16 ? wave * kSkSlots * 64 : 0) + lane, 64);
-  // H_pre = sigmoid / (sum + eps) on lanes 0..3, H_post = 2 sigmoid on lanes 4..7.
-  const bool is_pre = (e & 4) == 0;
-  const float al_pp = is_pre ? *P.alpha_pre : *P.alpha_post;
-  const float sg = sigmoidf(inv_rms * al_pp * raw_pp + (is_pre ? P.bias_pre[j] : P.bias_post[j]));
-  const float hp = h_pre.p[r * h_pre.stride + j];
-  const float den = sum_row16(sg) + eps;   // quad 0: sum of the H_pre sigmoids
-  const float dot = sum_row16(gpre * hp);  // quad 0: <g_pre, H_pre>
-  const float gs_pp = is_pre ? (gpre - dot) / den * sg * (1.f - sg) : gpost * 2.f * sg * (1.f - sg);
-  const bool has_pp = e < 8;
-  // Group sums for grad_alpha and the rms path.
-  const float ga_res = sum_all16(gs_res * inv_rms * raw_res);
-  const float ga_pp = sum_row16(has_pp ? gs_pp * inv_rms * raw_pp : 0.f);  // lane 0: pre, lane 4: post
-  const float g_inv = sum_all16(gs_res * ar * raw_res + (has_pp ? gs_pp * al_pp * raw_pp : 0.f));
-  if (!live) return;
-  float* rb = rowbuf + r * kRow;
-  rb[8 + e] = gs_res * inv_rms * ar;
-  rb[33 + e] = gs_res;
-  if (has_pp) {
-    rb[e] = gs_pp * inv_rms * al_pp;
-    rb[25 + e] = gs_pp;
-  }
-  // inv_rms = 1/rms, rms = sqrt(sum x^2 / K + eps): d rms / d x = x / (K rms)
-  if (e == 0) {
-    rb[24] = g_inv * (-inv_rms * inv_rms) * inv_rms / (float)K;
-    rb[49] = ga_pp;
-    rb[51] = ga_res;
-  }
-  if (e == 4) rb[50] = ga_pp;
+  weights_row16_bwd(e, aux + r * kPart, P, h_pre.p[r * h_pre.stride + j], gpre, gpost, gres, rowbuf + r * kRow, K,
+                    iters, eps, slots + (RPW == 16 ? wave * kSkSlots * 64 : 0) + lane, live);
 }
 
 // Thread per k over the rows of one row chunk (grid.y):

@@ -142,55 +142,63 @@ static int branch_input_any(const void* H, int dtype, const float* w, void* bi, 
   });
 }
 
-// branch_input with the Eq. 14-19 epilogue in front, for a call of few tiles (decode, short
-// prompts): the first wave of every workgroup forms its batch's weights from the projection
-// records, as dynw_finalize_kernel does (the same bits), while the tile's H loads are in flight;
-// the batch's first workgroup writes them (w, aux).  The launch that this saves costs as much as
-// the epilogue itself; with many tiles per batch the repeated epilogues would cost more.
-template <typename T, int W, int NT, bool RAG>
-__global__ __launch_bounds__(kThreads) void bi_finalize_kernel(const T* __restrict__ H, const float* __restrict__ part,
-                                                               int nK, int64_t K, DynParams P, float* __restrict__ w,
-                                                               float* __restrict__ aux, T* __restrict__ bi, Geom g,
-                                                               int iters, float eps) {
+// branch_input with the Eq. 14-19 epilogue in front: the first wave of every workgroup forms its
+// batch's weights from the projection records, as dynw_finalize_kernel does (the same bits), while
+// the first tile's H loads are in flight; the batch's first workgroup writes them (w, aux).  For a
+// call of few tiles (decode, short prompts; a workgroup per tile) and for short sequences in number
+// (a workgroup per batch, striding over its tiles): the launch that this saves costs as much as the
+// epilogue itself, and with many workgroups per batch the repeated epilogues would cost more.
+template <typename T, int W, int NT, bool RAG, int NTH>
+__global__ __launch_bounds__(NTH) void bi_finalize_kernel(const T* __restrict__ H, const float* __restrict__ part,
+                                                          int nK, int64_t K, DynParams P, float* __restrict__ w,
+                                                          float* __restrict__ aux, T* __restrict__ bi, Geom g,
+                                                          int iters, float eps) {
   __shared__ float quarter[4][kPart];
   __shared__ float pre[4];
   const int64_t b = g.b0 + blockIdx.y;
   const int64_t D = g.D;
-  const int64_t s_lo = (int64_t)(blockIdx.x * kThreads) / g.nch;
-  const int64_t t0 = b * g.S + s_lo;
-  const int64_t rest = g.S - s_lo;
-  const typename SpanOf<T, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
-  const typename SpanOf<T, W, RAG>::type bis(bi + t0 * D, rest * D);
-  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  const bool ok = i < g.items;
-  const uint32_t s = ok ? i / g.nch : (uint32_t)s_lo;
-  const RowCol<W, RAG> rc(ok ? i - s * g.nch : 0, (uint32_t)D);
-  const uint32_t e1 = (s - (uint32_t)s_lo) * (uint32_t)D + rc.col;
-  const uint32_t e4 = (s - (uint32_t)s_lo) * 4 * (uint32_t)D + rc.col;
   Frag<T, W> hf[4];
-  if (ok) {
+  float p[4];
+  for (uint32_t tile = blockIdx.x; tile < g.ntiles; tile += gridDim.x) {
+    const int64_t s_lo = (int64_t)(tile * NTH) / g.nch;
+    const int64_t t0 = b * g.S + s_lo;
+    const int64_t rest = g.S - s_lo;
+    const typename SpanOf<T, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
+    const typename SpanOf<T, W, RAG>::type bis(bi + t0 * D, rest * D);
+    const uint32_t i = tile * NTH + threadIdx.x;
+    const bool ok = i < g.items;
+    const uint32_t s = ok ? i / g.nch : (uint32_t)s_lo;
+    const RowCol<W, RAG> rc(ok ? i - s * g.nch : 0, (uint32_t)D);
+    const uint32_t e1 = (s - (uint32_t)s_lo) * (uint32_t)D + rc.col;
+    const uint32_t e4 = (s - (uint32_t)s_lo) * 4 * (uint32_t)D + rc.col;
+    if (ok) {
 #pragma unroll
-    for (int n = 0; n < 4; ++n) hf[n].template load<(NT & 1) != 0>(hs, e4 + n * (uint32_t)D);
+      for (int n = 0; n < 4; ++n) hf[n].template load<(NT & 1) != 0>(hs, e4 + n * (uint32_t)D);
+    }
+    loads_issued();
+    if (tile == blockIdx.x) {  // the first tile: every thread of the workgroup comes through here once
+      if (threadIdx.x < 64) sum_records(part + b * nK * kPart, nK, threadIdx.x, quarter);
+      __syncthreads();
+      if (threadIdx.x < 16) {
+        const int e = threadIdx.x;
+        const float raw_res = row_total(quarter, 8 + e), raw_pp = row_total(quarter, e & 7);
+        const Row16 o = weights_row16(e, raw_res, raw_pp, row_total(quarter, kOut), K, P, iters, eps);
+        if (e < 4) pre[e] = o.pp;
+        if (blockIdx.x == 0)
+          store_row16(e, b, o, raw_res, raw_pp, OutRow{w, kOut}, OutRow{w + 4, kOut}, OutRow{w + 8, kOut}, aux);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int n = 0; n < 4; ++n) p[n] = pre[n];
+    }
+    if (!ok) continue;
+    float h[4][W], r[W];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) hf[n].unpack(h[n]);
+#pragma unroll
+    for (int e = 0; e < W; ++e) r[e] = p[0] * h[0][e] + p[1] * h[1][e] + p[2] * h[2][e] + p[3] * h[3][e];
+    st_from<T, W, (NT & 2) != 0>(bis, e1, r, rc.skip);
   }
-  loads_issued();
-  if (threadIdx.x < 64) sum_records(part + b * nK * kPart, nK, threadIdx.x, quarter);
-  __syncthreads();
-  if (threadIdx.x < 16) {
-    const int e = threadIdx.x;
-    const float raw_res = row_total(quarter, 8 + e), raw_pp = row_total(quarter, e & 7);
-    const Row16 o = weights_row16(e, raw_res, raw_pp, row_total(quarter, kOut), K, P, iters, eps);
-    if (e < 4) pre[e] = o.pp;
-    if (blockIdx.x == 0)
-      store_row16(e, b, o, raw_res, raw_pp, OutRow{w, kOut}, OutRow{w + 4, kOut}, OutRow{w + 8, kOut}, aux);
-  }
-  __syncthreads();
-  if (!ok) return;
-  float h[4][W], r[W];
-#pragma unroll
-  for (int n = 0; n < 4; ++n) hf[n].unpack(h[n]);
-#pragma unroll
-  for (int e = 0; e < W; ++e) r[e] = pre[0] * h[0][e] + pre[1] * h[1][e] + pre[2] * h[2][e] + pre[3] * h[3][e];
-  st_from<T, W, (NT & 2) != 0>(bis, e1, r, rc.skip);
 }
 
 // The dynamic forward's last step: the epilogue of the projection records part[b][nK][25] (the
@@ -202,10 +210,20 @@ static int finalize_and_bi(const void* H, int dtype, const float* part, int nK, 
   const int rc = MHC_DISPATCH_DTYPE(dtype, [&] {
     return with_width<Vec<T>::N>(B, S, D, {H, bi}, [&](auto w_, auto rag_) {
       constexpr int W = decltype(w_)::value;
-      const Geom g = make_geom<W, kLU>(S, D, 0);
-      if (g.ntiles == 0 || B * (int64_t)g.ntiles > kFusedEpilogueTiles) return -1;
-      bi_finalize_kernel<T, W, kNtCached, decltype(rag_)::value><<<dim3(g.ntiles, (unsigned)B), kThreads, 0, st>>>(
-          (const T*)H, part, nK, K, P, w, aux, (T*)bi, g, iters, eps);
+      constexpr bool RAG = decltype(rag_)::value;
+      const Geom g1 = make_geom<W, kLU>(S, D, 0);
+      if (g1.ntiles > 0 && B * (int64_t)g1.ntiles <= kFusedEpilogueTiles)
+        bi_finalize_kernel<T, W, kNtCached, RAG, kThreads><<<dim3(g1.ntiles, (unsigned)B), kThreads, 0, st>>>(
+            (const T*)H, part, nK, K, P, w, aux, (T*)bi, g1, iters, eps);
+      else if (W > 1 && whole_batch(B, S, D, W))
+        return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
+          const Geom g = make_geom<W, kLU, kBatchThreads>(S, D, b0);
+          bi_finalize_kernel<T, W, kNtCached, RAG, kBatchThreads><<<dim3(1, (unsigned)nb), kBatchThreads, 0, st>>>(
+              (const T*)H, part, nK, K, P, w, aux, (T*)bi, g, iters, eps);
+          return hip_status(hipGetLastError(), "layer finalize and branch_input launch");
+        });
+      else
+        return -1;
       return hip_status(hipGetLastError(), "layer finalize and branch_input launch");
     });
   });
@@ -326,6 +344,94 @@ static int mix_bwd_dispatch(const void* dbi, const void* dhn, const void* H, con
                                                                part, B, S, D, nblk, st);
     return launch_mix_bwd<T, W, RAG, false, REDUCE, WRITE_DH>((const T*)dbi, nullptr, (const T*)H, w, (T*)dH, part, B,
                                                               S, D, nblk, st);
+  });
+}
+
+// Pass B and the weights backward's rows in one, a workgroup per batch (whole_batch): the sums of
+// dH_pre and dH_res over the batch stay in the workgroup, whose first 16 lanes then run the row.
+// Separately the rows' kernel is a launch of a few microseconds that reads a handful of partials
+// per batch.
+template <typename T, int W, bool RAG, bool HAS_DHN>
+__global__ __launch_bounds__(kBatchThreads) void pass_b_rows_kernel(const T* __restrict__ dbi,
+                                                                    const T* __restrict__ dhn,
+                                                                    const T* __restrict__ H,
+                                                                    const float* __restrict__ w,
+                                                                    const float* __restrict__ dpost,
+                                                                    const float* __restrict__ aux, DynParams P,
+                                                                    float* __restrict__ rowbuf, int64_t K, int iters,
+                                                                    float eps, Geom g) {
+  __shared__ float lds[kBatchThreads / 16 * 20];
+  __shared__ float tot[20];
+  __shared__ float slots[kSkSlots * 64];
+  const int64_t b = g.b0 + blockIdx.y;
+  const int64_t D = g.D;
+  float acc[20];
+#pragma unroll
+  for (int k = 0; k < 20; ++k) acc[k] = 0.f;
+  for (uint32_t tile = 0; tile < g.ntiles; ++tile) {
+    const int64_t s_lo = (int64_t)(tile * kBatchThreads) / g.nch;
+    const int64_t t0 = b * g.S + s_lo;
+    const int64_t rest = g.S - s_lo;
+    const typename SpanOf<T, W, RAG>::type dbs(dbi + t0 * D, rest * D);
+    const typename SpanOf<T, W, RAG>::type dns(dhn + t0 * 4 * D, rest * 4 * D);
+    const typename SpanOf<T, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
+    const uint32_t i = tile * kBatchThreads + threadIdx.x;
+    if (i >= g.items) break;
+    const uint32_t s = i / g.nch;
+    const RowCol<W, RAG> rc(i - s * g.nch, (uint32_t)D);
+    const uint32_t dt = s - (uint32_t)s_lo;
+    const uint32_t e4 = dt * 4 * (uint32_t)D + rc.col;
+    // nt on the H loads alone: d_bi and dH_new are read again by pass C
+    float db[W], dn[4][W], h[4][W];
+    ld<T, W, false>(dbs, dt * (uint32_t)D + rc.col, db);
+    if constexpr (HAS_DHN) {
+#pragma unroll
+      for (int n = 0; n < 4; ++n) ld<T, W, false>(dns, e4 + n * (uint32_t)D, dn[n]);
+    }
+#pragma unroll
+    for (int n = 0; n < 4; ++n) ld<T, W, true>(hs, e4 + n * (uint32_t)D, h[n]);
+#pragma unroll
+    for (int n = 0; n < 4; ++n) drop_skipped<W, RAG>(h[n], rc.skip);
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[n] += db[e] * h[n][e];
+      if constexpr (HAS_DHN) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+          for (int m = 0; m < 4; ++m) acc[4 + 4 * n + m] += dn[n][e] * h[m][e];
+      }
+    }
+  }
+  const float t = block_sum_rows<20, kBatchThreads>(acc, lds);
+  if (threadIdx.x < 20) tot[threadIdx.x] = t;
+  __syncthreads();
+  if (threadIdx.x >= 16) return;
+  const int e = threadIdx.x, j = e & 3;
+  weights_row16_bwd(e, aux + b * kPart, P, w[b * kOut + j], tot[j], dpost ? dpost[b * 4 + j] : 0.f, tot[4 + e],
+                    rowbuf + b * kRow, K, iters, eps, slots + e, true);
+}
+
+// Runs it where a batch is one workgroup's work; -1 where it is not.
+template <typename T>
+static int pass_b_rows(const void* dbi, const void* dhn, const void* H, const float* w, const float* dpost,
+                       const float* aux, const DynParams& P, float* rowbuf, int64_t B, int64_t S, int64_t D, int iters,
+                       float eps, hipStream_t st) {
+  return with_width<Vec<T>::N>(B, S, D, {dbi, dhn, H}, [&](auto w_, auto rag_) {
+    constexpr int W = decltype(w_)::value;
+    constexpr bool RAG = decltype(rag_)::value;
+    if constexpr (W > 1) {
+      if (whole_batch(B, S, D, W))
+        return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
+          const Geom g = make_geom<W, 1, kBatchThreads>(S, D, b0);
+          auto* k = dhn ? pass_b_rows_kernel<T, W, RAG, true> : pass_b_rows_kernel<T, W, RAG, false>;
+          k<<<dim3(1, (unsigned)nb), kBatchThreads, 0, st>>>((const T*)dbi, (const T*)dhn, (const T*)H, w, dpost, aux,
+                                                             P, rowbuf, 4 * D, iters, eps, g);
+          return hip_status(hipGetLastError(), "layer backward pass B launch");
+        });
+    }
+    return -1;
   });
 }
 
@@ -635,30 +741,34 @@ extern "C" int mhc_layer_dynamic_backward(const void* H, int dtype, const void* 
   float* part = (float*)(wsb + L.red_part);
   float* rowbuf = (float*)(wsb + L.rowbuf);
   float* gx = (float*)(wsb + L.gx);
-  // Pass B: dH_pre, dH_res.
-  uint32_t nblk = 0;
-  int rc = MHC_DISPATCH_DTYPE(dtype, [&] {
-    return mix_bwd_dispatch<T, true, false>(d_branch_input, dH_new, H, w, nullptr, part, B, S, D,
-                                                   &nblk, st);
-  });
-  if (rc) return rc;
-  // Weights backward: the rows kernel sums the pass-B partials itself; the wide
-  // kernel also sums grad_bias / grad_alpha.
   DynParams P{H_pre_base, H_post_base, H_res_base, alpha_pre, alpha_post, alpha_res};
   const int64_t K = 4 * D;
-  // A workgroup per batch sums up to thousands of partials (B = 1: 2048); with at most 64 per
-  // batch (from 32 batches on) one wave's lanes hold them all, so a workgroup takes four batches,
-  // a wave each, and adds the same four 16-lane row sums in the same order (B = 4096, S = 1:
-  // 16.0 us for one batch per workgroup, whose Sinkhorn backward then keeps 16 of 64 lanes busy).
-  if (nblk <= 64)
-    dynw_bwd_rows_kernel<4><<<dim3((unsigned)((B + 3) / 4)), kThreads, 0, st>>>(
-        aux, P, InRow{w, kOut}, InRow{nullptr, 0}, InRow{dH_post, 4}, InRow{nullptr, 0}, part, (int)nblk, rowbuf,
-        B, K, iters, eps);
-  else
-    dynw_bwd_rows_kernel<1><<<dim3((unsigned)B), kThreads, 0, st>>>(
-        aux, P, InRow{w, kOut}, InRow{nullptr, 0}, InRow{dH_post, 4}, InRow{nullptr, 0}, part, (int)nblk, rowbuf,
-        B, K, iters, eps);
-  if ((rc = hip_status(hipGetLastError(), "layer weights backward rows launch"))) return rc;
+  int rc = MHC_DISPATCH_DTYPE(dtype, [&] {
+    return pass_b_rows<T>(d_branch_input, dH_new, H, w, dH_post, aux, P, rowbuf, B, S, D, iters, eps, st);
+  });
+  if (rc > 0) return rc;
+  if (rc == -1) {
+    // Pass B: dH_pre, dH_res.
+    uint32_t nblk = 0;
+    rc = MHC_DISPATCH_DTYPE(dtype, [&] {
+      return mix_bwd_dispatch<T, true, false>(d_branch_input, dH_new, H, w, nullptr, part, B, S, D, &nblk, st);
+    });
+    if (rc) return rc;
+    // Weights backward: the rows kernel sums the pass-B partials itself; the wide
+    // kernel also sums grad_bias / grad_alpha.
+    // A workgroup per batch sums up to thousands of partials (B = 1: 2048); with at most 64 per
+    // batch (from 32 batches on) one wave's lanes hold them all, so a workgroup takes four batches,
+    // a wave each, and adds the same four 16-lane row sums in the same order.
+    if (nblk <= 64)
+      dynw_bwd_rows_kernel<4><<<dim3((unsigned)((B + 3) / 4)), kThreads, 0, st>>>(
+          aux, P, InRow{w, kOut}, InRow{nullptr, 0}, InRow{dH_post, 4}, InRow{nullptr, 0}, part, (int)nblk, rowbuf,
+          B, K, iters, eps);
+    else
+      dynw_bwd_rows_kernel<1><<<dim3((unsigned)B), kThreads, 0, st>>>(
+          aux, P, InRow{w, kOut}, InRow{nullptr, 0}, InRow{dH_post, 4}, InRow{nullptr, 0}, part, (int)nblk, rowbuf,
+          B, K, iters, eps);
+    if ((rc = hip_status(hipGetLastError(), "layer weights backward rows launch"))) return rc;
+  }
   // The pooled rows: x, or without it (S = 1) H's own rows, read in H's dtype; grad_x stays f32.
   const void* xr = x ? (const void*)x : H;
   const int xdt = x ? MHC_DTYPE_F32 : dtype;

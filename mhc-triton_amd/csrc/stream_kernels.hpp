@@ -59,14 +59,14 @@ struct Geom {
   int64_t b0;     // first batch of this launch
 };
 
-template <int W, int U>
+template <int W, int U, int NTH = kThreads>
 __host__ inline Geom make_geom(int64_t S, int64_t D, int64_t b0) {
   Geom g;
   g.S = S;
   g.D = D;
   g.nch = (uint32_t)((D + W - 1) / W);
   g.items = (uint32_t)(S * ((D + W - 1) / W));
-  g.ntiles = (g.items + kThreads * U - 1) / (kThreads * U);
+  g.ntiles = (g.items + NTH * U - 1) / (NTH * U);
   g.b0 = b0;
   return g;
 }
@@ -227,21 +227,22 @@ __global__ __launch_bounds__(kThreads) void add_residual_fwd_kernel(const T* __r
 //   d_bo[s,:] = sum_n post[n] dHn[s,n,:]              (written, dtype TB)
 //   part[k]   = sum dHn[s,k,:] * bo[s,:]   k < 4      (reduced -> dH_post)
 // ---------------------------------------------------------------------------
-template <typename T, typename TB, int W, int U, int NT = 0, bool RAG = false, bool ONE = false>
-__global__ __launch_bounds__(kThreads) void add_residual_bwd_kernel(const T* __restrict__ dhn,
+template <typename T, typename TB, int W, int U, int NT = 0, bool RAG = false, bool ONE = false, int NTH = kThreads>
+__global__ __launch_bounds__(NTH) void add_residual_bwd_kernel(const T* __restrict__ dhn,
                                                                     const TB* __restrict__ bo, WRow post,
                                                                     TB* __restrict__ dbo, float* __restrict__ part,
                                                                     Geom g) {
   // ONE: one workgroup per tile (grid.x == g.ntiles), the weights fetched behind the tile's loads;
-  // otherwise workgroups stride over the tiles.
-  __shared__ float lds[16 * 4];
+  // otherwise workgroups stride over the tiles.  With one workgroup per batch (grid.x == 1) part is
+  // dH_post itself.
+  __shared__ float lds[NTH / 16 * 4];
   const int64_t b = g.b0 + blockIdx.y;
   float wq[4];
   if constexpr (!ONE) load_w4(post, b, wq);
   const int64_t D = g.D;
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   for (uint32_t tile = blockIdx.x; tile < g.ntiles; tile += gridDim.x) {
-    const int64_t s_lo = (int64_t)(tile * (kThreads * U)) / g.nch;
+    const int64_t s_lo = (int64_t)(tile * (NTH * U)) / g.nch;
     const int64_t t0 = b * g.S + s_lo;
     const int64_t rest = g.S - s_lo;
     const typename SpanOf<T, W, RAG>::type hs(dhn + t0 * 4 * D, rest * 4 * D);
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(kThreads) void add_residual_bwd_kernel(const T* __r
     bool ok[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint32_t i = tile * (kThreads * U) + u * kThreads + threadIdx.x;
+      const uint32_t i = tile * (NTH * U) + u * NTH + threadIdx.x;
       ok[u] = i < g.items;
       const uint32_t s = ok[u] ? i / g.nch : (uint32_t)s_lo;
       const RowCol<W, RAG> rc(ok[u] ? i - s * g.nch : 0, (uint32_t)D);
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(kThreads) void add_residual_bwd_kernel(const T* __r
     }
     if constexpr (ONE) break;
   }
-  const float tot = block_sum_rows<4>(acc, lds);
+  const float tot = block_sum_rows<4, NTH>(acc, lds);
   if (threadIdx.x < 4) part[(b * gridDim.x + blockIdx.x) * 4 + threadIdx.x] = tot;
 }
 
@@ -674,6 +675,21 @@ inline int with_width(int64_t B, int64_t S, int64_t D, std::initializer_list<con
   if (vec_ok(D, WV, ptrs)) return fn(std::integral_constant<int, WV>{}, std::false_type{});
   if (rag_ok(B * S * D, D, WV)) return fn(std::integral_constant<int, WV>{}, std::true_type{});
   return fn(std::integral_constant<int, 1>{}, std::false_type{});
+}
+
+// Short sequences: one workgroup of kBatchThreads lanes takes a whole batch, so a reduction over it
+// needs no partials and no second kernel, and what follows per batch can run in the workgroup
+// itself.  It pays where a batch is a tile or two, and for up to eight where batches alone fill the
+// GPU.  Training steps as graphs, bf16, apart -> whole batches: B=1, S=1, D=4096 (one tile) 33.5 ->
+// 29.8 us, B=64 49.2 -> 44.9, B=8, S=4, D=2048 (two) 39.0 -> 37.5, B=512, S=8, D=2048 (four) 169.3
+// -> 161.4, B=512, S=16 (eight) 282.7 -> 275.3; but B=64, S=8, D=2048 (four) 55.6 -> 60.2, and with
+// many batches of one tile each workgroup's serial end costs more than the launches: B=1024 equal,
+// B=4096 381 -> 397.
+constexpr int kBatchThreads = 512;
+
+inline bool whole_batch(int64_t B, int64_t S, int64_t D, int W) {
+  const int64_t tiles = (S * ((D + W - 1) / W) + kBatchThreads - 1) / kBatchThreads;
+  return tiles >= 1 && B <= 1024 && (tiles <= 2 || (B >= 256 && tiles <= 8));
 }
 
 // Workgroups per batch for a reduction kernel: about kRedBlocks in total

@@ -59,6 +59,14 @@ static int add_res_fwd(const TH* hr, const TB* bo, const float* post, TH* out, i
 template <typename TH, typename TB, int W, bool RAG>
 static int add_res_bwd(const TH* dhn, const TB* bo, WRow post, TB* dbo, float* dpost, int64_t B, int64_t S,
                        int64_t D, float* part, hipStream_t st) {
+  if constexpr (W > 1)
+    if (whole_batch(B, S, D, W))
+      return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
+        const Geom g = make_geom<W, kU, kBatchThreads>(S, D, b0);
+        add_residual_bwd_kernel<TH, TB, W, kU, kNt, RAG, false, kBatchThreads>
+            <<<dim3(1, nb), kBatchThreads, 0, st>>>(dhn, bo, post, dbo, dpost, g);
+        return hip_status(hipGetLastError(), "add_residual_backward launch");
+      });
   // Vectors: one workgroup per tile at 4 per CU (the closure backward at
   // config-3 size: 134 -> 128 us against 512 looping workgroups per batch at
   // 2 per CU).  Single elements: a capped count of looping workgroups.

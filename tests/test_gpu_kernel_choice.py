@@ -152,3 +152,49 @@ def test_mean_pool_chunks(B, S, D, dtype):
     assert float((mean_pool(H).double() - want).abs().max()) <= 2.0 ** -16
     hc, H, bo, dHn, dbi = make_case(min(B, 3), S, D, dtype, phi_std=0.02)
     check_layer(hc, H, bo, dHn, dbi, *FWD[dtype], 1e-4)
+
+
+@pytest.mark.parametrize("B,S,D,dtype,iters", [
+    # a workgroup per batch: one partial tile, exactly one and two tiles, one vector past them (where
+    # few batches take the other kernels), rows in 32 bits, ragged rows
+    (1, 1, 8, torch.bfloat16, 20), (3, 1, 4096, torch.bfloat16, 20), (2, 2, 4096, torch.float16, 7),
+    (2, 1, 8200, torch.bfloat16, 20), (5, 3, 1368, torch.float32, 33), (300, 5, 1001, torch.bfloat16, 7),
+    # 256 batches and more: three tiles with a partial last one, eight, and one vector past eight
+    (256, 3, 3000, torch.bfloat16, 20), (257, 8, 4096, torch.bfloat16, 20), (256, 1, 32776, torch.bfloat16, 20),
+    # the most batches, and one more
+    (1024, 2, 64, torch.float16, 20), (1025, 2, 64, torch.float16, 20)])
+def test_whole_batch_workgroups(B, S, D, dtype, iters):
+    hc, H, bo, dHn, dbi = make_case(B, S, D, dtype, phi_std=0.02)
+    hc.sinkhorn_iters = iters
+    if B * S * D > 1 << 23:  # too slow for the oracle in full: the first batches of the same call
+        from oracle import mhc_oracle as O
+        from test_gpu_module import params_np, rel_err, run_gpu, to_np
+
+        bi, Hn, grads = run_gpu(hc, H, bo, dHn, dbi)
+        n = 2
+        p = params_np(hc)
+        obi, oHn, cache = O.layer_forward(p, to_np(H[:n]), to_np(bo[:n]), True, True, iters, hc.eps)
+        og = O.layer_backward(p, cache, to_np(dHn[:n]), to_np(dbi[:n]))
+        for got, want in ((bi[:n], obi), (Hn[:n], oHn), (grads["H"][:n], og["H"]), (grads["bo"][:n], og["bo"])):
+            assert rel_err(to_np(got), want) < 2e-2
+        return
+    check_layer(hc, H, bo, dHn, dbi, *FWD[dtype], 1e-4)
+
+
+@pytest.mark.parametrize("B,S,D", [(4, 2, 512), (256, 4, 2048)])
+def test_whole_batch_without_a_closure_gradient(B, S, D):
+    """No dH_new and no dH_post: the same gradients as with zeros for both."""
+    hc, H, bo, dHn, dbi = make_case(B, S, D, torch.bfloat16, phi_std=0.02)
+
+    def step(zeros):
+        hc.zero_grad(set_to_none=True)
+        Hl = H.clone().requires_grad_(True)
+        bi, add = hc(Hl)
+        if zeros:
+            torch.autograd.backward([add(bo), bi], [torch.zeros_like(dHn), dbi])
+        else:
+            bi.backward(dbi)
+        return [Hl.grad] + [p.grad for p in hc.parameters()]
+
+    for a, b in zip(step(False), step(True)):
+        assert torch.equal(a, b)
