@@ -63,27 +63,49 @@ __device__ __forceinline__ void sk_init(float (&m)[16], float eps) {
 // when carrying u and v themselves), with a normwise error against an fp64
 // evaluation of the explicit form of 1.7e-7 (2.2e-7 for the explicit fp32
 // update).  The backward keeps sk_round for its recomputed states.
+//
+// SMALL: with eps <= kSkSmallEps the eps terms are left out from the second round on, where they
+// are below half a unit in the last place.  From then on one round changes w by a factor of at most
+// 4: P_ij u_i v_j <= 1 after a normalisation bounds every term of the new (P0 v)_i by the old w_i, so
+// w_new <= 4 w_old, the same holds for z, and then z_new = sum P_ij / w_new >= z_old / 4 (up to
+// eps) and likewise for w.  eps w_old is thus at most 4 eps (P0 v)_i, 2^-24 of it.  The first round,
+// where w starts from 1 whatever the size of P0, keeps them (a matrix of zeros needs it to).  32 VALU
+// + 8 v_rcp (a quarter-rate instruction) per round instead of 40 + 8.
+constexpr float kSkSmallEps = 0x1p-26f;
+
+// One half round: s[k] <- sum of P0's row or column k scaled by the other side's vector, + eps s[k].
+template <bool SMALL>
+__device__ __forceinline__ float sk_carry(float eps, float old, float dot, bool first) {
+  return SMALL && !first ? dot : __builtin_fmaf(eps, old, dot);
+}
+
+template <bool SMALL>
+__device__ __forceinline__ void sk_forward_round(const float (&m)[16], float (&w)[4], float (&z)[4], float eps,
+                                                 bool first) {
+  float v[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = fast_rcp(z[j]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float dot = m[4 * i] * v[0] + m[4 * i + 1] * v[1] + m[4 * i + 2] * v[2] + m[4 * i + 3] * v[3];
+    w[i] = sk_carry<SMALL>(eps, w[i], dot, first);
+  }
+  float u[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) u[i] = fast_rcp(w[i]);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float dot = u[0] * m[j] + u[1] * m[4 + j] + u[2] * m[8 + j] + u[3] * m[12 + j];
+    z[j] = sk_carry<SMALL>(eps, z[j], dot, first);
+  }
+}
+
+template <bool SMALL>
 __device__ __forceinline__ void sk_forward(float (&m)[16], int iters, float eps) {
   sk_init(m, eps);
   float w[4] = {1.f, 1.f, 1.f, 1.f}, z[4] = {1.f, 1.f, 1.f, 1.f};
-  for (int t = 0; t < iters; ++t) {
-    float v[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = fast_rcp(z[j]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float dot = m[4 * i] * v[0] + m[4 * i + 1] * v[1] + m[4 * i + 2] * v[2] + m[4 * i + 3] * v[3];
-      w[i] = __builtin_fmaf(eps, w[i], dot);
-    }
-    float u[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) u[i] = fast_rcp(w[i]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float dot = u[0] * m[j] + u[1] * m[4 + j] + u[2] * m[8 + j] + u[3] * m[12 + j];
-      z[j] = __builtin_fmaf(eps, z[j], dot);
-    }
-  }
+  if (iters > 0) sk_forward_round<SMALL>(m, w, z, eps, true);
+  for (int t = 1; t < iters; ++t) sk_forward_round<SMALL>(m, w, z, eps, false);
   float u[4], v[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -190,7 +212,7 @@ __device__ __forceinline__ void sk_backward(const float (&mat)[16], float (&d)[1
 // (the explicit form of sk_round_backward on the scaled state took about
 // 128 + 8 v_rcp); the forward is 40 VALU + 8 v_rcp per round.  g starts as
 // dP_T * u_T v_T^T and ends as dP0 (u_0 = v_0 = 1).
-template <int TMAX>
+template <int TMAX, bool SMALL>
 __device__ __forceinline__ void sk_backward_scaled(const float (&mat)[16], float (&d)[16], int iters, float eps) {
   float p0[16];
   uint32_t neg = 0u, zero = 0u;  // sgn(M) as two bit masks, so that M need not stay live
@@ -212,14 +234,14 @@ __device__ __forceinline__ void sk_backward_scaled(const float (&mat)[16], float
         for (int i = 0; i < 4; ++i) {
           const float dot = p0[4 * i] * V[t][0] + p0[4 * i + 1] * V[t][1] + p0[4 * i + 2] * V[t][2] +
                             p0[4 * i + 3] * V[t][3];
-          w[i] = __builtin_fmaf(eps, w[i], dot);
+          w[i] = sk_carry<SMALL>(eps, w[i], dot, t == 0);
           U[t + 1][i] = fast_rcp(w[i]);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const float dot = U[t + 1][0] * p0[j] + U[t + 1][1] * p0[4 + j] + U[t + 1][2] * p0[8 + j] +
                             U[t + 1][3] * p0[12 + j];
-          z[j] = __builtin_fmaf(eps, z[j], dot);
+          z[j] = sk_carry<SMALL>(eps, z[j], dot, t == 0);
           V[t + 1][j] = fast_rcp(z[j]);
         }
       }
@@ -270,7 +292,7 @@ __device__ __forceinline__ void sk_backward_scaled(const float (&mat)[16], float
 // forward's) and runs sk_backward_scaled's round backward over them.  Every
 // round is recomputed once, against several times for the explicit-state
 // checkpoints of sk_backward.  Requires iters <= TSEG * NSEG.
-template <int TSEG, int NSEG>
+template <int TSEG, int NSEG, bool SMALL>
 __device__ __forceinline__ void sk_backward_segmented(const float (&mat)[16], float (&d)[16], int iters, float eps) {
   float p0[16];
   uint32_t neg = 0u, zero = 0u;
@@ -281,17 +303,17 @@ __device__ __forceinline__ void sk_backward_segmented(const float (&mat)[16], fl
     zero |= (mat[k] == 0.f ? 1u : 0u) << k;
   }
   // one round of the carried iteration: w from v, u = rcp(w), z from u, v = rcp(z)
-  auto sk_step = [&](float (&w)[4], float (&z)[4], const float (&v)[4], float (&u1)[4], float (&v1)[4]) {
+  auto sk_step = [&](float (&w)[4], float (&z)[4], const float (&v)[4], float (&u1)[4], float (&v1)[4], bool first) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float dot = p0[4 * i] * v[0] + p0[4 * i + 1] * v[1] + p0[4 * i + 2] * v[2] + p0[4 * i + 3] * v[3];
-      w[i] = __builtin_fmaf(eps, w[i], dot);
+      w[i] = sk_carry<SMALL>(eps, w[i], dot, first);
       u1[i] = fast_rcp(w[i]);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float dot = u1[0] * p0[j] + u1[1] * p0[4 + j] + u1[2] * p0[8 + j] + u1[3] * p0[12 + j];
-      z[j] = __builtin_fmaf(eps, z[j], dot);
+      z[j] = sk_carry<SMALL>(eps, z[j], dot, first);
       v1[j] = fast_rcp(z[j]);
     }
   };
@@ -308,7 +330,7 @@ __device__ __forceinline__ void sk_backward_segmented(const float (&mat)[16], fl
       const int tend = iters < (k + 1) * TSEG ? iters : (k + 1) * TSEG;
       for (int t = k * TSEG; t < tend; ++t) {
         float u1[4], v1[4];
-        sk_step(w, z, v, u1, v1);
+        sk_step(w, z, v, u1, v1, t == 0);
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = v1[q];
       }
@@ -342,7 +364,7 @@ __device__ __forceinline__ void sk_backward_segmented(const float (&mat)[16], fl
     }
 #pragma unroll
     for (int tt = 0; tt < TSEG; ++tt)
-      if (t0 + tt < iters) sk_step(w, z, V[tt], U[tt + 1], V[tt + 1]);
+      if (t0 + tt < iters) sk_step(w, z, V[tt], U[tt + 1], V[tt + 1], t0 + tt == 0);
 #pragma unroll
     for (int tt = TSEG - 1; tt >= 0; --tt) {
       if (t0 + tt < iters) {

@@ -198,3 +198,27 @@ def test_whole_batch_without_a_closure_gradient(B, S, D):
 
     for a, b in zip(step(False), step(True)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n", [1, 64, 257])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("eps", [0.0, 2.0 ** -26, 2.0 ** -25])
+@pytest.mark.parametrize("iters", [0, 2, 33])
+def test_sinkhorn_forms(n, dtype, eps, iters):
+    """Partial waves, and eps on both sides of the line up to which its terms are left out after the
+    first round (below half a unit there): entries over twelve decades, zeros among them where eps
+    keeps the sums positive.  One v_rcp and one rounding per normalised entry: 4e-7 of the largest."""
+    import mhc
+    from helpers import rel_err, to_np
+    from oracle import mhc_oracle as O
+
+    g = torch.Generator(device=DEV).manual_seed(n + iters)
+    M = torch.randn((n, 4, 4), generator=g, device=DEV)
+    M = (M * 10 ** (torch.rand((n, 1, 1), generator=g, device=DEV) * 8 - 4)).to(dtype)
+    if eps:
+        M[0, 1] = 0
+        M[n // 2, :, 2] = 0
+    P = mhc.sinkhorn_knopp(M, iters, eps)
+    want = O.sinkhorn(to_np(M), iters, eps)
+    half = {torch.float32: 0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert rel_err(to_np(P), want) < 1e-6 + half
