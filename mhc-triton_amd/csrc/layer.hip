@@ -53,11 +53,13 @@ constexpr int64_t kLayerBulkRows = 64;
 constexpr int64_t kLayerBulkProjRowsS1 = 64;
 constexpr int64_t kLayerBulkProjElems = (int64_t)1 << 19;  // B * D
 
-// Workgroups of branch_input up to which the epilogue runs in front of it (bi_finalize_kernel).
-// No-grad forwards as graphs, epilogue apart -> in front: B = 128, S = 1, D = 4096 (256 workgroups)
-// 21.5 -> 18.6 us, B = 256 24.5 -> 22.0, B = 512 29.3 -> 27.0, B = 1, S = 512 (1024) 29.1 -> 27.7;
-// at 2048 workgroups equal (38.5, 39.0), at 4096 equal or slower (69.9 -> 70.3).
-constexpr int64_t kFusedEpilogueTiles = 1024;
+// Workgroups of branch_input up to which the epilogue runs in front of it (bi_finalize_kernel), with
+// one item per lane or, up to twice the tiles, two.  No-grad forwards as graphs, epilogue apart -> in
+// front: B = 128, S = 1, D = 4096 (256 workgroups) 21.5 -> 18.6 us, B = 512 29.3 -> 27.0, B = 1,
+// S = 600 (1200) 28.2 -> 26.8; two items B = 4, S = 512, D = 2048 (1024 of 2048 tiles) 38.3 -> 37.1,
+// its training step 87.0 -> 85.7.  Workgroups of one item at 2048 gain nothing (39.2), and four items
+// at 4000 tiles lose what they save (58.8 -> 59.7).
+constexpr int64_t kFusedEpilogueTiles = 1536;
 
 constexpr int kLU = 1;   // items per lane per tile, streaming passes
 constexpr int kLRU = 2;  // items per lane per tile, the reduction-only pass B
@@ -148,7 +150,7 @@ static int branch_input_any(const void* H, int dtype, const float* w, void* bi, 
 // call of few tiles (decode, short prompts; a workgroup per tile) and for short sequences in number
 // (a workgroup per batch, striding over its tiles): the launch that this saves costs as much as the
 // epilogue itself, and with many workgroups per batch the repeated epilogues would cost more.
-template <typename T, int W, int NT, bool RAG, int NTH>
+template <typename T, int W, int NT, bool RAG, int NTH, int U>
 __global__ __launch_bounds__(NTH) void bi_finalize_kernel(const T* __restrict__ H, const float* __restrict__ part,
                                                           int nK, int64_t K, DynParams P, float* __restrict__ w,
                                                           float* __restrict__ aux, T* __restrict__ bi, Geom g,
@@ -157,23 +159,29 @@ __global__ __launch_bounds__(NTH) void bi_finalize_kernel(const T* __restrict__ 
   __shared__ float pre[4];
   const int64_t b = g.b0 + blockIdx.y;
   const int64_t D = g.D;
-  Frag<T, W> hf[4];
+  Frag<T, W> hf[U][4];
   float p[4];
   for (uint32_t tile = blockIdx.x; tile < g.ntiles; tile += gridDim.x) {
-    const int64_t s_lo = (int64_t)(tile * NTH) / g.nch;
+    const int64_t s_lo = (int64_t)(tile * (NTH * U)) / g.nch;
     const int64_t t0 = b * g.S + s_lo;
     const int64_t rest = g.S - s_lo;
     const typename SpanOf<T, W, RAG>::type hs(H + t0 * 4 * D, rest * 4 * D);
     const typename SpanOf<T, W, RAG>::type bis(bi + t0 * D, rest * D);
-    const uint32_t i = tile * NTH + threadIdx.x;
-    const bool ok = i < g.items;
-    const uint32_t s = ok ? i / g.nch : (uint32_t)s_lo;
-    const RowCol<W, RAG> rc(ok ? i - s * g.nch : 0, (uint32_t)D);
-    const uint32_t e1 = (s - (uint32_t)s_lo) * (uint32_t)D + rc.col;
-    const uint32_t e4 = (s - (uint32_t)s_lo) * 4 * (uint32_t)D + rc.col;
-    if (ok) {
+    uint32_t e1[U], skip[U];
+    bool ok[U];
 #pragma unroll
-      for (int n = 0; n < 4; ++n) hf[n].template load<(NT & 1) != 0>(hs, e4 + n * (uint32_t)D);
+    for (int u = 0; u < U; ++u) {
+      const uint32_t i = tile * (NTH * U) + u * NTH + threadIdx.x;
+      ok[u] = i < g.items;
+      const uint32_t s = ok[u] ? i / g.nch : (uint32_t)s_lo;
+      const RowCol<W, RAG> rc(ok[u] ? i - s * g.nch : 0, (uint32_t)D);
+      e1[u] = (s - (uint32_t)s_lo) * (uint32_t)D + rc.col;
+      skip[u] = rc.skip;
+      const uint32_t e4 = (s - (uint32_t)s_lo) * 4 * (uint32_t)D + rc.col;
+      if (ok[u]) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) hf[u][n].template load<(NT & 1) != 0>(hs, e4 + n * (uint32_t)D);
+      }
     }
     loads_issued();
     if (tile == blockIdx.x) {  // the first tile: every thread of the workgroup comes through here once
@@ -191,13 +199,16 @@ __global__ __launch_bounds__(NTH) void bi_finalize_kernel(const T* __restrict__ 
 #pragma unroll
       for (int n = 0; n < 4; ++n) p[n] = pre[n];
     }
-    if (!ok) continue;
-    float h[4][W], r[W];
 #pragma unroll
-    for (int n = 0; n < 4; ++n) hf[n].unpack(h[n]);
+    for (int u = 0; u < U; ++u) {
+      if (!ok[u]) continue;
+      float h[4][W], r[W];
 #pragma unroll
-    for (int e = 0; e < W; ++e) r[e] = p[0] * h[0][e] + p[1] * h[1][e] + p[2] * h[2][e] + p[3] * h[3][e];
-    st_from<T, W, (NT & 2) != 0>(bis, e1, r, rc.skip);
+      for (int n = 0; n < 4; ++n) hf[u][n].unpack(h[n]);
+#pragma unroll
+      for (int e = 0; e < W; ++e) r[e] = p[0] * h[0][e] + p[1] * h[1][e] + p[2] * h[2][e] + p[3] * h[3][e];
+      st_from<T, W, (NT & 2) != 0>(bis, e1[u], r, skip[u]);
+    }
   }
 }
 
@@ -211,20 +222,25 @@ static int finalize_and_bi(const void* H, int dtype, const float* part, int nK, 
     return with_width<Vec<T>::N>(B, S, D, {H, bi}, [&](auto w_, auto rag_) {
       constexpr int W = decltype(w_)::value;
       constexpr bool RAG = decltype(rag_)::value;
-      const Geom g1 = make_geom<W, kLU>(S, D, 0);
-      if (g1.ntiles > 0 && B * (int64_t)g1.ntiles <= kFusedEpilogueTiles)
-        bi_finalize_kernel<T, W, kNtCached, RAG, kThreads><<<dim3(g1.ntiles, (unsigned)B), kThreads, 0, st>>>(
-            (const T*)H, part, nK, K, P, w, aux, (T*)bi, g1, iters, eps);
-      else if (W > 1 && whole_batch(B, S, D, W))
+      // one workgroup per tile of one or two items per lane
+      auto tiles = [&](auto u_) {
+        constexpr int U = W > 1 ? decltype(u_)::value : 1;
+        const Geom g = make_geom<W, U>(S, D, 0);
+        if (g.ntiles == 0 || B * (int64_t)g.ntiles > kFusedEpilogueTiles) return -1;
+        bi_finalize_kernel<T, W, kNtCached, RAG, kThreads, U><<<dim3(g.ntiles, (unsigned)B), kThreads, 0, st>>>(
+            (const T*)H, part, nK, K, P, w, aux, (T*)bi, g, iters, eps);
+        return hip_status(hipGetLastError(), "layer finalize and branch_input launch");
+      };
+      int r = tiles(std::integral_constant<int, 1>{});
+      if (r == -1 && W > 1) r = tiles(std::integral_constant<int, 2>{});
+      if (r == -1 && W > 1 && whole_batch(B, S, D, W))
         return for_batch_chunks(B, [&](int64_t b0, int64_t nb) {
-          const Geom g = make_geom<W, kLU, kBatchThreads>(S, D, b0);
-          bi_finalize_kernel<T, W, kNtCached, RAG, kBatchThreads><<<dim3(1, (unsigned)nb), kBatchThreads, 0, st>>>(
+          const Geom g = make_geom<W, 1, kBatchThreads>(S, D, b0);
+          bi_finalize_kernel<T, W, kNtCached, RAG, kBatchThreads, 1><<<dim3(1, (unsigned)nb), kBatchThreads, 0, st>>>(
               (const T*)H, part, nK, K, P, w, aux, (T*)bi, g, iters, eps);
           return hip_status(hipGetLastError(), "layer finalize and branch_input launch");
         });
-      else
-        return -1;
-      return hip_status(hipGetLastError(), "layer finalize and branch_input launch");
+      return r;
     });
   });
   if (rc != -1) return rc;

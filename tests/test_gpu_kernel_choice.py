@@ -15,8 +15,10 @@ FWD = {torch.float32: (1e-5, 1e-4), torch.bfloat16: (2e-2, 2e-2), torch.float16:
     # the epilogue in front of branch_input: one partial tile, a tile that spans tokens, whole tiles
     # with a partial last one, several batches
     (1, 1, 8, torch.bfloat16), (3, 5, 72, torch.float16), (2, 7, 20, torch.float32), (2, 3, 2056, torch.bfloat16),
-    # 1024 workgroups (the most that take it) and 1028
-    (4, 512, 1024, torch.bfloat16), (4, 513, 1024, torch.bfloat16)])
+    # 1536 workgroups of one item per lane, the first of two items with a partial last one (772), and
+    # 1536 of two items against the kernels apart
+    (4, 768, 1024, torch.bfloat16), (4, 769, 1024, torch.bfloat16), (2, 3072, 1024, torch.float16),
+    (2, 3073, 1024, torch.float16), (3, 131, 1003, torch.float32)])
 def test_epilogue_in_front_of_branch_input(B, S, D, dtype):
     hc, H, bo, dHn, dbi = make_case(B, S, D, dtype, phi_std=0.02)
     check_layer(hc, H, bo, dHn, dbi, *FWD[dtype], 1e-4)
