@@ -206,8 +206,19 @@ static WidePlan wide_plan(int64_t R, int64_t K) {
 // Never more chunks than the wide plan w (whose workspace holds the partials);
 // chunks are split further while a chunk's buffer spans (esize-byte x or grad_x
 // elements) would pass 2^31 bytes.
+//
+// With fewer rows there is little to stream per workgroup, and what counts is the latency of its
+// one or two blocks: narrower workgroups (bwd_waves) share a CU and take longer chunks, which also
+// leaves fewer grad_phi partials, down to one chunk and no reduce after it.  Eight waves -> two, or
+// four past 512 rows, the call's fwd+bwd as a graph: R = 256, K = 4096 bf16 30.5 -> 26.4 us, the layer
+// at B = 64, S = 1, D = 4096 45.0 -> 41.0, B = 256 60.4 -> 55.9, B = 512, S = 8, D = 2048 162.0 ->
+// 158.9; R = 1000, K = 8192 fp32 46.9 -> 46.3, R = 4096, K = 8192 bf16 69.1 -> 67.6.  Two waves at
+// R = 4096 took 80.0, four at R = K = 16384 337.8 against 309.
+static int bwd_waves(int64_t R) { return R <= 512 ? 2 : R <= 4096 ? 4 : kBwdWaves; }
+
 static WidePlan mfma_bwd_plan(int64_t R, int64_t K, const WidePlan& w, int esize) {
-  const int64_t ncb = (K + 32 * kBwdWaves - 1) / (32 * kBwdWaves);
+  const int64_t cols = 32 * bwd_waves(R);
+  const int64_t ncb = (K + cols - 1) / cols;
   int64_t nr = (kMfmaTargetWg + ncb - 1) / ncb;
   if (nr > w.nR) nr = w.nR;
   for (;;) {
@@ -254,23 +265,24 @@ int dynw_grad_pass(const void* x, int dtype_x, const float* phi, const float* ro
     // rows in bulk: grad_x and grad_phi on MFMA.
     if (pl.nR > 1 && (grad_bias || grad_alpha))
       bias_part = (float*)(split_ws + align256((size_t)w.nR * K * kOut * sizeof(float)));
-    const dim3 grid((unsigned)((K + 32 * kBwdWaves - 1) / (32 * kBwdWaves)), (unsigned)pl.nR);
-    // Chunks of one 64-row block load it alone: with 16-bit x and grad_x, loads of the next
-    // block (out of range) in flight as well cost 1.3-2.2 us at R = 64-256, K = 16384; from two
-    // blocks on the two ahead time alike, from six (R = 1536) they win by 1.6-2.6 us.
+    const int nw = bwd_waves(R);
+    const dim3 grid((unsigned)((K + 32 * nw - 1) / (32 * nw)), (unsigned)pl.nR);
     rc = MHC_DISPATCH_DTYPE(dtype_x, [&] {
-      if (gx_f32)
-        dynw_bwd_mfma_kernel<T, float><<<grid, 64 * kBwdWaves, 0, st>>>(
-            (const T*)x, phi, rowbuf, (float*)grad_x, grad_phi, gphi_part, bias_part, grad_bias, grad_alpha, R, K,
-            pl.RC);
-      else if (pl.RC <= kBwdRows)
-        dynw_bwd_mfma_kernel<T, T, 1><<<grid, 64 * kBwdWaves, 0, st>>>(
-            (const T*)x, phi, rowbuf, (T*)grad_x, grad_phi, gphi_part, bias_part, grad_bias, grad_alpha, R, K,
-            pl.RC);
-      else
-        dynw_bwd_mfma_kernel<T><<<grid, 64 * kBwdWaves, 0, st>>>((const T*)x, phi, rowbuf, (T*)grad_x, grad_phi,
-                                                                 gphi_part, bias_part, grad_bias, grad_alpha, R,
-                                                                 K, pl.RC);
+      auto go = [&](auto* kernel, auto* gx) {
+        kernel<<<grid, 64 * nw, 0, st>>>((const T*)x, phi, rowbuf, gx, grad_phi, gphi_part, bias_part, grad_bias,
+                                         grad_alpha, R, K, pl.RC);
+      };
+      // grad_x in x's type or in f32; blocks of loads in flight as the kernel's default has it for long
+      // chunks, one for narrow workgroups (their chunks are short: loads of a next block, out of
+      // range, cost 1.3-2.2 us at R = 64-256, K = 16384)
+      auto pick = [&](auto* gx) {
+        using TG = std::remove_pointer_t<decltype(gx)>;
+        if (nw == 2) go(dynw_bwd_mfma_kernel<T, TG, 1, 2>, gx);
+        else if (nw == 4) go(dynw_bwd_mfma_kernel<T, TG, 1, 4>, gx);
+        else go(dynw_bwd_mfma_kernel<T, TG>, gx);
+      };
+      if (gx_f32) pick((float*)grad_x);
+      else pick((T*)grad_x);
       return hip_status(hipGetLastError(), "dynamic_weights_backward mfma launch");
     });
   } else {

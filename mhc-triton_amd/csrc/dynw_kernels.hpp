@@ -899,7 +899,7 @@ __global__ __launch_bounds__(64 * NW, MINW) void dynw_bwd_mfma_kernel(const TX* 
   // Blocks of loads in flight (AH): by default one for fp32 x, whose blocks are twice the bytes in
   // the same registers, and for an f32 grad_x from 16-bit x (layer backward at S = 1, D = 4096:
   // 32.2 -> 30.0 us at 64 rows, the same at 1024 and 4096 rows), else kBwdAhead; the launcher
-  // takes one for chunks of a single block.
+  // takes one for its narrow workgroups.
   constexpr int A = AH;
   static_assert(A >= 1 && A <= kBwdAhead, "blocks ahead");
   // The x and grad_x tiles hold TX and TG values (fp32: 2 x 66.5 KiB of LDS); the G planes are bf16.

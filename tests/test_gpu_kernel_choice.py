@@ -224,3 +224,12 @@ def test_sinkhorn_forms(n, dtype, eps, iters):
     want = O.sinkhorn(to_np(M), iters, eps)
     half = {torch.float32: 0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
     assert rel_err(to_np(P), want) < 1e-6 + half
+
+
+@pytest.mark.parametrize("R,K", [
+    # two-wave column blocks (64 columns): one row chunk, several, a partial last block and column
+    # block; four-wave ones from 513 rows; eight from 4097
+    (64, 16384), (130, 4096), (512, 1000), (513, 1000), (1025, 8192), (4096, 1160), (4097, 264)])
+@pytest.mark.parametrize("xdtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_weights_backward_column_blocks(R, K, xdtype):
+    check_dynamic_weights(R, K, xdtype)
