@@ -804,6 +804,89 @@ inline hipError_t launch_dynw_bwd_wide(const TX* x, const float* phi, const floa
   return hipGetLastError();
 }
 
+// The rows and the wide pass in one launch, for the layer's few batches with few partials each:
+// every one-wave workgroup sums the rows' partials and runs their row backward itself, a 16-lane group
+// per row, into LDS.  The rows' own kernel is a launch of 5 us for the same chain, with the GPU idle
+// around it.  Workgroup K / 64 (the last) sums the records into grad_bias and grad_alpha.  Training
+// steps as graphs, apart -> in one: fp32 B=2, S=128, D=512 (32 partials per row) 40.5 -> 38.5 us, bf16
+// B=4, S=256, D=1024 (64) 48.3 -> 45.7, B=4, S=256, D=2048 (128) 57.5 -> 55.5, B=4, S=512, D=2048
+// (256) equal at 85.4 but a launch less for the host; B=1, S=512, D=4096 (512) 58.5 -> 60.6.
+constexpr int kFusedRows = 4;
+constexpr int kFusedPartials = 256;  // partials per row
+
+template <typename TX>
+__global__ __launch_bounds__(kWideThreads) void dynw_bwd_rows_wide_kernel(
+    const TX* __restrict__ x, const float* __restrict__ phi, const float* __restrict__ aux, DynParams P,
+    const float* __restrict__ w, const float* __restrict__ dpost, const float* __restrict__ part20, int nblk,
+    float* __restrict__ gx, float* __restrict__ gphi, float* __restrict__ gbias, float* __restrict__ galpha, int R,
+    int64_t K, int iters, float eps, bool phi_vec) {
+  __shared__ __attribute__((aligned(16))) float tot[kFusedRows][20];
+  __shared__ float rec[kFusedRows][kRow];
+  __shared__ float slots[kSkSlots * 64];
+  const int lane = threadIdx.x, e = lane & 15, grp = lane >> 4;
+  const int64_t k = (int64_t)blockIdx.x * kWideThreads + lane;
+  const bool bias_wg = blockIdx.x == gridDim.x - 1;
+  const bool live_k = !bias_wg && k < K;
+  // this column's phi and x first, in flight behind the rows
+  float ph[kOut], xv[kFusedRows];
+#pragma unroll
+  for (int j = 0; j < kOut; ++j) ph[j] = 0.f;
+  if (live_k) load_phi_row(phi, k, phi_vec, ph);
+#pragma unroll
+  for (int q = 0; q < kFusedRows; ++q) xv[q] = live_k && q < R ? to_f32(x[q * K + k]) : 0.f;
+  const int r = grp < R ? grp : R - 1;  // idle groups redo the last row and store nothing
+  f32x4 acc[5];
+#pragma unroll
+  for (int q = 0; q < 5; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int n = e; n < nblk; n += 16) {
+    const f32x4* p = reinterpret_cast<const f32x4*>(part20 + ((int64_t)r * nblk + n) * 20);
+#pragma unroll
+    for (int q = 0; q < 5; ++q) acc[q] += p[q];
+  }
+#pragma unroll
+  for (int q = 0; q < 5; ++q) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float v = sum_all16(acc[q][c]);
+      if (e == 0) tot[grp][4 * q + c] = v;
+    }
+  }
+  __syncthreads();
+  const int j4 = e & 3;
+  weights_row16_bwd(e, aux + r * kPart, P, w[r * kOut + j4], tot[grp][j4], dpost ? dpost[r * 4 + j4] : 0.f,
+                    tot[grp][4 + e], rec[grp], K, iters, eps, slots + lane, true);
+  __syncthreads();
+  if (bias_wg) {
+    if (lane < 27) {
+      float t = 0.f;
+      for (int q = 0; q < R; ++q) t += rec[q][25 + lane];
+      if (lane < kOut) { if (gbias) gbias[lane] = t; }
+      else if (galpha) galpha[lane - kOut] = t;
+    }
+    return;
+  }
+  if (!live_k) return;
+  float gp[kOut];
+#pragma unroll
+  for (int j = 0; j < kOut; ++j) gp[j] = 0.f;
+#pragma unroll
+  for (int q = 0; q < kFusedRows; ++q) {
+    if (q >= R) break;
+    float v = rec[q][24] * xv[q];
+#pragma unroll
+    for (int j = 0; j < kOut; ++j) {
+      v += rec[q][j] * ph[j];
+      gp[j] += xv[q] * rec[q][j];
+    }
+    if (gx) gx[q * K + k] = v;
+  }
+  if (gphi) {
+#pragma unroll
+    for (int j = 0; j < kOut; ++j) gphi[k * kOut + j] = gp[j];
+  }
+}
+
 // The wide pass for many rows (the standalone op at R = tokens), both products
 // on MFMA (v_mfma_f32_32x32x16_bf16; fragment layout above; fp16 x is split
 // exactly into bf16 hi + lo for grad_phi, fp32 x into hi + mid):

@@ -775,6 +775,18 @@ extern "C" int mhc_layer_dynamic_backward(const void* H, int dtype, const void* 
     // A workgroup per batch sums up to thousands of partials (B = 1: 2048); with at most 64 per
     // batch (from 32 batches on) one wave's lanes hold them all, so a workgroup takes four batches,
     // a wave each, and adds the same four 16-lane row sums in the same order.
+    if (B <= kFusedRows && nblk <= kFusedPartials && K > 0) {
+      const void* xf = x ? (const void*)x : H;
+      rc = MHC_DISPATCH_DTYPE(x ? MHC_DTYPE_F32 : dtype, [&] {
+        dynw_bwd_rows_wide_kernel<T>
+            <<<dim3((unsigned)((K + kWideThreads - 1) / kWideThreads) + 1u), kWideThreads, 0, st>>>(
+                (const T*)xf, phi, aux, P, w, dH_post, part, (int)nblk, dH ? gx : nullptr, grad_phi, grad_bias,
+                grad_alpha, (int)B, K, iters, eps, aligned16(phi));
+        return hip_status(hipGetLastError(), "layer weights backward launch");
+      });
+      if (rc || !dH || S * D == 0) return rc;
+      return MHC_DISPATCH_DTYPE(dtype, [&] { return dh_dispatch<T>(d_branch_input, dH_new, gx, w, dH, B, S, D, st); });
+    }
     if (nblk <= 64)
       dynw_bwd_rows_kernel<4><<<dim3((unsigned)((B + 3) / 4)), kThreads, 0, st>>>(
           aux, P, InRow{w, kOut}, InRow{nullptr, 0}, InRow{dH_post, 4}, InRow{nullptr, 0}, part, (int)nblk, rowbuf,

@@ -233,3 +233,26 @@ def test_sinkhorn_forms(n, dtype, eps, iters):
 @pytest.mark.parametrize("xdtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_weights_backward_column_blocks(R, K, xdtype):
     check_dynamic_weights(R, K, xdtype)
+
+
+@pytest.mark.parametrize("B,S,D,dtype,iters", [
+    # rows and wide pass in one: up to four rows, with three partials each (one past a whole batch's
+    # two tiles), sixteen and seventeen, 256 and (apart again) 257 and five rows; K not a whole wave
+    (1, 3, 4096, torch.bfloat16, 20), (4, 16, 4096, torch.float16, 20), (3, 17, 2050, torch.float32, 7),
+    (2, 256, 4096, torch.bfloat16, 33), (2, 257, 4096, torch.bfloat16, 20), (5, 17, 2048, torch.float32, 20),
+    (4, 130, 37, torch.bfloat16, 20)])
+@pytest.mark.parametrize("frozen_h", [False, True])
+def test_rows_in_the_wide_pass(B, S, D, dtype, iters, frozen_h):
+    hc, H, bo, dHn, dbi = make_case(B, S, D, dtype, phi_std=0.02)
+    hc.sinkhorn_iters = iters
+    if not frozen_h:
+        check_layer(hc, H, bo, dHn, dbi, *FWD[dtype], 1e-4)
+        return
+    grads = []
+    for needs in (True, False):  # without dH the parameter gradients are the same bits
+        hc.zero_grad(set_to_none=True)
+        bi, add = hc(H.clone().requires_grad_(needs))
+        torch.autograd.backward([add(bo), bi], [dHn, dbi])
+        grads.append([p.grad for p in hc.parameters()])
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
