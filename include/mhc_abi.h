@@ -215,7 +215,7 @@ int mhc_layer_dynamic_forward(const void* H, int dtype, const float* phi,
  * partials and the projection partials) is a static device array of
  * MHC_NOALLOC_SCRATCH_BYTES; the call allocates nothing.  It returns
  * MHC_ERR_WORKSPACE, before any device work, when the shape needs more:
- * about 17.6 * B * D bytes once that exceeds 3 MiB (6 MiB for fp32 H), so
+ * about 17.6 * B * D bytes once that exceeds about 1 MiB, so
  * B * D up to about 950k fits (B = 232 at D = 4096, any S).  The scratch
  * starts from nothing it has to find zeroed: each call overwrites every entry
  * it reads.  All calls on one GPU share that GPU's array, so calls that overlap
