@@ -230,7 +230,7 @@ template <typename T, int W> struct SpanOf<T, W, true> { using type = RagSpan<T>
 
 // The ragged path covers a row of n elements with ceil(n / W) lanes.  The last lane's vector is
 // moved back to end with the row, so its first `skip` elements are also its neighbour's: it computes
-// them too and leaves them out of what it stores and sums.
+// them too and leaves them out of what it stores and sums.  n is the whole row's (at least W).
 template <int W, bool RAG>
 struct RowCol {
   uint32_t col, skip;

@@ -1348,8 +1348,10 @@ __global__ __launch_bounds__(kThreads) void colsum_kernel(const T* __restrict__ 
   const int rg = __builtin_amdgcn_readfirstlane(threadIdx.x / LW);
   const int64_t cblk = (int64_t)blockIdx.x * (LW * W);
   const bool live = cblk + (int64_t)lane * W < K;
-  const RowCol<W, RAG> rc(live ? lane : 0, (uint32_t)(K - cblk < LW * W ? K - cblk : LW * W));
-  const int64_t col = cblk + rc.col;
+  // Ragged columns count from the row's start: the last block of a row may hold less than one vector.
+  const int64_t base_col = RAG ? 0 : cblk;
+  const RowCol<W, RAG> rc(RAG ? (live ? blockIdx.x * LW + lane : 0) : lane, (uint32_t)K);
+  const int64_t col = base_col + rc.col;
   // the chunk's rows in RG consecutive runs, one per row group
   const int64_t sbeg0 = (int64_t)sc * SC;
   const int64_t send0 = sbeg0 + SC < S ? sbeg0 + SC : S;
@@ -1361,7 +1363,7 @@ __global__ __launch_bounds__(kThreads) void colsum_kernel(const T* __restrict__ 
 #pragma unroll
   for (int e = 0; e < W; ++e) acc[e] = 0.f;
   if (live) {
-    const T* base = H + b * S * K + cblk;
+    const T* base = H + b * S * K + base_col;
     const uint32_t lane_e = rc.col;
     int64_t s = sbeg;
     colsum_rows<true, T, W, UN, RAG>(base, K, lane_e, s, smid, acc);
@@ -1485,8 +1487,8 @@ __global__ __launch_bounds__(kThreads) void colsum_direct_vec_kernel(const T* __
   const int64_t b = b0 + blockIdx.y;
   const int64_t cblk = (int64_t)blockIdx.x * (kThreads * W);
   if (cblk + (int64_t)threadIdx.x * W >= K) return;
-  const RowCol<W, RAG> rc(threadIdx.x, (uint32_t)(K - cblk < kThreads * W ? K - cblk : kThreads * W));
-  const int64_t c = cblk + rc.col;
+  const RowCol<W, RAG> rc(RAG ? blockIdx.x * kThreads + threadIdx.x : threadIdx.x, (uint32_t)K);
+  const int64_t c = (RAG ? 0 : cblk) + rc.col;
   const T* p = H + b * S * K + c;
   float v[W];
 #pragma unroll

@@ -114,7 +114,11 @@ def test_ops_on_ragged_rows_match_whole_vectors(B, S, D, dtype, shifted):
 
 
 @pytest.mark.parametrize("B,S,D,dtype", [(5, 7, 11235, torch.bfloat16), (3, 130, 1009, torch.float16),
-                                         (2, 9, 21846, torch.float32)])
+                                         (2, 9, 21846, torch.float32),
+                                         # 4 D just past a whole number of column blocks: the last block
+                                         # of a row is half a vector (64-lane and 256-lane blocks)
+                                         (1, 3200, 129, torch.bfloat16), (2, 200, 1025, torch.float16),
+                                         (110, 7, 513, torch.bfloat16)])
 @pytest.mark.parametrize("shifted", [False, True])
 def test_mean_pool_on_ragged_rows(B, S, D, dtype, shifted):
     """fp32 sums of S values each: 2 S 2^-24 of the mean of |H|, at most 2^-14 here."""
