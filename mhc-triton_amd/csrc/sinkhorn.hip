@@ -6,7 +6,7 @@
 // 256.  The forward is VALU-bound at 20 rounds (32 VALU ops and 8 v_rcp per
 // round in the scaling-vector form of sk_forward with a small eps, 40 + 8
 // otherwise: 2^20 bf16 matrices 39.1 -> 32.5 us; fp32 forward 45.4 -> 39.7,
-// fwd + bwd 129.1 -> 123.3 on one box with its reads and writes coalesced, and at 32 rounds
+// fwd + bwd 129.1 -> 123.3 in one comparison with its reads and writes coalesced, and at 32 rounds
 // 229 -> 202); the backward keeps every round's
 // scaling vectors in registers for up to 20 rounds and carries the adjoint in
 // scaled coordinates (sk_backward_scaled: 95-100 us at 2^20 matrices, 20
