@@ -811,6 +811,8 @@ inline hipError_t launch_dynw_bwd_wide(const TX* x, const float* phi, const floa
 // steps as graphs, apart -> in one: fp32 B=2, S=128, D=512 (32 partials per row) 40.5 -> 38.5 us, bf16
 // B=4, S=256, D=1024 (64) 48.3 -> 45.7, B=4, S=256, D=2048 (128) 57.5 -> 55.5, B=4, S=512, D=2048
 // (256) equal at 85.4 but a launch less for the host; B=1, S=512, D=4096 (512) 58.5 -> 60.6.
+// Those with a lane's records summed one by one in f32; four at a time and f64 sums, as below, gave
+// 45.7 -> 45.3, 55.3 -> 54.8 and 84.9 -> 84.0 for 64, 128 and 256 partials (fp32 equal at 38.6).
 constexpr int kFusedRows = 4;
 constexpr int kFusedPartials = 256;  // partials per row
 
@@ -820,7 +822,8 @@ __global__ __launch_bounds__(kWideThreads) void dynw_bwd_rows_wide_kernel(
     const float* __restrict__ w, const float* __restrict__ dpost, const float* __restrict__ part20, int nblk,
     float* __restrict__ gx, float* __restrict__ gphi, float* __restrict__ gbias, float* __restrict__ galpha, int R,
     int64_t K, int iters, float eps, bool phi_vec) {
-  __shared__ __attribute__((aligned(16))) float tot[kFusedRows][20];
+  __shared__ float tot[kFusedRows][20];
+  __shared__ double lanes[64][21];
   __shared__ float rec[kFusedRows][kRow];
   __shared__ float slots[kSkSlots * 64];
   const int lane = threadIdx.x, e = lane & 15, grp = lane >> 4;
@@ -835,22 +838,39 @@ __global__ __launch_bounds__(kWideThreads) void dynw_bwd_rows_wide_kernel(
 #pragma unroll
   for (int q = 0; q < kFusedRows; ++q) xv[q] = live_k && q < R ? to_f32(x[q * K + k]) : 0.f;
   const int r = grp < R ? grp : R - 1;  // idle groups redo the last row and store nothing
-  f32x4 acc[5];
+  // Four records in an f32 tree, what they give and the lanes' sums in f64: a chain of f32 sums over
+  // the 16 records of a lane would round more than the rows kernel's trees do.
+  double acc[20];
 #pragma unroll
-  for (int q = 0; q < 5; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-  for (int n = e; n < nblk; n += 16) {
-    const f32x4* p = reinterpret_cast<const f32x4*>(part20 + ((int64_t)r * nblk + n) * 20);
+  for (int v = 0; v < 20; ++v) acc[v] = 0.0;
+  const f32x4* p = reinterpret_cast<const f32x4*>(part20 + ((int64_t)r * nblk + e) * 20);
+  constexpr int kStep = 16 * 5;  // vectors from a lane's record to its next
+  int n = e;
+  for (; n + 48 < nblk; n += 64, p += 4 * kStep) {
 #pragma unroll
-    for (int q = 0; q < 5; ++q) acc[q] += p[q];
+    for (int q = 0; q < 5; ++q) {
+      const f32x4 t = (p[q] + p[kStep + q]) + (p[2 * kStep + q] + p[3 * kStep + q]);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[4 * q + c] += t[c];
+    }
+  }
+  for (; n < nblk; n += 16, p += kStep) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+      const f32x4 t = p[q];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[4 * q + c] += t[c];
+    }
   }
 #pragma unroll
-  for (int q = 0; q < 5; ++q) {
+  for (int v = 0; v < 20; ++v) lanes[lane][v] = acc[v];
+  __syncthreads();
+  for (int i = lane; i < kFusedRows * 20; i += 64) {
+    const int g = i / 20, v = i % 20;
+    double t = 0.0;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float v = sum_all16(acc[q][c]);
-      if (e == 0) tot[grp][4 * q + c] = v;
-    }
+    for (int l = 0; l < 16; ++l) t += lanes[16 * g + l][v];
+    tot[g][v] = (float)t;
   }
   __syncthreads();
   const int j4 = e & 3;
