@@ -3,11 +3,11 @@
 // src/mhc/_backward.py:29-262,503-530).
 //
 // One matrix per lane: a wave handles 64 matrices, a 256-thread workgroup
-// 256.  The forward is VALU-bound at 20 rounds (32 VALU ops and 8 v_rcp per
-// round in the scaling-vector form of sk_forward with a small eps, 40 + 8
-// otherwise: 2^20 bf16 matrices 39.1 -> 32.5 us; fp32 forward 45.4 -> 39.7,
-// fwd + bwd 129.1 -> 123.3 in one comparison with its reads and writes coalesced, and at 32 rounds
-// 229 -> 202); the backward keeps every round's
+// 256.  The forward is VALU-bound at 20 rounds (40 VALU ops and 8 v_rcp per
+// round in the scaling-vector form of sk_forward, 32 + 8 from the eighth round
+// on with a small eps: 2^20 bf16 matrices 38.5 -> 33.6 us; fp32, whose reads and
+// writes are also coalesced, 40.6 -> 38.8 us, fwd + bwd 118.8 -> 113.4 and at 32
+// rounds 227 -> 210); the backward keeps every round's
 // scaling vectors in registers for up to 20 rounds and carries the adjoint in
 // scaled coordinates (sk_backward_scaled: 95-100 us at 2^20 matrices, 20
 // rounds, when chosen, against 131 us for the explicit normalisation backward on the same
@@ -174,8 +174,8 @@ extern "C" int mhc_sinkhorn_forward(const void* M, void* out, int64_t n_mat, int
   const bool vec = aligned16(M) && aligned16(out);
   const dim3 grid((unsigned)((n_mat + kThreads - 1) / kThreads));
   return MHC_DISPATCH_DTYPE(dtype, [&] {
-    auto* k = vec ? (eps <= kSkSmallEps ? sinkhorn_fwd_kernel<T, true, true> : sinkhorn_fwd_kernel<T, true, false>)
-                  : (eps <= kSkSmallEps ? sinkhorn_fwd_kernel<T, false, true> : sinkhorn_fwd_kernel<T, false, false>);
+    auto* k = vec ? (sk_small_eps(eps) ? sinkhorn_fwd_kernel<T, true, true> : sinkhorn_fwd_kernel<T, true, false>)
+                  : (sk_small_eps(eps) ? sinkhorn_fwd_kernel<T, false, true> : sinkhorn_fwd_kernel<T, false, false>);
     k<<<grid, kThreads, 0, (hipStream_t)stream>>>((const T*)M, (T*)out, n_mat, iters, eps);
     return hip_status(hipGetLastError(), "sinkhorn_forward launch");
   });
@@ -191,8 +191,8 @@ extern "C" int mhc_sinkhorn_backward(const void* M, int dtype_M, const void* dP,
   return MHC_DISPATCH_DTYPE(dtype_M, [&] {
     using TM = T;
     return MHC_DISPATCH_DTYPE(dtype_dP, [&] {
-      auto* k = vec ? (eps <= kSkSmallEps ? sinkhorn_bwd_kernel<TM, T, true, true> : sinkhorn_bwd_kernel<TM, T, true, false>)
-                    : (eps <= kSkSmallEps ? sinkhorn_bwd_kernel<TM, T, false, true>
+      auto* k = vec ? (sk_small_eps(eps) ? sinkhorn_bwd_kernel<TM, T, true, true> : sinkhorn_bwd_kernel<TM, T, true, false>)
+                    : (sk_small_eps(eps) ? sinkhorn_bwd_kernel<TM, T, false, true>
                                           : sinkhorn_bwd_kernel<TM, T, false, false>);
       k<<<grid, kThreads, 0, (hipStream_t)stream>>>((const TM*)M, (const T*)dP, (TM*)dM, n_mat, iters, eps);
       return hip_status(hipGetLastError(), "sinkhorn_backward launch");

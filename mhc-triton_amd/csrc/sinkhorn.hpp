@@ -64,31 +64,43 @@ __device__ __forceinline__ void sk_init(float (&m)[16], float eps) {
 // evaluation of the explicit form of 1.7e-7 (2.2e-7 for the explicit fp32
 // update).  The backward keeps sk_round for its recomputed states.
 //
-// SMALL: with eps <= kSkSmallEps the eps terms are left out from the second round on, where they
-// are below half a unit in the last place.  From then on one round changes w by a factor of at most
-// 4: P_ij u_i v_j <= 1 after a normalisation bounds every term of the new (P0 v)_i by the old w_i, so
-// w_new <= 4 w_old, the same holds for z, and then z_new = sum P_ij / w_new >= z_old / 4 (up to
-// eps) and likewise for w.  eps w_old is thus at most 4 eps (P0 v)_i, 2^-24 of it.  The first round,
-// where w starts from 1 whatever the size of P0, keeps them (a matrix of zeros needs it to).  32 VALU
-// + 8 v_rcp (a quarter-rate instruction) per round instead of 40 + 8.
+// SMALL: with 0 <= eps <= kSkSmallEps the eps terms are left out after the first kSkEpsRounds rounds,
+// where each is at most 2^-24 of the sum it belongs to (a rounding of that sum; near eps itself, 2^-27,
+// once the matrix has converged).  With d_t the dot of round t's half round, so that z_t = d_t +
+// eps z_{t-1}:
+//   * d_{t+1} >= d_t / (4 + eps) on both sides: z_t,j >= P0_ij / w_t,i bounds each of the four terms
+//     P0_ij / z_t,j of w_{t+1},i by w_t,i, hence w_{t+1} <= (4 + eps) w_t, and the terms P0_ij / w_i of
+//     the next d shrink by no more; likewise with the sides exchanged.
+//   * So the eps share r_t = eps z_{t-1} / d_t obeys r_{t+1} <= (4 + eps) eps (1 + r_t): it falls by 2^24 a
+//     round until it is 4 eps.
+//   * For w it starts at r_1 <= 1/4 (P0 >= eps gives d_1 >= 4 eps).  For z it starts anywhere below a quarter
+//     of the largest row sum: d_1 is a column's share of normalised rows, 4e-12 for a zero column
+//     beside rows of size 1e4, and z_1 is then all eps.  From 2^126, the most that finite row sums allow,
+//     it is under 2^-17 after seven rounds and 4 eps in the eighth.
+// 32 VALU + 8 v_rcp (a quarter-rate instruction) per round instead of 40 + 8 from there on.  (Leaving
+// the terms out from the second round on moved P by 4e-5 after two rounds of size 1e4 and by 4e-3 of size
+// 1e6, where a column was zero.)
 constexpr float kSkSmallEps = 0x1p-26f;
+constexpr int kSkEpsRounds = 7;
+
+inline bool sk_small_eps(float eps) { return eps >= 0.f && eps <= kSkSmallEps; }
 
 // One half round: s[k] <- sum of P0's row or column k scaled by the other side's vector, + eps s[k].
 template <bool SMALL>
-__device__ __forceinline__ float sk_carry(float eps, float old, float dot, bool first) {
-  return SMALL && !first ? dot : __builtin_fmaf(eps, old, dot);
+__device__ __forceinline__ float sk_carry(float eps, float old, float dot, bool early) {
+  return SMALL && !early ? dot : __builtin_fmaf(eps, old, dot);
 }
 
 template <bool SMALL>
 __device__ __forceinline__ void sk_forward_round(const float (&m)[16], float (&w)[4], float (&z)[4], float eps,
-                                                 bool first) {
+                                                 bool early) {
   float v[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) v[j] = fast_rcp(z[j]);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const float dot = m[4 * i] * v[0] + m[4 * i + 1] * v[1] + m[4 * i + 2] * v[2] + m[4 * i + 3] * v[3];
-    w[i] = sk_carry<SMALL>(eps, w[i], dot, first);
+    w[i] = sk_carry<SMALL>(eps, w[i], dot, early);
   }
   float u[4];
 #pragma unroll
@@ -96,7 +108,7 @@ __device__ __forceinline__ void sk_forward_round(const float (&m)[16], float (&w
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const float dot = u[0] * m[j] + u[1] * m[4 + j] + u[2] * m[8 + j] + u[3] * m[12 + j];
-    z[j] = sk_carry<SMALL>(eps, z[j], dot, first);
+    z[j] = sk_carry<SMALL>(eps, z[j], dot, early);
   }
 }
 
@@ -104,8 +116,9 @@ template <bool SMALL>
 __device__ __forceinline__ void sk_forward(float (&m)[16], int iters, float eps) {
   sk_init(m, eps);
   float w[4] = {1.f, 1.f, 1.f, 1.f}, z[4] = {1.f, 1.f, 1.f, 1.f};
-  if (iters > 0) sk_forward_round<SMALL>(m, w, z, eps, true);
-  for (int t = 1; t < iters; ++t) sk_forward_round<SMALL>(m, w, z, eps, false);
+  const int early = SMALL && iters > kSkEpsRounds ? kSkEpsRounds : iters;
+  for (int t = 0; t < early; ++t) sk_forward_round<SMALL>(m, w, z, eps, true);
+  for (int t = early; t < iters; ++t) sk_forward_round<SMALL>(m, w, z, eps, false);
   float u[4], v[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -234,14 +247,14 @@ __device__ __forceinline__ void sk_backward_scaled(const float (&mat)[16], float
         for (int i = 0; i < 4; ++i) {
           const float dot = p0[4 * i] * V[t][0] + p0[4 * i + 1] * V[t][1] + p0[4 * i + 2] * V[t][2] +
                             p0[4 * i + 3] * V[t][3];
-          w[i] = sk_carry<SMALL>(eps, w[i], dot, t == 0);
+          w[i] = sk_carry<SMALL>(eps, w[i], dot, t < kSkEpsRounds);
           U[t + 1][i] = fast_rcp(w[i]);
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const float dot = U[t + 1][0] * p0[j] + U[t + 1][1] * p0[4 + j] + U[t + 1][2] * p0[8 + j] +
                             U[t + 1][3] * p0[12 + j];
-          z[j] = sk_carry<SMALL>(eps, z[j], dot, t == 0);
+          z[j] = sk_carry<SMALL>(eps, z[j], dot, t < kSkEpsRounds);
           V[t + 1][j] = fast_rcp(z[j]);
         }
       }
@@ -303,17 +316,18 @@ __device__ __forceinline__ void sk_backward_segmented(const float (&mat)[16], fl
     zero |= (mat[k] == 0.f ? 1u : 0u) << k;
   }
   // one round of the carried iteration: w from v, u = rcp(w), z from u, v = rcp(z)
-  auto sk_step = [&](float (&w)[4], float (&z)[4], const float (&v)[4], float (&u1)[4], float (&v1)[4], bool first) {
+  static_assert(TSEG >= kSkEpsRounds, "the rounds with eps lie in the first segment");
+  auto sk_step = [&](float (&w)[4], float (&z)[4], const float (&v)[4], float (&u1)[4], float (&v1)[4], bool early) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float dot = p0[4 * i] * v[0] + p0[4 * i + 1] * v[1] + p0[4 * i + 2] * v[2] + p0[4 * i + 3] * v[3];
-      w[i] = sk_carry<SMALL>(eps, w[i], dot, first);
+      w[i] = sk_carry<SMALL>(eps, w[i], dot, early);
       u1[i] = fast_rcp(w[i]);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float dot = u1[0] * p0[j] + u1[1] * p0[4 + j] + u1[2] * p0[8 + j] + u1[3] * p0[12 + j];
-      z[j] = sk_carry<SMALL>(eps, z[j], dot, first);
+      z[j] = sk_carry<SMALL>(eps, z[j], dot, early);
       v1[j] = fast_rcp(z[j]);
     }
   };
@@ -330,7 +344,7 @@ __device__ __forceinline__ void sk_backward_segmented(const float (&mat)[16], fl
       const int tend = iters < (k + 1) * TSEG ? iters : (k + 1) * TSEG;
       for (int t = k * TSEG; t < tend; ++t) {
         float u1[4], v1[4];
-        sk_step(w, z, v, u1, v1, t == 0);
+        sk_step(w, z, v, u1, v1, k == 0 && t < kSkEpsRounds);
 #pragma unroll
         for (int q = 0; q < 4; ++q) v[q] = v1[q];
       }
@@ -364,7 +378,7 @@ __device__ __forceinline__ void sk_backward_segmented(const float (&mat)[16], fl
     }
 #pragma unroll
     for (int tt = 0; tt < TSEG; ++tt)
-      if (t0 + tt < iters) sk_step(w, z, V[tt], U[tt + 1], V[tt + 1], t0 + tt == 0);
+      if (t0 + tt < iters) sk_step(w, z, V[tt], U[tt + 1], V[tt + 1], k == 0 && tt < kSkEpsRounds);
 #pragma unroll
     for (int tt = TSEG - 1; tt >= 0; --tt) {
       if (t0 + tt < iters) {

@@ -1,5 +1,6 @@
 """Kernels and dispatch lines that the launchers pick by size, at the sizes where they can go wrong."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -211,9 +212,9 @@ def test_whole_batch_without_a_closure_gradient(B, S, D):
 @pytest.mark.parametrize("eps", [0.0, 2.0 ** -26, 2.0 ** -25])
 @pytest.mark.parametrize("iters", [0, 2, 33])
 def test_sinkhorn_forms(n, dtype, eps, iters):
-    """Partial waves, and eps on both sides of the line up to which its terms are left out after the
-    first round (below half a unit there): entries over twelve decades, zeros among them where eps
-    keeps the sums positive.  One v_rcp and one rounding per normalised entry: 4e-7 of the largest."""
+    """Partial waves of matrices whose sizes spread over eight decades, with a zero row and a zero column
+    where eps keeps the sums positive.  One v_rcp and one rounding per normalised entry: 4e-7 of the
+    largest."""
     import mhc
     from helpers import rel_err, to_np
     from oracle import mhc_oracle as O
@@ -228,6 +229,47 @@ def test_sinkhorn_forms(n, dtype, eps, iters):
     want = O.sinkhorn(to_np(M), iters, eps)
     half = {torch.float32: 0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
     assert rel_err(to_np(P), want) < 1e-6 + half
+
+
+@pytest.mark.parametrize("eps", [1e-8, 2.0 ** -26, 1e-6])
+@pytest.mark.parametrize("iters", [1, 2, 3, 7, 8, 20, 33, 65])
+@pytest.mark.parametrize("shifted", [False, True])
+def test_sinkhorn_of_tiny_rows_and_columns(eps, iters, shifted):
+    """P and dM where a row or a column is zero, or a millionth of the others, in matrices of sizes from
+    0.01 to 1e20: there eps, or what it left in the column sums, outweighs that column for several
+    rounds (at size 1e6 an eps term left out of the second round moves P by 4e-3, at 1e20 one left out of
+    the third still moves it by more).  With eps on both sides of the line up to which its terms are
+    left out from the eighth round on.  Matrix by matrix, over its largest entry: a round rounds each
+    entry of P twice and its reciprocals once, so P is within a few 2^-23 whatever the round (each
+    renormalises), and the backward adds two roundings a round."""
+    import mhc
+    from helpers import to_np
+    from oracle import mhc_oracle as O
+
+    n = 96
+    g = torch.Generator(device=DEV).manual_seed(5)
+    M = torch.randn((6, n, 4, 4), generator=g, device=DEV)
+    M *= torch.tensor([1e-2, 1.0, 1e2, 1e4, 1e6, 1e20], device=DEV)[:, None, None, None]
+    M[:, 1::6, :, 2] = 0
+    M[:, 2::6, 1] = 0
+    M[:, 3::6, :, 0] *= 1e-6
+    M[:, 4::6, 3] *= 1e-6
+    M[:, 5::6, :, 2] = 0
+    M[:, 5::6, 1] = 0
+    M = M.reshape(-1, 4, 4)
+    dP = torch.randn(M.shape, generator=g, device=DEV)
+    if shifted:
+        M, dP = off_by_one(M), off_by_one(dP)
+    M.requires_grad_(True)
+    P = mhc.sinkhorn_knopp(M, iters, eps)
+    P.backward(dP)
+    eps32 = float(np.float32(eps))
+    for got, want, tol in ((P, O.sinkhorn(to_np(M), iters, eps32), 8 * 2.0 ** -23),
+                           (M.grad, O.sinkhorn_backward(to_np(M), to_np(dP), iters, eps32),
+                            (2 * iters + 8) * 2.0 ** -23)):
+        err = np.abs(to_np(got) - want).max(axis=(1, 2)) / np.abs(want).max(axis=(1, 2))
+        print(f"sinkhorn eps={eps} iters={iters} shifted={shifted}: worst {err.max():.2e} of {tol:.2e}", flush=True)
+        assert err.max() < tol
 
 
 @pytest.mark.parametrize("R,K", [

@@ -70,3 +70,34 @@ def test_scaled_forward_vectors_reproduce_the_explicit_state():
         v = 1.0 / z
         P = p0 * u[:, :, None] * v[:, None, :]
         np.testing.assert_allclose(P, O.sinkhorn(M, t, eps), rtol=1e-12, atol=0)
+
+
+def carried_f32(M, iters, eps, eps_rounds):
+    """The kernel's carried iteration in float32: w = P0 v + eps w, z = P0^T u + eps z, u = 1/w, v = 1/z,
+    with the eps terms in the first eps_rounds rounds only."""
+    f = np.float32
+    p0 = np.abs(M).astype(f) + f(eps)
+    w = np.ones(M.shape[:2], f)
+    z = np.ones(M.shape[:2], f)
+    for t in range(iters):
+        e = f(eps) if t < eps_rounds else f(0)
+        w = (p0 * (f(1) / z)[:, None, :]).sum(axis=2, dtype=f) + e * w
+        z = (p0 * (f(1) / w)[:, :, None]).sum(axis=1, dtype=f) + e * z
+    return (f(1) / w)[:, :, None] * p0 * (f(1) / z)[:, None, :]
+
+
+@pytest.mark.parametrize("size", [1e-2, 1.0, 1e2, 1e4, 1e6, 1e12, 1e20, 1e30])
+@pytest.mark.parametrize("iters", [1, 2, 3, 7, 8, 9, 20])
+@pytest.mark.parametrize("eps", [1e-8, 2.0 ** -26])
+def test_eps_counts_in_the_first_rounds(size, iters, eps):
+    """With a zero column the first round leaves z = eps there (its start value's share), and the second
+    round's sum is only about eps / size: eps z counts.  Kept for seven rounds (kSkEpsRounds), P is within
+    a few 2^-23 of the oracle; kept for one, it is off by more than 1e-10 size after two rounds."""
+    eps = float(np.float32(eps))
+    M = (np.random.default_rng(0).standard_normal((64, 4, 4)) * size).astype(np.float32)
+    M[::2, :, 2] = 0
+    M[1::4, 1] = 0
+    ref = O.sinkhorn(M, iters, eps)
+    assert np.abs(carried_f32(M, iters, eps, 7) - ref).max() < 8 * 2.0 ** -23
+    if iters == 2 and 1e4 <= size <= 1e6:
+        assert np.abs(carried_f32(M, iters, eps, 1) - ref).max() > 1e-10 * size
