@@ -5,9 +5,9 @@
 // One matrix per lane: a wave handles 64 matrices, a 256-thread workgroup
 // 256.  The forward is VALU-bound at 20 rounds (40 VALU ops and 8 v_rcp per
 // round in the scaling-vector form of sk_forward, 32 + 8 from the eighth round
-// on with a small eps: 2^20 bf16 matrices 38.5 -> 33.6 us; fp32, whose reads and
-// writes are also coalesced, 40.6 -> 38.8 us, fwd + bwd 118.8 -> 113.4 and at 32
-// rounds 227 -> 210); the backward keeps every round's
+// on with a small eps: 2^20 bf16 matrices 38.5 -> 33.3 us, fp16 39.6 -> 34.4;
+// fp32, whose reads and writes also go through LDS, 40.6 -> 38.8, and fwd + bwd
+// 118.8 -> 113.4, at 32 rounds 227 -> 210); the backward keeps every round's
 // scaling vectors in registers for up to 20 rounds and carries the adjoint in
 // scaled coordinates (sk_backward_scaled: 95-100 us at 2^20 matrices, 20
 // rounds, when chosen, against 131 us for the explicit normalisation backward on the same
@@ -22,12 +22,13 @@
 
 namespace mhc {
 
-// A wave's 64 matrices are one contiguous span (4 KiB in fp32, 2 KiB in 16 bits).  It is read and
-// written 1 KiB per access, 16 bytes a lane, and changes hands in the wave's own LDS tile, where lane
-// l picks up the chunks of matrix l (a lane loading its own matrix directly touches 32 lines per
-// access: the forward over 2^20 fp32 matrices took 41.3 us at 20 rounds and 40.7 at 7, against
-// 35.7-39.7 and 31.1-32.1 so).  Chunk c sits in slot c with its low three bits turned by c / 8, so that eight lanes in a row
-// hit different banks both ways.
+// A wave's 64 fp32 matrices are one contiguous span of 4 KiB.  The forward reads and writes it 1 KiB
+// per access, 16 bytes a lane, and it changes hands in the wave's own LDS tile, where lane l picks up
+// the chunks of matrix l.  A lane loading its own 64 bytes touches 32 lines per access: 2^20 matrices
+// at 7 rounds took 34.8 us against 26.9 so.  Of 16 bits (32 bytes a lane)
+// lanes load their own: 21.4 against 22.5 us at 7 rounds, 33.3 against 33.6 at 20 in bf16, 22.2 against
+// 23.8 and 34.4 against 36.3 in fp16.  Chunk c sits in slot c with its low three bits turned by c / 8,
+// so that eight lanes in a row hit different banks both ways.
 template <typename T>
 struct WaveTile {
   static constexpr int N = Vec<T>::N;   // elements per chunk
@@ -108,7 +109,7 @@ template <typename T, bool VEC, bool SMALL>
 __global__ __launch_bounds__(kThreads) void sinkhorn_fwd_kernel(const T* __restrict__ M, T* __restrict__ out,
                                                                 int64_t n, int iters, float eps) {
   float m[16];
-  if constexpr (VEC) {
+  if constexpr (VEC && sizeof(T) == 4) {
     using Tile = WaveTile<T>;
     __shared__ __attribute__((aligned(16))) u32x4 tiles[kSkWaves][64 * Tile::Q];
     const int64_t i0 = (int64_t)blockIdx.x * kThreads + (threadIdx.x & ~63);  // the wave's first matrix
@@ -123,9 +124,9 @@ __global__ __launch_bounds__(kThreads) void sinkhorn_fwd_kernel(const T* __restr
   } else {
     const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (i >= n) return;
-    load_mat<T, false>(M + i * 16, m);
+    load_mat<T, VEC>(M + i * 16, m);
     sk_forward<SMALL>(m, iters, eps);
-    store_mat<T, false>(out + i * 16, m);
+    store_mat<T, VEC>(out + i * 16, m);
   }
 }
 
