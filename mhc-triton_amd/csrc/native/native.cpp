@@ -86,14 +86,13 @@ Tensor empty_f32(at::IntArrayRef sizes, const Tensor& like) {
 
 // The f32 values of N <= 8 parameters: the parameters' own memory, or, where any is stored in another
 // dtype, one buffer of them all, converted in one launch.  The forward keeps the buffer for the
-// backward (which then reads nothing from the parameters, so what a saved-tensor hook does to their
-// layout does not matter).
+// backward, which then reads nothing from the parameters.
 template <int N>
 struct Params {
   const float* p[N];
   Tensor buf;
 
-  Params(const Tensor* t, const Tensor& have) : buf(have) {
+  Params(const Tensor* t, const Tensor& have) : buf(f32(have)) {
     int64_t at[N], total = 0;
     bool own = !buf.defined();
     for (int i = 0; i < N; ++i) {
@@ -277,9 +276,9 @@ struct DynamicLayer : Function<DynamicLayer> {
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const variable_list s = ctx->get_saved_variables();
-    const Tensor& H = s[0];
+    const c10::DeviceGuard guard(s[0].device());
+    const Tensor H = s[0].contiguous();
     const Tensor* prm = &s[4];
-    const c10::DeviceGuard guard(H.device());
     const Dims d(H);
     const Tensor d_bi = d_bi_or_zeros(g[0], H, d);
     const Tensor dHn = in_dtype(g[2], H.scalar_type());
@@ -288,7 +287,7 @@ struct DynamicLayer : Function<DynamicLayer> {
     const float* const* p = q.p;
     const Tensor x = f32(s[1]), w = f32(s[2]), aux = f32(s[3]);
     Tensor dH;
-    if (ctx->needs_input_grad(0)) dH = at::empty_like(H);
+    if (ctx->needs_input_grad(0)) dH = at::empty(H.sizes(), H.options().requires_grad(false));
     const Tensor gphi = empty_f32({4 * d.D, 24}, H);
     const Tensor small = empty_f32({27}, H);  // grad_bias [24], grad_alpha [3]
     const Workspace ws(mhc_layer_workspace_bytes(d.B, d.S, d.D, code(H)), H);
@@ -365,16 +364,16 @@ struct StaticLayer : Function<StaticLayer> {
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
     const variable_list s = ctx->get_saved_variables();
-    const Tensor& H = s[0];
+    const c10::DeviceGuard guard(s[0].device());
+    const Tensor H = s[0].contiguous();
     const Tensor* prm = &s[2];
-    const c10::DeviceGuard guard(H.device());
     const Dims d(H);
     const Tensor d_bi = d_bi_or_zeros(g[0], H, d);
     const Tensor dHn = in_dtype(g[2], H.scalar_type());
     const Tensor dpost = f32(g[3]), w = f32(s[1]);
     const Params<3> q(prm, s[5]);
     Tensor dH;
-    if (ctx->needs_input_grad(0)) dH = at::empty_like(H);
+    if (ctx->needs_input_grad(0)) dH = at::empty(H.sizes(), H.options().requires_grad(false));
     const Tensor gb = empty_f32({24}, H);
     const Workspace ws(mhc_layer_workspace_bytes(d.B, d.S, d.D, code(H)), H);
     check(mhc_layer_static_backward(ptr(H), code(H), ptr(d_bi), ptr(dHn), fptr(dpost), q.p[0], q.p[1], q.p[2], fptr(w), ptr(dH), wptr(gb), d.B, d.S, d.D,
@@ -655,11 +654,12 @@ struct DynamicWeights : Function<DynamicWeights> {
     const int64_t R = x.size(0), K = x.size(1);
     const Params<kDw - 1> q(&s[1], s[8]);
     const float* const* p = q.p;
+    const Tensor pre = f32(s[6]), aux = f32(s[7]);
     const Tensor g0 = f32(g[0]), g1 = f32(g[1]), g2 = f32(g[2]);
     const Tensor gx = at::empty(x.sizes(), x.options().requires_grad(false));
     const Tensor gphi = empty_f32({K, 24}, x), small = empty_f32({27}, x);
     const Workspace ws(mhc_dynamic_weights_backward_workspace_bytes(R, K), x);
-    check(mhc_dynamic_weights_backward(ptr(x), code(x), p[0], p[1], p[2], p[3], p[4], fptr(s[7]), fptr(s[6]), fptr(g0),
+    check(mhc_dynamic_weights_backward(ptr(x), code(x), p[0], p[1], p[2], p[3], p[4], fptr(aux), fptr(pre), fptr(g0),
                                        fptr(g1), fptr(g2), ptr(gx), wptr(gphi), wptr(small), wptr(small) + 24, R, K,
                                        (int)ctx->saved_data["iters"].toInt(),
                                        (float)ctx->saved_data["eps"].toDouble(), ws.p(), ws.bytes, stream(x)),

@@ -195,3 +195,60 @@ def test_converted_parameters(monkeypatch, dtypes, offload):
         return [bi, Hn] + [grads[k] for k in sorted(grads)]
 
     same(*both(monkeypatch, step))
+
+
+def strided(t):
+    """t's values in every second element of a storage of its own (no dimension is contiguous)."""
+    return torch.stack((t, torch.full_like(t, 7)), dim=-1)[..., 0]
+
+
+def turned(t):
+    """t's values with its dimensions laid out in reverse order."""
+    order = tuple(range(t.dim()))[::-1]
+    return t.permute(order).contiguous().permute(order)
+
+
+@pytest.mark.parametrize("layout", [strided, turned])
+@pytest.mark.parametrize("dynamic,half_params", [(True, False), (True, True), (False, False), (False, True)])
+def test_layer_backward_from_saved_tensors_in_other_strides(monkeypatch, layout, dynamic, half_params):
+    """An unpack hook that hands every saved tensor back in other strides: the gradients without it, in
+    the default layout."""
+    hc, H, bo, dHn, dbi = make_case(3, 6, 40, torch.float32, dynamic=dynamic, phi_std=0.02, res_std=1.0)
+    hc = hc.to(torch.bfloat16) if half_params else hc
+    _, _, plain = run_gpu(hc, H, bo, dHn, dbi)
+
+    def step():
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, layout):
+            _, _, grads = run_gpu(hc, H, bo, dHn, dbi)
+        assert all(g.is_contiguous() for g in grads.values())
+        return [grads[k] for k in sorted(grads)]
+
+    got, want = both(monkeypatch, step)
+    same(got, want)
+    same(got, [plain[k] for k in sorted(plain)])
+
+
+def ops_step(hooks):
+    """Gradients of the low-level ops with saved-tensor hooks."""
+    import mhc
+    from mhc import streams
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    r = lambda *s: torch.randn(s, generator=g, device=DEV)  # noqa: E731
+    L = [r(2, 6, 24), r(2, 6, 24), r(5, 4, 4), r(2, 4), r(2, 4).bfloat16(), r(2, 4, 4), r(6, 96), r(96, 24) * 0.1,
+         r(24).bfloat16(), r(1), r(1), r(1)]
+    L = [t.requires_grad_(True) for t in L]
+    with torch.autograd.graph.saved_tensors_hooks(*hooks):
+        bi, hr = mhc.fused_stream_mix(streams.expand_streams(L[0]), L[3], L[5])
+        y = streams.collapse_streams(mhc.fused_add_residual(hr, L[1], L[4]))
+        P = mhc.sinkhorn_knopp(L[2], 9, 1e-6)
+        W = mhc.fused_dynamic_weights(*L[6:12], 7, 1e-5)
+        out = [bi, y, P, *W]
+    w = [torch.randn(t.shape, generator=g, device=DEV) for t in out]
+    torch.autograd.backward(out, w)
+    return [t.grad for t in L]
+
+
+@pytest.mark.parametrize("layout", [strided, turned])
+def test_op_backwards_from_saved_tensors_in_other_strides(layout):
+    same(ops_step((lambda t: t, layout)), ops_step((lambda t: t, lambda t: t)))
