@@ -84,6 +84,21 @@ Tensor empty_f32(at::IntArrayRef sizes, const Tensor& like) {
   return at::empty(sizes, like.options().dtype(at::kFloat).requires_grad(false));
 }
 
+// What a node saved.  An unpack hook may hand back other strides, another dtype or another device: the
+// backwards take each tensor through contiguous() or f32(), and a tensor that is not on the first
+// one's GPU is refused here, as the Python nodes refuse it (_lib.require_gpu).
+variable_list saved(AutogradContext* ctx) {
+  variable_list s = ctx->get_saved_variables();
+  for (const Tensor& t : s) {
+    if (!t.defined()) continue;
+    TORCH_CHECK(t.is_cuda(), "mhc: the HIP kernels need tensors on a ROCm GPU, got device '", t.device(),
+                "' from a saved-tensor hook");
+    TORCH_CHECK(t.device() == s[0].device(), "mhc: tensors on different devices (", s[0].device(), " and ", t.device(),
+                ")");
+  }
+  return s;
+}
+
 // The f32 values of N <= 8 parameters: the parameters' own memory, or, where any is stored in another
 // dtype, one buffer of them all, converted in one launch.  The forward keeps the buffer for the
 // backward, which then reads nothing from the parameters.
@@ -275,7 +290,7 @@ struct DynamicLayer : Function<DynamicLayer> {
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    const variable_list s = ctx->get_saved_variables();
+    const variable_list s = saved(ctx);
     const c10::DeviceGuard guard(s[0].device());
     const Tensor H = s[0].contiguous();
     const Tensor* prm = &s[4];
@@ -363,7 +378,7 @@ struct StaticLayer : Function<StaticLayer> {
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    const variable_list s = ctx->get_saved_variables();
+    const variable_list s = saved(ctx);
     const c10::DeviceGuard guard(s[0].device());
     const Tensor H = s[0].contiguous();
     const Tensor* prm = &s[2];
@@ -428,7 +443,7 @@ struct LayerAdd : Function<LayerAdd> {
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    const variable_list s = ctx->get_saved_variables();
+    const variable_list s = saved(ctx);
     const c10::DeviceGuard guard(g[0].device());
     const Tensor dHn = in_dtype(g[0], (at::ScalarType)ctx->saved_data["h_dtype"].toInt());
     const Dims d(dHn);
@@ -483,7 +498,7 @@ struct Sinkhorn : Function<Sinkhorn> {
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    const Tensor M = ctx->get_saved_variables()[0].contiguous();
+    const Tensor M = saved(ctx)[0].contiguous();
     const c10::DeviceGuard guard(M.device());
     const Tensor dP = g[0].contiguous();
     const Tensor dM = at::empty(M.sizes(), M.options().requires_grad(false));
@@ -531,7 +546,7 @@ struct StreamMix : Function<StreamMix> {
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    const variable_list s = ctx->get_saved_variables();
+    const variable_list s = saved(ctx);
     const c10::DeviceGuard guard(s[0].device());
     const Tensor H = s[0].contiguous();
     const Dims d(H);
@@ -582,7 +597,7 @@ struct AddResidual : Function<AddResidual> {
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    const variable_list s = ctx->get_saved_variables();
+    const variable_list s = saved(ctx);
     const c10::DeviceGuard guard(g[0].device());
     const Tensor dHn = g[0].contiguous(), bo = s[0].contiguous(), post = f32(s[1]);
     const Dims d(dHn);
@@ -648,7 +663,7 @@ struct DynamicWeights : Function<DynamicWeights> {
   }
 
   static variable_list backward(AutogradContext* ctx, const variable_list& g) {
-    const variable_list s = ctx->get_saved_variables();
+    const variable_list s = saved(ctx);
     const c10::DeviceGuard guard(s[0].device());
     const Tensor x = s[0].contiguous();
     const int64_t R = x.size(0), K = x.size(1);

@@ -252,3 +252,17 @@ def ops_step(hooks):
 @pytest.mark.parametrize("layout", [strided, turned])
 def test_op_backwards_from_saved_tensors_in_other_strides(layout):
     same(ops_step((lambda t: t, layout)), ops_step((lambda t: t, lambda t: t)))
+
+
+@pytest.mark.parametrize("dynamic", [True, False])
+def test_saved_tensors_off_the_gpu_are_refused(dynamic):
+    """An unpack hook that leaves the tensors in host memory: the backward raises before any launch."""
+    hc, H, bo, dHn, dbi = make_case(2, 6, 32, torch.float32, dynamic=dynamic, phi_std=0.02)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t):
+        bi, add = hc(H.clone().requires_grad_(True))
+        Hn = add(bo.clone().requires_grad_(True))
+    for out, g in ((bi, dbi), (Hn, dHn)):
+        with pytest.raises(RuntimeError, match="ROCm GPU"):
+            out.backward(g, retain_graph=True)
+    with pytest.raises(RuntimeError, match="ROCm GPU"):
+        ops_step((lambda t: t.cpu(), lambda t: t))
