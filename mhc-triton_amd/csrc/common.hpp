@@ -365,13 +365,20 @@ __device__ __forceinline__ void ld(const RagSpan<T>& sp, uint32_t e, float* f) {
   fr.unpack(f);
 }
 
-// Zeroes the elements that a ragged row's last lane must not sum.
+// Zeroes the elements that a ragged row's last lane must not sum, in every factor of the sums'
+// products: a zero times an infinity of the neighbour's would be NaN.
 template <int W, bool RAG>
 __device__ __forceinline__ void drop_skipped(float (&v)[W], uint32_t skip) {
   if constexpr (RAG) {
 #pragma unroll
     for (int e = 0; e < W; ++e) v[e] = (uint32_t)e < skip ? 0.f : v[e];
   }
+}
+
+template <int W, bool RAG, int N>
+__device__ __forceinline__ void drop_skipped(float (&v)[N][W], uint32_t skip) {
+#pragma unroll
+  for (int n = 0; n < N; ++n) drop_skipped<W, RAG>(v[n], skip);
 }
 
 template <typename T, int W, bool NT, bool BUF>

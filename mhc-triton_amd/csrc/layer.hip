@@ -406,8 +406,9 @@ __global__ __launch_bounds__(kBatchThreads) void pass_b_rows_kernel(const T* __r
     }
 #pragma unroll
     for (int n = 0; n < 4; ++n) ld<T, W, true>(hs, e4 + n * (uint32_t)D, h[n]);
-#pragma unroll
-    for (int n = 0; n < 4; ++n) drop_skipped<W, RAG>(h[n], rc.skip);
+    drop_skipped<W, RAG>(db, rc.skip);
+    if constexpr (HAS_DHN) drop_skipped<W, RAG>(dn, rc.skip);
+    drop_skipped<W, RAG>(h, rc.skip);
 #pragma unroll
     for (int e = 0; e < W; ++e) {
 #pragma unroll

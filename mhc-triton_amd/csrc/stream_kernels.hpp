@@ -273,6 +273,7 @@ __global__ __launch_bounds__(NTH) void add_residual_bwd_kernel(const T* __restri
     for (int u = 0; u < U; ++u) {
       if (!ok[u]) continue;
       drop_skipped<W, RAG>(bv[u], skip[u]);
+      drop_skipped<W, RAG>(h[u], skip[u]);
       float r[W];
 #pragma unroll
       for (int e = 0; e < W; ++e) {
@@ -361,8 +362,9 @@ __global__ __launch_bounds__(kThreads) void mix_bwd_kernel(const T* __restrict__
     for (int u = 0; u < U; ++u) {
       if (!ok[u]) continue;
       if constexpr (REDUCE) {
-#pragma unroll
-        for (int n = 0; n < 4; ++n) drop_skipped<W, RAG>(h[u][n], skip[u]);
+        drop_skipped<W, RAG>(db[u], skip[u]);
+        if constexpr (HAS_DHN) drop_skipped<W, RAG>(dn[u], skip[u]);
+        drop_skipped<W, RAG>(h[u], skip[u]);
 #pragma unroll
         for (int e = 0; e < W; ++e) {
 #pragma unroll

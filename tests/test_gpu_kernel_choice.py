@@ -132,6 +132,44 @@ def test_mean_pool_on_ragged_rows(B, S, D, dtype, shifted):
     assert float((x.double() - want).abs().max()) <= 2.0 ** -14
 
 
+@pytest.mark.parametrize("B,S,D,dtype", [
+    # a workgroup per tile, a workgroup per batch, rows of one vector and an element, rows in 32 bits
+    (2, 197, 1001, torch.bfloat16), (300, 5, 1001, torch.float16), (2, 21850, 9, torch.bfloat16),
+    (3, 131, 1003, torch.float32)])
+@pytest.mark.parametrize("factor", [0, 1])
+def test_infinities_on_ragged_rows(B, S, D, dtype, factor):
+    """An infinity or a NaN where the last two lanes of a row overlap reaches dH_post, dH_pre and dH_res
+    once, as in plain products: +-inf stays +-inf.  The finite sums as in the test above."""
+    import mhc
+    from mhc import _layer
+
+    g = torch.Generator(device=DEV).manual_seed(12)
+    c = D - (4 if dtype == torch.float32 else 8)  # the last lane's first column, its neighbour's too
+    H, dHn = (torch.randn((B, S, 4, D), generator=g, device=DEV).to(dtype) for _ in range(2))
+    bo, dbi = (torch.randn((B, S, D), generator=g, device=DEV).to(dtype) for _ in range(2))
+    inf, nan = float("inf"), float("nan")
+    if factor == 0:
+        dHn[0, S // 2, 1, c], dHn[1, 0, 2, c + 1], dHn[1, 0, 3, c] = inf, -inf, nan
+        dbi[0, 1, c] = inf
+    else:
+        bo[0, S // 2, c], H[1, 1, 2, c + 1] = -inf, inf
+    post, pre, res = (torch.rand(s, generator=g, device=DEV) for s in ((B, 4), (B, 4), (B, 4, 4)))
+    want = [(dHn.double() * bo.double()[:, :, None]).sum((1, 3)), (H.double() * dbi.double()[:, :, None]).sum((1, 3)),
+            torch.stack([torch.stack([(dHn[:, :, n].double() * H[:, :, m].double()).sum((1, 2)) for m in range(4)], -1)
+                         for n in range(4)], 1)]
+    hr, b, post = H.clone().requires_grad_(True), bo.clone().requires_grad_(True), post.requires_grad_(True)
+    mhc.fused_add_residual(hr, b, post).backward(dHn)
+    Hl, pre, res = H.clone().requires_grad_(True), pre.requires_grad_(True), res.requires_grad_(True)
+    torch.autograd.backward(mhc.fused_stream_mix(Hl, pre, res), [dbi, dHn])
+    _, dpre, dres = _layer.mix_backward(H, dbi, dHn, torch.rand((B, 24), generator=g, device=DEV), need_dH=False)
+    for what, got, ref in (("dH_post", post.grad, want[0]), ("dH_pre", pre.grad, want[1]), ("dH_res", res.grad, want[2]),
+                           ("layer dH_pre", dpre, want[1]), ("layer dH_res", dres.reshape(B, 4, 4), want[2])):
+        fin = ref.isfinite()
+        assert not fin.all(), what
+        assert torch.equal(got[~fin].nan_to_num(1, 2, 3), ref[~fin].float().nan_to_num(1, 2, 3)), what
+        assert float((got[fin] - ref[fin]).abs().max()) <= 1e-4 * float(ref[fin].abs().max()), what
+
+
 def test_mixed_types_on_ragged_rows():
     """H in fp32 with a bf16 branch output (8 elements a lane): the bits of the single-element path,
     which the same rows take in pieces too small for the ragged one."""
