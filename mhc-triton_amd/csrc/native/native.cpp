@@ -150,7 +150,8 @@ void param_grads(const Tensor* prm, const Tensor* part, variable_list& out) {
   int64_t count[N];
   for (int i = 0; i < N; ++i) {
     const Tensor& p = prm[i];
-    if (p.scalar_type() == at::kFloat || code(p) < 0) {
+    // a parameter of another size than the kernels' gradient: the reshape refuses it
+    if (p.scalar_type() == at::kFloat || code(p) < 0 || p.numel() != part[i].numel()) {
       out.push_back(grad_like(part[i], p));
       continue;
     }

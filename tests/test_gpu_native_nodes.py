@@ -266,3 +266,13 @@ def test_saved_tensors_off_the_gpu_are_refused(dynamic):
             out.backward(g, retain_graph=True)
     with pytest.raises(RuntimeError, match="ROCm GPU"):
         ops_step((lambda t: t.cpu(), lambda t: t))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_parameter_of_another_size_is_refused_in_the_backward(dtype):
+    """phi with rows to spare: the kernels read what they need, and the gradient does not fit it."""
+    hc, H, bo, dHn, dbi = make_case(2, 6, 32, torch.float32, phi_std=0.02)
+    hc.phi = torch.nn.Parameter(torch.zeros((256, 24), device=DEV, dtype=dtype))
+    bi, add = hc(H.clone().requires_grad_(True))
+    with pytest.raises(RuntimeError, match="shape"):
+        torch.autograd.backward([add(bo), bi], [dHn, dbi])
