@@ -461,7 +461,9 @@ __device__ __forceinline__ float sum_all16(float v) { return sum_col16(sum_row16
 // of value threadIdx.x in threads < NV.  A wave butterfly over __shfl_xor costs
 // 6 ds_bpermute per value instead (600 for the weights projection's 100
 // partials).
-// `lds` must hold NTH / 16 * NV floats.
+// `lds` must hold NTH / 16 * NV floats.  Past 256 threads the row sums add in fp64: there are more
+// of them, and they are the largest values of the whole reduction (a workgroup per batch: what two
+// kernels' fp64 and smaller trees did before it).
 template <int NV, int NTH = kThreads>
 __device__ __forceinline__ float block_sum_rows(float (&v)[NV], float* lds) {
   static_assert(NV <= NTH, "one output per thread");
@@ -473,12 +475,12 @@ __device__ __forceinline__ float block_sum_rows(float (&v)[NV], float* lds) {
     for (int i = 0; i < NV; ++i) lds[row * NV + i] = v[i];
   }
   __syncthreads();
-  float t = 0.f;
+  std::conditional_t<(NTH > kThreads), double, float> t = 0;
   if (threadIdx.x < NV) {
 #pragma unroll
     for (int q = 0; q < NTH / 16; ++q) t += lds[q * NV + threadIdx.x];
   }
-  return t;
+  return (float)t;
 }
 
 // block_sum for a workgroup of NT threads: one wave (the wave sum alone) or

@@ -409,17 +409,22 @@ __global__ __launch_bounds__(kBatchThreads) void pass_b_rows_kernel(const T* __r
     drop_skipped<W, RAG>(db, rc.skip);
     if constexpr (HAS_DHN) drop_skipped<W, RAG>(dn, rc.skip);
     drop_skipped<W, RAG>(h, rc.skip);
+    float sum[20];  // tile by tile: one chain over eight tiles would round more
+#pragma unroll
+    for (int k = 0; k < 20; ++k) sum[k] = 0.f;
 #pragma unroll
     for (int e = 0; e < W; ++e) {
 #pragma unroll
-      for (int n = 0; n < 4; ++n) acc[n] += db[e] * h[n][e];
+      for (int n = 0; n < 4; ++n) sum[n] += db[e] * h[n][e];
       if constexpr (HAS_DHN) {
 #pragma unroll
         for (int n = 0; n < 4; ++n)
 #pragma unroll
-          for (int m = 0; m < 4; ++m) acc[4 + 4 * n + m] += dn[n][e] * h[m][e];
+          for (int m = 0; m < 4; ++m) sum[4 + 4 * n + m] += dn[n][e] * h[m][e];
       }
     }
+#pragma unroll
+    for (int k = 0; k < 20; ++k) acc[k] += sum[k];
   }
   const float t = block_sum_rows<20, kBatchThreads>(acc, lds);
   if (threadIdx.x < 20) tot[threadIdx.x] = t;

@@ -234,7 +234,9 @@ __global__ __launch_bounds__(NTH) void add_residual_bwd_kernel(const T* __restri
                                                                     Geom g) {
   // ONE: one workgroup per tile (grid.x == g.ntiles), the weights fetched behind the tile's loads;
   // otherwise workgroups stride over the tiles.  With one workgroup per batch (grid.x == 1) part is
-  // dH_post itself.
+  // dH_post itself, and a lane sums tile by tile (one chain over eight tiles rounded more than the
+  // partials of a workgroup per tile did).
+  constexpr bool kByTile = NTH > kThreads;
   __shared__ float lds[NTH / 16 * 4];
   const int64_t b = g.b0 + blockIdx.y;
   float wq[4];
@@ -252,6 +254,8 @@ __global__ __launch_bounds__(NTH) void add_residual_bwd_kernel(const T* __restri
     float bv[U][W];
     uint32_t e1[U], skip[U];
     bool ok[U];
+    float tile_sum[4] = {0.f, 0.f, 0.f, 0.f};
+    float(&sum)[4] = kByTile ? tile_sum : acc;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t i = tile * (NTH * U) + u * NTH + threadIdx.x;
@@ -279,9 +283,13 @@ __global__ __launch_bounds__(NTH) void add_residual_bwd_kernel(const T* __restri
       for (int e = 0; e < W; ++e) {
         r[e] = wq[0] * h[u][0][e] + wq[1] * h[u][1][e] + wq[2] * h[u][2][e] + wq[3] * h[u][3][e];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) acc[n] += h[u][n][e] * bv[u][e];
+        for (int n = 0; n < 4; ++n) sum[n] += h[u][n][e] * bv[u][e];
       }
       st_from<TB, W, (NT & 2) != 0>(ds_, e1[u], r, skip[u]);
+    }
+    if constexpr (kByTile) {
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[n] += tile_sum[n];
     }
     if constexpr (ONE) break;
   }

@@ -204,14 +204,16 @@ def test_mean_pool_chunks(B, S, D, dtype):
     # few batches take the other kernels), rows in 32 bits, ragged rows
     (1, 1, 8, torch.bfloat16, 20), (3, 1, 4096, torch.bfloat16, 20), (2, 2, 4096, torch.float16, 7),
     (2, 1, 8200, torch.bfloat16, 20), (5, 3, 1368, torch.float32, 33), (300, 5, 1001, torch.bfloat16, 7),
-    # 256 batches and more: three tiles with a partial last one, eight, and one vector past eight
-    (256, 3, 3000, torch.bfloat16, 20), (257, 8, 4096, torch.bfloat16, 20), (256, 1, 32776, torch.bfloat16, 20),
+    # 256 batches and more: three tiles with a partial last one, four, eight, and (outputs only) eight
+    # of another type and one vector past eight
+    (256, 3, 3000, torch.bfloat16, 20), (256, 4, 4096, torch.bfloat16, 20), (260, 4, 2040, torch.float32, 20),
+    (256, 8, 2048, torch.float32, 20), (257, 8, 4096, torch.bfloat16, 20), (256, 1, 32776, torch.bfloat16, 20),
     # the most batches, and one more
     (1024, 2, 64, torch.float16, 20), (1025, 2, 64, torch.float16, 20)])
 def test_whole_batch_workgroups(B, S, D, dtype, iters):
     hc, H, bo, dHn, dbi = make_case(B, S, D, dtype, phi_std=0.02)
     hc.sinkhorn_iters = iters
-    if B * S * D > 1 << 23:  # too slow for the oracle in full: the first batches of the same call
+    if B * S * D > 1 << 23:  # too slow for the oracle in full: what the first batches of the same call put out
         from oracle import mhc_oracle as O
         from test_gpu_module import params_np, rel_err, run_gpu, to_np
 
@@ -224,6 +226,26 @@ def test_whole_batch_workgroups(B, S, D, dtype, iters):
             assert rel_err(to_np(got), want) < 2e-2
         return
     check_layer(hc, H, bo, dHn, dbi, *FWD[dtype], 1e-4)
+
+
+@pytest.mark.parametrize("B,S,D,tiles", [(64, 4, 1024, 2), (256, 4, 2048, 4), (256, 8, 2048, 8)])
+def test_whole_batch_sums_round_as_little_as_a_tree(B, S, D, tiles):
+    """dH_post of a workgroup per batch, in fp32 from unit normals: a sum of n products is about sqrt(n), and
+    a rounding at a partial sum of k of them adds sqrt(k) 2^-25 or less (rms).  Lanes chain 4 products a
+    tile (2.5 n of such k in all) and add their tiles (the k / tiles of the second on), 16 lanes add in a
+    tree (4 n), the 32 row sums add in fp64, and the result rounds once (n).  Summed in fp32 the rows
+    would add 16.5 n."""
+    import mhc
+
+    g = torch.Generator(device=DEV).manual_seed(6)
+    hr, bo = torch.randn((B, S, 4, D), generator=g, device=DEV), torch.randn((B, S, D), generator=g, device=DEV)
+    post = torch.rand((B, 4), generator=g, device=DEV).requires_grad_(True)
+    mhc.fused_add_residual(hr, bo, post).backward(hr)
+    want = (hr.double() * bo.double()[:, :, None]).sum((1, 3))
+    err = float((post.grad.double() - want).norm() / want.norm())
+    bound = (2.5 + sum(range(2, tiles + 1)) / tiles + 4 + 1) ** 0.5 * 2.0 ** -25
+    print(f"dH_post B={B} S={S} D={D}: {err:.2e} of {bound:.2e}", flush=True)
+    assert err < 1.1 * bound
 
 
 @pytest.mark.parametrize("B,S,D", [(4, 2, 512), (256, 4, 2048)])
