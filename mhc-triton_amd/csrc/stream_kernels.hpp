@@ -690,16 +690,20 @@ inline int with_width(int64_t B, int64_t S, int64_t D, std::initializer_list<con
 // Short sequences: one workgroup of kBatchThreads lanes takes a whole batch, so a reduction over it
 // needs no partials and no second kernel, and what follows per batch can run in the workgroup
 // itself.  It pays where a batch is a tile or two, and for up to eight where batches alone fill the
-// GPU.  Training steps as graphs, bf16, apart -> whole batches: B=1, S=1, D=4096 (one tile) 33.5 ->
-// 29.8 us, B=64 49.2 -> 44.9, B=8, S=4, D=2048 (two) 39.0 -> 37.5, B=512, S=8, D=2048 (four) 169.3
-// -> 161.4, B=512, S=16 (eight) 282.7 -> 275.3; but B=64, S=8, D=2048 (four) 55.6 -> 60.2, and with
-// many batches of one tile each workgroup's serial end costs more than the launches: B=1024 equal,
-// B=4096 381 -> 397.
+// GPU, the last round of one per CU at least half.  Training steps as graphs, bf16, apart -> whole
+// batches: B=1, S=1, D=4096 (one tile) 33.5 -> 29.8 us, B=64 42.3 -> 38.0, B=512 81.2 -> 79.7, B=8, S=4,
+// D=2048 (two) 39.0 -> 37.5, B=64 45.4 -> 44.3, B=512 112.9 -> 109.3; but B=64, S=8, D=2048 (four) 55.6 ->
+// 60.2, and with many batches of one tile each workgroup's serial end costs more than the launches:
+// B=4096 381 -> 397.  The last round: S=8, D=4096 (eight) B=256 165 -> 158, B=257 170 -> 178, B=320 194 ->
+// 199, B=384 221 -> 219, B=512 285 -> 282, B=528 304 -> 317, B=640 352 -> 350; S=4, D=4096 (four) in the
+// same order 112 -> 108, 117 -> 118, 130 -> 131, 147 -> 144, 177 -> 168, 189 -> 191, 214 -> 210.
 constexpr int kBatchThreads = 512;
+constexpr int64_t kBatchRound = 256;  // a workgroup per CU
 
 inline bool whole_batch(int64_t B, int64_t S, int64_t D, int W) {
   const int64_t tiles = (S * ((D + W - 1) / W) + kBatchThreads - 1) / kBatchThreads;
-  return tiles >= 1 && B <= 1024 && (tiles <= 2 || (B >= 256 && tiles <= 8));
+  const bool filled = B >= kBatchRound && (B - 1) % kBatchRound + 1 >= kBatchRound / 2;
+  return tiles >= 1 && B <= 1024 && (tiles <= 2 || (filled && tiles <= 8));
 }
 
 // Workgroups per batch for a reduction kernel: about kRedBlocks in total

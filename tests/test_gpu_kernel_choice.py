@@ -206,8 +206,10 @@ def test_mean_pool_chunks(B, S, D, dtype):
     (2, 1, 8200, torch.bfloat16, 20), (5, 3, 1368, torch.float32, 33), (300, 5, 1001, torch.bfloat16, 7),
     # 256 batches and more: three tiles with a partial last one, four, eight, and (outputs only) eight
     # of another type and one vector past eight
-    (256, 3, 3000, torch.bfloat16, 20), (256, 4, 4096, torch.bfloat16, 20), (260, 4, 2040, torch.float32, 20),
-    (256, 8, 2048, torch.float32, 20), (257, 8, 4096, torch.bfloat16, 20), (256, 1, 32776, torch.bfloat16, 20),
+    (256, 3, 3000, torch.bfloat16, 20), (256, 4, 4096, torch.bfloat16, 20), (384, 4, 2040, torch.float32, 20),
+    (256, 8, 2048, torch.float32, 20), (384, 8, 4096, torch.bfloat16, 20), (256, 1, 32776, torch.bfloat16, 20),
+    # a last round of 256 that is less than half (the other kernels), and half
+    (257, 3, 3000, torch.bfloat16, 20), (383, 3, 3000, torch.float16, 20), (384, 3, 3000, torch.float16, 20),
     # the most batches, and one more
     (1024, 2, 64, torch.float16, 20), (1025, 2, 64, torch.float16, 20)])
 def test_whole_batch_workgroups(B, S, D, dtype, iters):
