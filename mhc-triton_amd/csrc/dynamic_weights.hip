@@ -208,16 +208,28 @@ static WidePlan wide_plan(int64_t R, int64_t K) {
 // elements) would pass 2^31 bytes.
 //
 // With fewer rows there is little to stream per workgroup, and what counts is the latency of its
-// one or two blocks: narrower workgroups (bwd_waves) share a CU and take longer chunks, which also
-// leaves fewer grad_phi partials, down to one chunk and no reduce after it.  Eight waves -> two, or
-// four past 512 rows, the call's fwd+bwd as a graph: R = 256, K = 4096 bf16 30.5 -> 26.4 us, the layer
-// at B = 64, S = 1, D = 4096 45.0 -> 41.0, B = 256 60.4 -> 55.9, B = 512, S = 8, D = 2048 162.0 ->
-// 158.9; R = 1000, K = 8192 fp32 46.9 -> 46.3, R = 4096, K = 8192 bf16 69.1 -> 67.6.  Two waves at
-// R = 4096 took 80.0, four at R = K = 16384 337.8 against 309.
-static int bwd_waves(int64_t R) { return R <= 512 ? 2 : R <= 4096 ? 4 : kBwdWaves; }
+// one or two blocks: narrower workgroups (64 or 128 columns) share a CU and take longer chunks, which
+// also leaves fewer grad_phi partials, down to one chunk and no reduce after it.  Eight waves -> two, or
+// four past 512 rows, the call's fwd+bwd as a graph: R = 64, K = 16384 bf16 31.3 -> 25.2 us, R = 256, K =
+// 4096 32.9 -> 26.5, R = 512, K = 16384 42.0 -> 37.8 and K = 28672 59.5 -> 46.8, R = 1024 50.4 -> 47.7 and
+// 76.9 -> 67.3, R = 2048 69.1 -> 67.2 and 135 -> 122, R = 4096, K = 8192 68.5 -> 67.0; fp32 R = 1024, K =
+// 8192 46.6 -> 43.6, R = 4096, K = 16384 171 -> 167; the layer at S = 1, D = 4096, B = 64 41.9 -> 37.6, B =
+// 512 80.1 -> 79.6, B = 4096 378 -> 370.  Two waves took 78.9 at R = 2048 and 131 at R = 4096, K = 16384,
+// four 338 against 309 at R = K = 16384.
+// The wide strips come back first where they fill every CU once and there is the most to stream, with
+// 16 bits read and written: R = 3584, K = 16384 96.3 (four) -> 95.0 (eight), R = 4096 106.7 -> 101-105 and fp16
+// 110.9 -> 105.0, R = 4096, K = 32768 181 -> 172; with less to stream they lose (R = 4096, K = 8192 68.0 ->
+// 70.7), and so they do where K's blocks do not divide the CUs (R = 4096, K = 24576 177 -> 193).
+// esize: the wider of x and grad_x.
+static int bwd_waves(int64_t R, int64_t K, int esize) {
+  if (R <= 512) return 2;
+  if (R > 4096) return kBwdWaves;
+  const int64_t ncb = (K + 32 * kBwdWaves - 1) / (32 * kBwdWaves);
+  return esize == 2 && R * K >= (int64_t)3584 * 16384 && kMfmaTargetWg % ncb == 0 ? kBwdWaves : 4;
+}
 
 static WidePlan mfma_bwd_plan(int64_t R, int64_t K, const WidePlan& w, int esize) {
-  const int64_t cols = 32 * bwd_waves(R);
+  const int64_t cols = 32 * bwd_waves(R, K, esize);
   const int64_t ncb = (K + cols - 1) / cols;
   int64_t nr = (kMfmaTargetWg + ncb - 1) / ncb;
   if (nr > w.nR) nr = w.nR;
@@ -265,7 +277,7 @@ int dynw_grad_pass(const void* x, int dtype_x, const float* phi, const float* ro
     // rows in bulk: grad_x and grad_phi on MFMA.
     if (pl.nR > 1 && (grad_bias || grad_alpha))
       bias_part = (float*)(split_ws + align256((size_t)w.nR * K * kOut * sizeof(float)));
-    const int nw = bwd_waves(R);
+    const int nw = bwd_waves(R, K, span_esize);
     const dim3 grid((unsigned)((K + 32 * nw - 1) / (32 * nw)), (unsigned)pl.nR);
     rc = MHC_DISPATCH_DTYPE(dtype_x, [&] {
       auto go = [&](auto* kernel, auto* gx) {

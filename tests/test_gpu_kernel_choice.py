@@ -343,6 +343,11 @@ def test_weights_backward_column_blocks(R, K, xdtype):
     check_dynamic_weights(R, K, xdtype)
 
 
+def test_weights_backward_wide_blocks_of_few_rows():
+    """Eight-wave column blocks below 4097 rows: 16 bits, and one block row per CU (3584 rows of 16384)."""
+    check_dynamic_weights(3584, 16384, torch.bfloat16)
+
+
 @pytest.mark.parametrize("B,S,D,dtype,iters", [
     # rows and wide pass in one: up to four rows, with three partials each (one past a whole batch's
     # two tiles), sixteen and seventeen, 256 and (apart again) 257 and five rows; K not a whole wave
