@@ -153,3 +153,12 @@ def test_stream_ceiling_probe_rejects_bad_shapes_without_gpu(lib):
     assert fn(2, 0, 0, 0, fake, null, null, null, 16, 8192, 0, 1, fake, null) == 1  # unsupported mix
     assert fn(4, 0, 0, 0, fake, null, null, null, 16, 1 << 30, 0, 1, fake, null) == 1  # span >= 2^31
     assert not hasattr(lib, "mhc_probe_stream")
+
+
+def test_the_library_alone_builds_without_torch():
+    """`make lib` is the C ABI's build: no compiler but hipcc, and neither Python nor torch."""
+    import subprocess
+
+    out = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "mhc-triton_amd"), "lib"], check=True,
+                         capture_output=True, text=True).stdout
+    assert "libmhc_hip.so" in out and "native" not in out and "torch" not in out and "python" not in out
