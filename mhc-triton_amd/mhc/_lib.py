@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 import torch
 
@@ -99,12 +100,21 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+class _NoBinding:
+    """Stands in for a binding that cannot be loaded: leaves every call to the Python nodes."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 _native = None
 
 
 def native():
     """The binding of the eager entry points (csrc/native/native.cpp, built next to the library).  Its
-    functions return None for calls they leave to the Python nodes."""
+    functions return None for calls they leave to the Python nodes.  Where it is not built or not
+    loadable (it needs the torch it was built against; the library needs none), every call is left to them:
+    the same kernels and results at more host time per call, after a RuntimeWarning."""
     global _native
     if _native is None:
         load()
@@ -112,10 +122,13 @@ def native():
             if _native is None:
                 try:
                     from . import _native as mod
+
+                    mod.set_error(MHCError)
                 except ImportError as e:
-                    raise MHCError(f"mhc: binding not built or not loadable ({e}); run `make -C mhc-triton_amd` or "
-                                   "`python -c 'import __graft_entry__ as g; g.build()'`") from e
-                mod.set_error(MHCError)
+                    warnings.warn(f"mhc: C++ binding not built or not loadable ({e}); eager calls take the slower "
+                                  "Python nodes. Run `make -C mhc-triton_amd` or "
+                                  "`python -c 'import __graft_entry__ as g; g.build()'`", RuntimeWarning, stacklevel=3)
+                    mod = _NoBinding()
                 _native = mod
     return _native
 

@@ -162,3 +162,18 @@ def test_the_library_alone_builds_without_torch():
     out = subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "mhc-triton_amd"), "lib"], check=True,
                          capture_output=True, text=True).stdout
     assert "libmhc_hip.so" in out and "native" not in out and "torch" not in out and "python" not in out
+
+
+def test_without_the_binding_calls_are_left_to_the_python_nodes(lib, monkeypatch):
+    import sys
+
+    import mhc
+    from mhc import _lib
+
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.delattr(mhc, "_native", raising=False)
+    monkeypatch.setitem(sys.modules, "mhc._native", None)  # the import fails
+    with pytest.warns(RuntimeWarning, match="binding not built or not loadable"):
+        native = _lib.native()
+    assert native.sinkhorn(None, 20, 1e-8) is None and native.dynamic_layer() is None
+    assert _lib.native() is native  # warned once
