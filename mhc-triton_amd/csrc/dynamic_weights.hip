@@ -33,9 +33,10 @@ static DynPlan dyn_plan(int64_t R, int64_t K) {
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // MFMA plan for x with many rows (dynw_mfma_kernel): K chunks of
-// mfma_steps(esize) * kMfmaWaves steps (1024 k for 16-bit x, 512 k for fp32),
-// and row ranges of whole 32-row tiles so that about kMfmaTargetWg workgroups
-// run, one per CU (the kernel's LDS allows one).
+// mfma_steps(esize) * kMfmaWaves steps (1024 k for 16-bit x, 512 k for fp32; for
+// few rows down to kMfmaMinSteps * kMfmaWaves, 256 k), and row ranges of whole
+// 32-row tiles so that about kMfmaTargetWg workgroups run, one per CU (the
+// kernel's LDS allows one).
 // At R = K = 16384, 16-bit x: 16 chunks x 16 ranges of 1024 rows.
 constexpr int64_t kMfmaMinRows = 64;
 constexpr int64_t kMfmaTargetWg = 256;
@@ -373,8 +374,8 @@ extern "C" int mhc_dynamic_weights_backward(const void* x, int dtype_x, const fl
 namespace mhc {
 
 constexpr int kPoolUN = 4;  // rows in flight per lane in colsum_kernel
-// Sequences up to this length take colsum_direct_kernel (one launch): at such lengths the pass is a few microseconds of latency, and the
-// second launch and the column-partial round trip are most of it.
+// Sequences up to this length take colsum_direct_kernel (one launch): at such lengths the pass is a few
+// microseconds of latency, and the second launch and the column-partial round trip are most of it.
 constexpr int64_t kPoolDirectRows = 8;
 constexpr int64_t kPoolPlainBytes = (int64_t)64 << 20;  // H up to here is read without the nt policy
 
@@ -455,7 +456,8 @@ int mean_pool_any(const void* H, int dtype, float* x, const float* phi, float* p
     };
     if (vec) return go(std::integral_constant<int, WV>{}, std::false_type{});
     // ragged: K = 4 D is not whole vectors (odd D in 16 bits), or H does not start on one
-    if (rag_ok(B * S * D, K, WV) && span_ok(kPoolUN * K, 4)) return go(std::integral_constant<int, WV>{}, std::true_type{});
+    if (rag_ok(B * S * D, K, WV) && span_ok(kPoolUN * K, 4))
+      return go(std::integral_constant<int, WV>{}, std::true_type{});
     return go(std::integral_constant<int, 1>{}, std::false_type{});
   });
 }

@@ -151,7 +151,10 @@ constexpr int kMfmaChunkSteps = kMfmaWaves * kMfmaSteps;  // steps per K chunk (
 // fp32 x: half the steps per slice, so that a slice is still 256 bytes of a row
 // and the LDS tiles keep their size.  A few rows take shorter slices (mfma_plan).
 __host__ __device__ constexpr int mfma_steps(int esize) { return esize == 4 ? kMfmaSteps / 2 : kMfmaSteps; }
-constexpr int kMfmaMinSteps = 2;  // K chunks of 256: as many records per row as the VALU plans hold
+constexpr int kMfmaMinSteps = 2;
+// The shortest slices make K chunks of 256, as many records per row as the mean-pool's reduce writes: the
+// layer's projection-partial region holds ceil(K / kThreads) of them and no more.
+static_assert(kMfmaMinSteps * kMfmaWaves * 16 >= kThreads, "the projection's records fit the layer's workspace");
 constexpr int kMfmaRedCols = kPart;                       // 24 dot products and the sum of squares
 constexpr int kMfmaRedPitch = 36;                         // floats per (wave, column): 32 rows + pad
 

@@ -555,8 +555,8 @@ static int layer_dynamic_forward_run(const void* H, int dtype, const float* phi,
   int nK = 0;
   const int64_t K = 4 * D;
   DynParams P{H_pre_base, H_post_base, H_res_base, alpha_pre, alpha_post, alpha_res};
-  // Many batches: the mean-pool alone, then the pooled rows' projection on MFMA (its records
-  // fit the projection-partial region: at most K / 512 chunks against K / 256).  At S = 1 the
+  // Many batches: the mean-pool alone, then the pooled rows' projection on MFMA (its records fit
+  // the projection-partial region: chunks of K of at least kThreads, as kMfmaMinSteps ensures).  At S = 1 the
   // pooled rows are H's own rows, projected as they are (half the bytes of the f32 rows in
   // 16-bit H), and the f32 copy is written only for a backward that asks for it.  For S > 1
   // without x (no backward follows) the pooled rows go to the workspace's grad_x region, so

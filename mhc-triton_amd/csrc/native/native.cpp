@@ -392,8 +392,9 @@ struct StaticLayer : Function<StaticLayer> {
     if (ctx->needs_input_grad(0)) dH = at::empty(H.sizes(), H.options().requires_grad(false));
     const Tensor gb = empty_f32({24}, H);
     const Workspace ws(mhc_layer_workspace_bytes(d.B, d.S, d.D, code(H)), H);
-    check(mhc_layer_static_backward(ptr(H), code(H), ptr(d_bi), ptr(dHn), fptr(dpost), q.p[0], q.p[1], q.p[2], fptr(w), ptr(dH), wptr(gb), d.B, d.S, d.D,
-                                    (int)ctx->saved_data["iters"].toInt(), ws.p(), ws.bytes, stream(H)),
+    check(mhc_layer_static_backward(ptr(H), code(H), ptr(d_bi), ptr(dHn), fptr(dpost), q.p[0], q.p[1], q.p[2], fptr(w),
+                                    ptr(dH), wptr(gb), d.B, d.S, d.D, (int)ctx->saved_data["iters"].toInt(), ws.p(),
+                                    ws.bytes, stream(H)),
           "layer_static_backward");
     const Tensor part[3] = {gb.narrow(0, 0, 4), gb.narrow(0, 4, 4), gb.narrow(0, 8, 16)};
     variable_list out{dH};
@@ -644,8 +645,9 @@ DwOut dynamic_weights_forward(const Tensor* t, int64_t iters, double eps) {
   const float* const* p = q.p;
   DwOut o{empty_f32({R, 4}, x), empty_f32({R, 4}, x), empty_f32({R, 4, 4}, x), empty_f32({R, 25}, x), q.buf};
   const Workspace ws(mhc_dynamic_weights_workspace_bytes(R, K), x);
-  check(mhc_dynamic_weights_forward(ptr(x), code(x), p[0], p[1], p[2], p[3], p[4], wptr(o.pre), wptr(o.post), wptr(o.res), wptr(o.aux), R, K, (int)iters, (float)eps,
-                                    ws.p(), ws.bytes, stream(x)),
+  check(mhc_dynamic_weights_forward(ptr(x), code(x), p[0], p[1], p[2], p[3], p[4], wptr(o.pre), wptr(o.post),
+                                    wptr(o.res), wptr(o.aux), R, K, (int)iters, (float)eps, ws.p(), ws.bytes,
+                                    stream(x)),
         "dynamic_weights_forward");
   return o;
 }

@@ -192,7 +192,8 @@ extern "C" int mhc_sinkhorn_backward(const void* M, int dtype_M, const void* dP,
   return MHC_DISPATCH_DTYPE(dtype_M, [&] {
     using TM = T;
     return MHC_DISPATCH_DTYPE(dtype_dP, [&] {
-      auto* k = vec ? (sk_small_eps(eps) ? sinkhorn_bwd_kernel<TM, T, true, true> : sinkhorn_bwd_kernel<TM, T, true, false>)
+      auto* k = vec ? (sk_small_eps(eps) ? sinkhorn_bwd_kernel<TM, T, true, true>
+                                         : sinkhorn_bwd_kernel<TM, T, true, false>)
                     : (sk_small_eps(eps) ? sinkhorn_bwd_kernel<TM, T, false, true>
                                           : sinkhorn_bwd_kernel<TM, T, false, false>);
       k<<<grid, kThreads, 0, (hipStream_t)stream>>>((const TM*)M, (const T*)dP, (TM*)dM, n_mat, iters, eps);
