@@ -217,20 +217,41 @@ static WidePlan wide_plan(int64_t R, int64_t K) {
 // 8192 46.6 -> 43.6, R = 4096, K = 16384 171 -> 167; the layer at S = 1, D = 4096, B = 64 41.9 -> 37.6, B =
 // 512 80.1 -> 79.6, B = 4096 378 -> 370.  Two waves took 78.9 at R = 2048 and 131 at R = 4096, K = 16384,
 // four 338 against 309 at R = K = 16384.
-// The wide strips come back first where they fill every CU once and there is the most to stream, with
-// 16 bits read and written: R = 3584, K = 16384 96.3 (four) -> 95.0 (eight), R = 4096 106.7 -> 101-105 and fp16
-// 110.9 -> 105.0, R = 4096, K = 32768 181 -> 172; with less to stream they lose (R = 4096, K = 8192 68.0 ->
-// 70.7), and so they do where K's blocks do not divide the CUs (R = 4096, K = 24576 177 -> 193).
+//
+// From 2560 rows on it is streaming again, and the wide strips come back where the narrow ones leave a
+// CU more to do (bwd_load: the blocks of the busiest one), by as much again or, with rows of 32 KiB and
+// more, as much: R = 4096 bf16 K = 3872 (31 x 9 workgroups of four waves, 16 x 16 of eight) 55.1 (four) ->
+// 50.5 (eight), K = 16384 106.7 -> 101-105, K = 16416 146.7 -> 141.0, K = 20512 172.7 -> 160.9, K = 32768
+// 181 -> 172, R = 3000 K = 20512 122 -> 117; fp32 K = 8208 135.1 -> 129.8, except where a round of fp32 just
+// fills the CUs (K = 8192 98.1 -> 103.0).  Elsewhere four win: K = 4096 48.7 against 51.7, K = 12288 118
+// against 124, K = 24576 177 against 193, K = 28704 197 against 201; the closest are K = 5000 (159.9, 159.3)
+// and K = 8224 (84.4, 83.1).
 // esize: the wider of x and grad_x.
-static int bwd_waves(int64_t R, int64_t K, int esize) {
+struct BwdLoad {
+  int64_t blocks;  // 64-row blocks of 32 columns on the busiest CU
+  int64_t rounds;
+};
+
+static BwdLoad bwd_load(int64_t R, int64_t K, const WidePlan& w, int waves) {
+  const int64_t ncb = (K + 32 * waves - 1) / (32 * waves);
+  int64_t nr = (kMfmaTargetWg + ncb - 1) / ncb;
+  if (nr > w.nR) nr = w.nR;
+  const int64_t rc = (R + nr - 1) / nr;
+  const int64_t rounds = (ncb * ((R + rc - 1) / rc) + kMfmaTargetWg - 1) / kMfmaTargetWg;
+  return {rounds * ((rc + kBwdRows - 1) / kBwdRows) * waves, rounds};
+}
+
+static int bwd_waves(int64_t R, int64_t K, const WidePlan& w, int esize) {
   if (R <= 512) return 2;
   if (R > 4096) return kBwdWaves;
-  const int64_t ncb = (K + 32 * kBwdWaves - 1) / (32 * kBwdWaves);
-  return esize == 2 && R * K >= (int64_t)3584 * 16384 && kMfmaTargetWg % ncb == 0 ? kBwdWaves : 4;
+  if (R < 2560) return 4;
+  const BwdLoad narrow = bwd_load(R, K, w, 4), wide = bwd_load(R, K, w, kBwdWaves);
+  const bool long_rows = K * esize >= 32768 && (esize == 2 || narrow.rounds > 1);
+  return narrow.blocks >= (long_rows ? 1 : 2) * wide.blocks ? kBwdWaves : 4;
 }
 
 static WidePlan mfma_bwd_plan(int64_t R, int64_t K, const WidePlan& w, int esize) {
-  const int64_t cols = 32 * bwd_waves(R, K, esize);
+  const int64_t cols = 32 * bwd_waves(R, K, w, esize);
   const int64_t ncb = (K + cols - 1) / cols;
   int64_t nr = (kMfmaTargetWg + ncb - 1) / ncb;
   if (nr > w.nR) nr = w.nR;
@@ -278,7 +299,7 @@ int dynw_grad_pass(const void* x, int dtype_x, const float* phi, const float* ro
     // rows in bulk: grad_x and grad_phi on MFMA.
     if (pl.nR > 1 && (grad_bias || grad_alpha))
       bias_part = (float*)(split_ws + align256((size_t)w.nR * K * kOut * sizeof(float)));
-    const int nw = bwd_waves(R, K, span_esize);
+    const int nw = bwd_waves(R, K, w, span_esize);
     const dim3 grid((unsigned)((K + 32 * nw - 1) / (32 * nw)), (unsigned)pl.nR);
     rc = MHC_DISPATCH_DTYPE(dtype_x, [&] {
       auto go = [&](auto* kernel, auto* gx) {

@@ -343,9 +343,13 @@ def test_weights_backward_column_blocks(R, K, xdtype):
     check_dynamic_weights(R, K, xdtype)
 
 
-def test_weights_backward_wide_blocks_of_few_rows():
-    """Eight-wave column blocks below 4097 rows: 16 bits, and one block row per CU (3584 rows of 16384)."""
-    check_dynamic_weights(3584, 16384, torch.bfloat16)
+@pytest.mark.parametrize("R,K,xdtype", [
+    # eight-wave column blocks below 4097 rows: long 16-bit rows in one round of the CUs, and where four-wave
+    # ones would leave the busiest CU twice the work; fp32 with and without a full round (eight, four)
+    (3584, 16384, torch.bfloat16), (3072, 3872, torch.float16), (2560, 8208, torch.float32),
+    (2560, 8192, torch.float32)])
+def test_weights_backward_wide_blocks_of_few_rows(R, K, xdtype):
+    check_dynamic_weights(R, K, xdtype)
 
 
 @pytest.mark.parametrize("B,S,D,dtype,iters", [
